@@ -86,9 +86,15 @@ SIGNATURES = {
         _p,                         # stream
     ]),
     "bvllm_silu_mul": (ctypes.c_int, [_p, _i64, _i32, _p, _p]),
+    "bvllm_linear_workspace_bytes": (ctypes.c_int64, [_i32, _i32, _i32, _i32]),
+    "bvllm_linear": (ctypes.c_int, [
+        _p, _i64, _p, _p, _p, _i64,  # x, stride, w, bias, out, stride
+        _i32, _i32, _i32, _i32,     # m, n, k, gated
+        _p, _p,                     # workspace, stream
+    ]),
 }
 
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 
 # Knobs of bvllm_set_tuning (include/babyvllm_amd.h).

@@ -4,10 +4,11 @@ Same module tree and parameter names as the reference (``model.layers[i].
 self_attn.qkv_proj`` with bias, ``o_proj``, ``mlp.gate_up_proj``,
 ``down_proj``, ``input_layernorm``, ``post_attention_layernorm``,
 ``model.norm``, ``lm_head`` unless embeddings are tied). Per layer a step runs:
-add + RMSNorm (HIP), the QKV GEMM (hipBLASLt through torch), fused RoPE + KV
-append (HIP, straight into the paged cache through the step's slot_mapping),
-paged attention (HIP decode or prefill kernel), the output GEMM, add + RMSNorm,
-the gate/up GEMM, SiLU·mul (HIP) and the down GEMM.
+add + RMSNorm (HIP), the QKV GEMM, fused RoPE + KV append (HIP, straight into the
+paged cache through the step's slot_mapping), paged attention (HIP decode or prefill
+kernel), the output GEMM, add + RMSNorm, the gate/up GEMM, SiLU·mul and the down
+GEMM. Steps of few tokens (decode) run the GEMMs on the HIP kernel, gate/up with
+SiLU·mul in its epilogue; the others on hipBLASLt through torch, with the HIP SiLU·mul.
 """
 
 from __future__ import annotations
@@ -17,21 +18,37 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from babyvllm.kernels.activation import fused_silu_mul
+from babyvllm.kernels.linear import gated_linear, skinny_linear
 from babyvllm.kernels.rope import fused_rope_and_cache
 from babyvllm.layers.attention import Attention
 from babyvllm.layers.layernorm import RMSNorm
+from babyvllm.layers.linear import Linear
 from babyvllm.layers.rotary import RotaryEmbedding
 from babyvllm.worker.context import get_forward_context
+
+
+def _has_hooks(m: nn.Module) -> bool:
+    g = torch.nn.modules.module
+    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
+                or g._global_backward_pre_hooks or "forward" in m.__dict__)
 
 
 class Qwen2MLP(nn.Module):
     def __init__(self, hidden_size: int, intermediate_size: int):
         super().__init__()
-        self.gate_up_proj = nn.Linear(hidden_size, 2 * intermediate_size, bias=False)
-        self.down_proj = nn.Linear(intermediate_size, hidden_size, bias=False)
+        self.gate_up_proj = Linear(hidden_size, 2 * intermediate_size, bias=False)
+        self.down_proj = Linear(intermediate_size, hidden_size, bias=False)
 
     def forward(self, x):
-        return self.down_proj(fused_silu_mul(self.gate_up_proj(x)))
+        proj = self.gate_up_proj
+        # The fused form skips the projection module's call: only where nothing is
+        # attached to it (hooks, a replaced or biased projection).
+        if type(proj) is Linear and proj.bias is None and not _has_hooks(proj):
+            act = gated_linear(x, proj.weight)
+            if act is not None:
+                return self.down_proj(act)
+        return self.down_proj(fused_silu_mul(proj(x)))
 
 
 class Qwen2Attention(nn.Module):
@@ -43,8 +60,8 @@ class Qwen2Attention(nn.Module):
         self.head_dim = cfg.head_dim
         self.q_size = self.num_heads * self.head_dim
         self.kv_size = self.num_kv_heads * self.head_dim
-        self.qkv_proj = nn.Linear(cfg.hidden_size, self.q_size + 2 * self.kv_size, bias=True)
-        self.o_proj = nn.Linear(self.q_size, cfg.hidden_size, bias=False)
+        self.qkv_proj = Linear(cfg.hidden_size, self.q_size + 2 * self.kv_size, bias=True)
+        self.o_proj = Linear(self.q_size, cfg.hidden_size, bias=False)
         self.attn = Attention(self.num_heads, self.head_dim, self.num_kv_heads)
 
     def forward(self, x, cos, sin):
@@ -101,10 +118,13 @@ class Qwen2ForCausalLM(nn.Module):
         super().__init__()
         self.config = cfg
         self.model = Qwen2Model(cfg)
-        self.lm_head = None if cfg.tie_word_embeddings else nn.Linear(cfg.hidden_size, cfg.vocab_size, bias=False)
+        self.lm_head = None if cfg.tie_word_embeddings else Linear(cfg.hidden_size, cfg.vocab_size, bias=False)
 
     def compute_logits(self, hidden, out=None):
         w = self.model.embed_tokens.weight if self.lm_head is None else self.lm_head.weight
+        logits = skinny_linear(hidden, w, None, out)
+        if logits is not None:
+            return logits
         if out is None:
             return F.linear(hidden, w)
         return torch.mm(hidden, w.t(), out=out)

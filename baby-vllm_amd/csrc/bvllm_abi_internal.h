@@ -95,6 +95,28 @@ struct SiluArgs {
   int32_t vec_ok;                          // 16-byte aligned, d % 8 == 0
 };
 
+struct LinearArgs {
+  const void* x; int64_t x_stride;         // [m, k] bf16
+  const void* w;                           // [n, k] bf16, or [2n, k] (gate rows, then up rows); contiguous
+  const void* bias;                        // [n] bf16 or null
+  void* out; int64_t out_stride;           // [m, n] bf16
+  float* partials;                         // LinearPlan::partial_bytes
+  int32_t m, n, k;
+  // Set by the launcher (linear_plan):
+  int32_t k_splits, row_groups, unit;
+};
+
+// How a linear layer of a few tokens runs (skinny_linear.hip).
+struct LinearPlan {
+  int32_t rw, kw;          // row waves x k slabs of a work-group; rw = 0: not a shape for this kernel
+  int32_t k_splits;        // k ranges over work-groups (> 1: fp32 partials and a second launch)
+  int32_t row_groups;      // work-groups per k range, an even split of the output columns ...
+  int32_t unit;            // ... in units of 2 or 4 columns
+  int64_t partial_bytes;
+};
+LinearPlan linear_plan(int32_t m, int32_t n, int32_t k, bool gated);
+hipError_t skinny_linear(const LinearArgs& a, bool gated, hipStream_t stream);
+
 hipError_t rope_kv_append(const RopeArgs& a, hipStream_t stream);
 int64_t argmax_workspace_bytes(int32_t rows, int32_t vocab);
 hipError_t greedy_argmax(const ArgmaxArgs& a, hipStream_t stream);

@@ -40,7 +40,7 @@ extern "C" {
 #endif
 
 /* ABI version of this header; bumped on any signature change. */
-#define BVLLM_ABI_VERSION 6
+#define BVLLM_ABI_VERSION 7
 
 #if defined(__GNUC__)
 #define BVLLM_API __attribute__((visibility("default")))
@@ -228,6 +228,25 @@ BVLLM_API int bvllm_fused_add_rms_norm(const void* input, int64_t input_stride, 
  * gate_up [rows, 2d] and out [rows, d] bf16, contiguous.
  */
 BVLLM_API int bvllm_silu_mul(const void* gate_up, int64_t rows, int32_t d, void* out, void* stream);
+
+/*
+ * Linear layer of a few tokens, for the decode steps of a model (the nn.Linear
+ * calls of babyvllm/models/qwen2.py:17-137): out[r, c] = bf16(sum over j of
+ * x[r, j] * w[c, j], in fp32, + bias[c]). x [m, k] bf16 with row stride x_stride,
+ * w [n, k] bf16 contiguous, bias [n] bf16 or NULL, out [m, n] bf16 with row stride
+ * out_stride. gated = 1: w is [2n, k] (gate rows, then up rows, no bias) and
+ * out = bf16(silu(gate) * up), silu and product in fp32.
+ * bvllm_linear_workspace_bytes returns the scratch one call needs, or -1 for a
+ * shape this kernel does not take (more than 64 tokens, k not a multiple of
+ * 128, n not of 4, ...): the caller then uses a library GEMM. Pointers of x and w
+ * are 16-byte aligned, x_stride a multiple of 8 elements, out 8-byte aligned with a
+ * stride multiple of 4. The order of the sums depends on (n, k, gated) and on
+ * whether m is at most 16, 32 or 64, on nothing else.
+ */
+BVLLM_API int64_t bvllm_linear_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t gated);
+BVLLM_API int bvllm_linear(const void* x, int64_t x_stride, const void* w, const void* bias, void* out,
+                 int64_t out_stride, int32_t m, int32_t n, int32_t k, int32_t gated, void* workspace,
+                 void* stream);
 
 #ifdef __cplusplus
 }

@@ -1,0 +1,114 @@
+"""Linear layers of a few tokens (bvllm_linear): values against float64, and which calls torch keeps."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+# (tokens, columns, k, gated): token-tile edges; columns that are no multiple of a
+# row tile or of the split's unit; one stage of k, slabs of unequal length, k split
+# over work-groups, and each wave layout of the launch rule.
+SHAPES = [
+    (1, 64, 128, False), (3, 100, 384, False), (16, 1152, 896, False), (17, 1156, 896, False),
+    (64, 896, 896, False), (5, 2564, 640, False), (16, 4608, 3584, False), (32, 4600, 1152, False),
+    (33, 4608, 3584, False), (1, 32772, 256, False), (16, 33000, 896, False), (48, 32768, 1024, False),
+    (2, 896, 8192, False), (16, 900, 18944, False), (33, 3584, 8320, False), (64, 260, 18944, False),
+    (24, 896, 4864, False), (64, 896, 4864, False),
+    (1, 64, 128, True), (16, 4864, 896, True), (33, 4868, 896, True), (64, 8196, 384, True),
+    (16, 18944, 3584, True), (17, 9000, 640, True),
+]
+
+
+def _reference(x, w, bias, gated):
+    y = x.double() @ w.double().T
+    if gated:
+        n = w.shape[0] // 2
+        return F.silu(y[:, :n]) * y[:, n:]
+    return y if bias is None else y + bias.double()
+
+
+@pytest.mark.parametrize("m,n,k,gated", SHAPES)
+def test_values_against_float64(m, n, k, gated):
+    from babyvllm.kernels.linear import gated_linear, skinny_linear
+
+    buf = torch.randn(m, k + 8, device="cuda", dtype=torch.bfloat16)
+    x = buf[:, :k]  # a strided view
+    w = torch.randn(n * (2 if gated else 1), k, device="cuda", dtype=torch.bfloat16) * 0.05
+    bias = None if gated else torch.randn(n, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        got = gated_linear(x, w) if gated else skinny_linear(x, w, bias)
+    assert got is not None and got.shape == (m, n)
+    want = _reference(x, w, bias, gated)
+    # fp32 sums of k bf16 products: at most k/2^24 of the sum of magnitudes off, then one
+    # bf16 rounding (2^-8 of the value). silu·up doubles the relative part.
+    mag = x.double().abs() @ w.double().abs().T
+    if gated:
+        mag = mag[:, :n] * mag[:, n:]
+    bound = (2 if gated else 1) * (want.abs() * 2 ** -8 + mag * k * 2 ** -24) + 1e-30
+    assert ((got.double() - want).abs() <= bound).all()
+
+
+def test_same_bits_for_any_batch_of_a_token_tile_count_and_in_a_graph():
+    from babyvllm.kernels.linear import skinny_linear
+
+    x = torch.randn(16, 8192, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(896, 8192, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        full = skinny_linear(x, w)
+        for m in (1, 7, 16):
+            assert torch.equal(skinny_linear(x[:m], w), full[:m])
+        out = torch.empty_like(full)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            skinny_linear(x, w, None, out)
+        for scale in (1.0, -2.0, 0.5):
+            x.mul_(scale)
+            graph.replay()
+            assert torch.equal(out, skinny_linear(x, w))
+
+
+def test_non_finite_weights_and_inputs_stay_in_their_row_and_column():
+    from babyvllm.kernels.linear import skinny_linear
+
+    x = torch.randn(5, 640, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(68, 640, device="cuda", dtype=torch.bfloat16)
+    w[67, 639], w[3, 0], x[4, 7] = float("inf"), float("nan"), float("nan")
+    with torch.no_grad():
+        got = skinny_linear(x, w)
+    want = x.double() @ w.double().T
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+
+
+def test_module_keeps_autograd_hooks_and_other_types():
+    from babyvllm.kernels.linear import gated_linear, skinny_linear
+    from babyvllm.layers.linear import Linear
+    from babyvllm.models.qwen2 import Qwen2MLP
+
+    lin = Linear(256, 64).to("cuda", torch.bfloat16)
+    ref = torch.nn.Linear(256, 64).to("cuda", torch.bfloat16)
+    ref.load_state_dict(lin.state_dict())
+    x = torch.randn(4, 256, device="cuda", dtype=torch.bfloat16)
+    assert skinny_linear(x, lin.weight, lin.bias) is None  # grad mode: torch's operation
+    lin(x).sum().backward()
+    ref(x).sum().backward()
+    assert torch.equal(lin.weight.grad, ref.weight.grad)
+    with torch.no_grad():
+        assert skinny_linear(x, lin.weight, lin.bias) is not None
+        assert skinny_linear(x.float(), lin.weight.float()) is None
+        assert skinny_linear(x[:, ::2], lin.weight[:, :128].contiguous()) is None
+        assert skinny_linear(x[:1].expand(4, 256), lin.weight) is None
+        assert skinny_linear(torch.randn(65, 256, device="cuda", dtype=torch.bfloat16), lin.weight) is None
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert skinny_linear(x, lin.weight, lin.bias) is None and lin(x).dtype == torch.float16
+        batched = torch.func.vmap(lambda r: lin(r))(x.view(4, 1, 256))
+        torch.testing.assert_close(batched.view(4, 64), ref(x), atol=2e-2, rtol=2e-2)
+
+        mlp = Qwen2MLP(256, 128).to("cuda", torch.bfloat16)
+        fused = mlp(x)
+        seen = []
+        hook = mlp.gate_up_proj.register_forward_hook(lambda m, i, o: seen.append(o))
+        torch.testing.assert_close(mlp(x), fused, atol=2e-3, rtol=2e-2)
+        hook.remove()
+        assert len(seen) == 1 and seen[0].shape == (4, 256)
+        assert gated_linear(x, mlp.gate_up_proj.weight) is not None
