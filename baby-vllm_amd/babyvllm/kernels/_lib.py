@@ -71,6 +71,20 @@ SIGNATURES = {
         _i32, _i32, _i32, _i32,     # H, Hkv, D, block_size
         _p,                         # stream
     ]),
+    "bvllm_paged_prefill_split": (ctypes.c_int, [
+        _p, _i64, _i64,             # q
+        _p, _p, _i64, _i64, _i64,   # caches + strides
+        _i32,                       # num_blocks
+        _p, _i64, _i32,             # block_tables, bt_stride, max_blocks
+        _p, _p, _p, _f32,           # query_start_loc, seq_lens, context_lens, scale
+        _p, _i64, _i64,             # out
+        _i32, _i32, _i32,           # num_seqs, num_tokens, max_query_len
+        _i32,                       # single_query_seqs (-1 = unknown)
+        _i32, _i32, _i32, _i32,     # H, Hkv, D, block_size
+        _p, _i32, _p,               # workspace, split_tiles, stream
+    ]),
+    "bvllm_prefill_split_tiles": (ctypes.c_int32, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i64]),
+    "bvllm_prefill_workspace_bytes": (ctypes.c_int64, [_i32, _i32, _i32, _i32, _i32]),
     "bvllm_set_tuning": (ctypes.c_int, [_i32, _i32]),
     "bvllm_argmax_workspace_bytes": (ctypes.c_int64, [_i32, _i32]),
     "bvllm_greedy_argmax": (ctypes.c_int, [

@@ -26,6 +26,30 @@ def _single_query_seqs(md, num_seqs):
     return sum(1 for i in range(num_seqs) if qsl[i + 1] - qsl[i] == 1)
 
 
+# Narrower tables never split: their sequences are a few key tiles long.
+_SPLIT_MIN_PAGES = 32
+
+
+def _split_tiles(md, num_seqs, num_tokens, single, num_heads, num_kv_heads, head_dim, width):
+    """Key tiles per range of a split launch, 0 for the plain one.
+
+    The choice looks at the work the host lists describe (the table's width stands in
+    for lists that are absent or of another length); the results do not depend on them.
+    """
+    if width < _SPLIT_MIN_PAGES:
+        return 0
+    tiles = -1
+    qsl, seq = getattr(md, "query_start_loc_cpu", None), getattr(md, "seq_lens_cpu", None)
+    if single >= 0 and qsl is not None and seq is not None and len(seq) == num_seqs and len(qsl) == num_seqs + 1:
+        group, tiles = num_heads // num_kv_heads, 0
+        for i in range(num_seqs):
+            n = qsl[i + 1] - qsl[i]
+            if n > 1:
+                tiles += ((n * group + 127) >> 7) * ((seq[i] + 63) >> 6)
+    return _lib.lib().bvllm_prefill_split_tiles(num_seqs, num_tokens, int(md.max_query_len), single, num_heads,
+                                                num_kv_heads, head_dim, width, int(tiles))
+
+
 def paged_prefill_attention(q, kv_cache, md, scale):
     """Causal attention for a flattened varlen batch, reading K/V from the paged cache.
 
@@ -64,16 +88,24 @@ def paged_prefill_attention(q, kv_cache, md, scale):
     if k_cache.stride() != v_cache.stride() or k_cache.stride(3) != 1:
         raise ValueError("K and V halves of kv_cache must share a layout with unit last stride")
     num_seqs = seq_lens.shape[0]
-    rc = _lib.lib().bvllm_paged_prefill(
+    single = _single_query_seqs(md, num_seqs)
+    split_tiles = _split_tiles(md, num_seqs, num_tokens, single, num_heads, num_kv_heads, head_dim, bt.shape[1])
+    args = (
         q.data_ptr(), q.stride(0), q.stride(1),
         k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1), k_cache.stride(2),
         kv_cache.shape[1],
         bt.data_ptr(), bt.stride(0), bt.shape[1],
         qsl.data_ptr(), seq_lens.data_ptr(), ctx_lens.data_ptr(), float(scale),
         out.data_ptr(), out.stride(0), out.stride(1),
-        num_seqs, num_tokens, int(md.max_query_len), _single_query_seqs(md, num_seqs),
+        num_seqs, num_tokens, int(md.max_query_len), single,
         num_heads, num_kv_heads, head_dim, page,
-        _lib.stream_handle(q.device),
     )
+    h = _lib.lib()
+    if split_tiles > 0:
+        nbytes = h.bvllm_prefill_workspace_bytes(num_tokens, num_heads, head_dim, bt.shape[1], split_tiles)
+        workspace = torch.empty(nbytes // 4, device=q.device, dtype=torch.float32)
+        rc = h.bvllm_paged_prefill_split(*args, workspace.data_ptr(), split_tiles, _lib.stream_handle(q.device))
+    else:
+        rc = h.bvllm_paged_prefill(*args, _lib.stream_handle(q.device))
     _lib.check(rc, "bvllm_paged_prefill")
     return out

@@ -133,6 +133,50 @@ extern "C" int bvllm_paged_decode(const void* q, int64_t q_stride_b, int64_t q_s
   return (int)paged_decode(a, (hipStream_t)stream);
 }
 
+// Checks and packs a prefill call; `nothing` is set when there is nothing to compute.
+static int pack_prefill(PrefillArgs& a, bool& nothing, const void* q, int64_t q_stride_t, int64_t q_stride_h,
+                        const void* k_cache, const void* v_cache,
+                        int64_t cache_stride_block, int64_t cache_stride_tok,
+                        int64_t cache_stride_head, int32_t num_blocks,
+                        const int32_t* block_tables, int64_t bt_stride, int32_t max_blocks,
+                        const int32_t* query_start_loc, const int32_t* seq_lens,
+                        const int32_t* context_lens, float scale,
+                        void* out, int64_t out_stride_t, int64_t out_stride_h,
+                        int32_t num_seqs, int32_t num_tokens, int32_t max_query_len,
+                        int32_t single_query_seqs,
+                        int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                        int32_t block_size) {
+  nothing = false;
+  if (num_seqs < 0 || num_tokens < 0 || max_query_len < 0) return kBad;
+  if (single_query_seqs < -1 || single_query_seqs > num_seqs) return kBad;
+  if (!valid_heads(num_heads, num_kv_heads)) return kBad;
+  if (head_dim != 64 && head_dim != 128) return kBad;
+  if (block_size != 16) return kBad;
+  if (num_tokens == 0 || num_seqs == 0 || max_query_len == 0) { nothing = true; return 0; }
+  if (!q || !out || !block_tables || !query_start_loc || !seq_lens || !context_lens) return kBad;
+  if (!cache_ok(k_cache, v_cache, cache_stride_block, cache_stride_tok, cache_stride_head, num_blocks))
+    return kBad;
+  if (!aligned16(q) || !aligned16(out) || q_stride_t % 8 || q_stride_h % 8 || out_stride_t % 8 ||
+      out_stride_h % 8)
+    return kBad;
+  if (max_blocks < 1 || bt_stride < max_blocks) return kBad;
+  // Offsets inside one page are 32-bit (decode kernel).
+  if ((int64_t)16 * cache_stride_tok > 0x7fffffff) return kBad;
+
+  a.q = q; a.q_st = q_stride_t; a.q_sh = q_stride_h;
+  a.k_cache = k_cache; a.v_cache = v_cache;
+  a.c_sb = cache_stride_block; a.c_st = cache_stride_tok; a.c_sh = cache_stride_head;
+  a.num_pages = num_blocks;
+  a.block_tables = block_tables; a.bt_stride = bt_stride; a.max_blocks = max_blocks;
+  a.query_start_loc = query_start_loc; a.seq_lens = seq_lens; a.context_lens = context_lens;
+  a.scale_log2 = scale * kLog2e;
+  a.out = out; a.o_st = out_stride_t; a.o_sh = out_stride_h;
+  a.num_seqs = num_seqs; a.num_tokens = num_tokens; a.max_query_len = max_query_len;
+  a.num_heads = num_heads; a.num_kv_heads = num_kv_heads; a.head_dim = head_dim;
+  a.single_query_seqs = single_query_seqs;
+  return 0;
+}
+
 extern "C" int bvllm_paged_prefill(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                                    const void* k_cache, const void* v_cache,
                                    int64_t cache_stride_block, int64_t cache_stride_tok,
@@ -145,34 +189,63 @@ extern "C" int bvllm_paged_prefill(const void* q, int64_t q_stride_t, int64_t q_
                                    int32_t single_query_seqs,
                                    int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
                                    int32_t block_size, void* stream) {
-  if (num_seqs < 0 || num_tokens < 0 || max_query_len < 0) return kBad;
-  if (single_query_seqs < -1 || single_query_seqs > num_seqs) return kBad;
-  if (!valid_heads(num_heads, num_kv_heads)) return kBad;
-  if (head_dim != 64 && head_dim != 128) return kBad;
-  if (block_size != 16) return kBad;
-  if (num_tokens == 0 || num_seqs == 0 || max_query_len == 0) return 0;
-  if (!q || !out || !block_tables || !query_start_loc || !seq_lens || !context_lens) return kBad;
-  if (!cache_ok(k_cache, v_cache, cache_stride_block, cache_stride_tok, cache_stride_head, num_blocks))
-    return kBad;
-  if (!aligned16(q) || !aligned16(out) || q_stride_t % 8 || q_stride_h % 8 || out_stride_t % 8 ||
-      out_stride_h % 8)
-    return kBad;
-  if (max_blocks < 1 || bt_stride < max_blocks) return kBad;
-  // Offsets inside one page are 32-bit (decode kernel).
-  if ((int64_t)16 * cache_stride_tok > 0x7fffffff) return kBad;
-
   PrefillArgs a{};
-  a.q = q; a.q_st = q_stride_t; a.q_sh = q_stride_h;
-  a.k_cache = k_cache; a.v_cache = v_cache;
-  a.c_sb = cache_stride_block; a.c_st = cache_stride_tok; a.c_sh = cache_stride_head;
-  a.num_pages = num_blocks;
-  a.block_tables = block_tables; a.bt_stride = bt_stride; a.max_blocks = max_blocks;
-  a.query_start_loc = query_start_loc; a.seq_lens = seq_lens; a.context_lens = context_lens;
-  a.scale_log2 = scale * kLog2e;
-  a.out = out; a.o_st = out_stride_t; a.o_sh = out_stride_h;
+  bool nothing;
+  const int rc = pack_prefill(a, nothing, q, q_stride_t, q_stride_h, k_cache, v_cache, cache_stride_block, cache_stride_tok,
+                              cache_stride_head, num_blocks, block_tables, bt_stride, max_blocks,
+                              query_start_loc, seq_lens, context_lens, scale, out, out_stride_t, out_stride_h,
+                              num_seqs, num_tokens, max_query_len, single_query_seqs, num_heads, num_kv_heads,
+                              head_dim, block_size);
+  return rc != 0 || nothing ? rc : (int)paged_prefill(a, (hipStream_t)stream);
+}
+
+extern "C" int32_t bvllm_prefill_split_tiles(int32_t num_seqs, int32_t num_tokens, int32_t max_query_len,
+                                             int32_t single_query_seqs, int32_t num_heads, int32_t num_kv_heads,
+                                             int32_t head_dim, int32_t max_blocks, int64_t key_tiles) {
+  if (num_seqs < 1 || num_tokens < 1 || max_query_len < 1 || max_blocks < 1) return 0;
+  if (!valid_heads(num_heads, num_kv_heads) || (head_dim != 64 && head_dim != 128)) return 0;
+  if (single_query_seqs < -1 || single_query_seqs > num_seqs) return 0;
+  PrefillArgs a{};
   a.num_seqs = num_seqs; a.num_tokens = num_tokens; a.max_query_len = max_query_len;
-  a.num_heads = num_heads; a.num_kv_heads = num_kv_heads; a.head_dim = head_dim;
   a.single_query_seqs = single_query_seqs;
+  a.num_heads = num_heads; a.num_kv_heads = num_kv_heads; a.head_dim = head_dim;
+  a.max_blocks = max_blocks;
+  return prefill_split_tiles(a, key_tiles);
+}
+
+extern "C" int64_t bvllm_prefill_workspace_bytes(int32_t num_tokens, int32_t num_heads, int32_t head_dim,
+                                                 int32_t max_blocks, int32_t split_tiles) {
+  if (num_tokens < 1 || num_heads < 1 || head_dim < 1 || max_blocks < 1 || split_tiles < 1) return 0;
+  return (int64_t)prefill_ranges(max_blocks, split_tiles) * num_tokens * num_heads * (head_dim + 2) *
+         (int64_t)sizeof(float);
+}
+
+extern "C" int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int64_t q_stride_h,
+                                   const void* k_cache, const void* v_cache,
+                                   int64_t cache_stride_block, int64_t cache_stride_tok,
+                                   int64_t cache_stride_head, int32_t num_blocks,
+                                   const int32_t* block_tables, int64_t bt_stride, int32_t max_blocks,
+                                   const int32_t* query_start_loc, const int32_t* seq_lens,
+                                   const int32_t* context_lens, float scale,
+                                   void* out, int64_t out_stride_t, int64_t out_stride_h,
+                                   int32_t num_seqs, int32_t num_tokens, int32_t max_query_len,
+                                   int32_t single_query_seqs,
+                                   int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                                   int32_t block_size, void* workspace, int32_t split_tiles,
+                                   void* stream) {
+  PrefillArgs a{};
+  bool nothing;
+  const int rc = pack_prefill(a, nothing, q, q_stride_t, q_stride_h, k_cache, v_cache, cache_stride_block, cache_stride_tok,
+                              cache_stride_head, num_blocks, block_tables, bt_stride, max_blocks,
+                              query_start_loc, seq_lens, context_lens, scale, out, out_stride_t, out_stride_h,
+                              num_seqs, num_tokens, max_query_len, single_query_seqs, num_heads, num_kv_heads,
+                              head_dim, block_size);
+  if (rc != 0 || nothing) return rc;
+  if (split_tiles < 1 || split_tiles > (1 << 20) || !workspace || !aligned16(workspace)) return kBad;
+  a.split_tiles = split_tiles;
+  a.num_ranges = prefill_ranges(max_blocks, split_tiles);
+  a.part_out = reinterpret_cast<float*>(workspace);
+  a.part_ml = a.part_out + (int64_t)a.num_ranges * num_tokens * num_heads * head_dim;
   return (int)paged_prefill(a, (hipStream_t)stream);
 }
 

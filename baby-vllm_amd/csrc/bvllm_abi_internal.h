@@ -65,6 +65,11 @@ struct PrefillArgs {
   // Sequences with exactly one query token: -1 = unknown, 0 = none. When not 0
   // those sequences run on the decode kernel and the prefill kernel skips them.
   int32_t single_query_seqs;
+  // Key ranges (split_tiles > 0): 64-key tiles per range, ranges of the longest
+  // sequence the table holds, and the ranges' fp32 partials.
+  int32_t split_tiles, num_ranges;
+  float* part_out;                         // [num_ranges, T, H, D], unnormalized
+  float* part_ml;                          // [num_ranges, T, H, 2]: reference max (log2 units), row sum
 };
 
 struct ArgmaxArgs {
@@ -163,6 +168,12 @@ enum TuneKnob {
 int tuning(int knob);
 int set_tuning(int knob, int value);
 hipError_t paged_prefill(const PrefillArgs& a, hipStream_t stream);
+// Key ranges of a prefill launch: tiles per range (0: no split) for the batch's shape
+// (key_tiles: 64-key tiles its 128-column blocks walk per KV head, or < 0 if unknown).
+int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles);
+inline int32_t prefill_ranges(int32_t max_blocks, int32_t split_tiles) {
+  return ((max_blocks + 3) / 4 + split_tiles - 1) / split_tiles;
+}
 // Compute units of the current device (cached per device).
 int device_cus();
 

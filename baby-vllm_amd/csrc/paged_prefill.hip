@@ -37,7 +37,8 @@
 #include "bvllm_abi_internal.h"
 #include "paged_decode_wg.h"
 
-#include <stdlib.h>
+#include <algorithm>
+#include <cmath>
 
 namespace bvllm {
 
@@ -100,7 +101,13 @@ constexpr int kDecodeDepth = 1;
 // and the two waves of a group take the two 32-key halves of every 64-key tile
 // (twice the columns per LDS read of K and V and per staged tile, for the same
 // waves); their partial states merge through LDS at the end.
-template <int D, int NW, int QT, bool MB, int KS>
+// SPL: a sequence's keys are cut into ranges of a.split_tiles tiles, one
+// work-group per (block, range): few new tokens behind long prefixes would
+// otherwise leave most of the chip idle while a few work-groups walk thousands of
+// keys. A range is a prefill of the sequence shifted by the range's start, so the
+// walk is unchanged; blocks of more than one range write unnormalized fp32
+// partials (with their reference max and row sum) that prefill_merge_kernel adds.
+template <int D, int NW, int QT, bool MB, int KS, bool SPL = false>
 __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a, int n_blocks_bound, int dense_qb,
                                                                   int xcd_group, int per_xcd, DecodeArgs dec,
                                                                   int n_dec_wgs, int bpw) {
@@ -136,6 +143,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
 
   const int G = a.num_heads / a.num_kv_heads;
   static_assert(KS == 1 || (KS == 2 && !MB && NW % 2 == 0), "key split: two halves, streaming path only");
+  static_assert(!SPL || (KS == 1 && !MB), "key ranges: single key walk only");
   constexpr int CB = NW / KS * QT * 16;  // columns of a work-group's block
 
   // Work-groups are dispatched round-robin over the 8 XCDs (XCD = id mod 8).
@@ -146,7 +154,13 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
   // by XCDs h·xcd_group .. +xcd_group-1, which deal its column blocks out in
   // boustrophedon order (0 1 | 1 0 | 0 1 ...): each L2 holds one KV head's
   // keys, and the heavy-to-light run of a sequence's blocks spreads evenly.
-  const int id = blockIdx.x;
+  // SPL: the ranges of a block are `bpw` whole grids apart, on the block's XCD.
+  const int grid_wgs = SPL ? n_pre_wgs / bpw : n_pre_wgs;
+  const int range = SPL ? (int)blockIdx.x / grid_wgs : 0;
+  const int id = SPL ? (int)blockIdx.x - range * grid_wgs : (int)blockIdx.x;
+  const int tile0 = SPL ? range * a.split_tiles : 0;  // first key tile of the range
+  const int max_blocks = SPL ? a.max_blocks - 4 * tile0 : a.max_blocks;
+  if (SPL && max_blocks <= 0) return;
   // The arguments that address the metadata and table loads below, read
   // with the mapping's own: otherwise their wait splits those loads' round trip.
   asm volatile("" ::"s"(a.block_tables), "s"(a.bt_stride), "s"(a.max_blocks), "s"(a.query_start_loc),
@@ -193,7 +207,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
   int ctx = ((ConstI32)a.context_lens)[s];
   constexpr int PAGES_PER_TILE = KT / 16;
   static_assert(PAGES_PER_TILE == 4, "page_finish consumes four entries");
-  const ConstI32 bts = (ConstI32)(a.block_tables + (int64_t)s * a.bt_stride);
+  const ConstI32 bts = (ConstI32)(a.block_tables + (int64_t)s * a.bt_stride + (SPL ? 4 * tile0 : 0));
   const uint32_t page_bytes = (uint32_t)a.c_sb * 2u;  // c_sb < 2^31, checked on the host
   // (No branch between the fast and the clamped form: the waits that close
   // each side of one would split the loads' round trip.)
@@ -207,7 +221,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
   // 2^28 are never needed (seq_len < 2^31 is at most 2^27 pages), which
   // keeps the byte offsets inside 32 bits.
   typedef const char __attribute__((address_space(4)))* ConstBytes;
-  const uint32_t bt_last = (uint32_t)min(a.max_blocks - 1, 1 << 28) * 4u;
+  const uint32_t bt_last = (uint32_t)min(max_blocks - 1, 1 << 28) * 4u;
   const uint32_t page_last = (uint32_t)(a.num_pages - 1);
   auto page_fetch = [&](int kt, int (&raw)[PAGES_PER_TILE]) __attribute__((always_inline)) {
     if constexpr (KS == 2) {
@@ -218,7 +232,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
     } else {
       const int i0 = kt * PAGES_PER_TILE;
 #pragma unroll
-      for (int pg = 0; pg < PAGES_PER_TILE; ++pg) raw[pg] = bts[min(i0 + pg, a.max_blocks - 1)];
+      for (int pg = 0; pg < PAGES_PER_TILE; ++pg) raw[pg] = bts[min(i0 + pg, max_blocks - 1)];
     }
   };
   auto page_finish = [&](int (&raw)[PAGES_PER_TILE], int64_t (&po)[PAGES_PER_TILE]) __attribute__((always_inline)) {
@@ -242,6 +256,10 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
   }
   const int q_len = q_end - q_start;
   const int n_cols = q_len * G;
+  if constexpr (SPL) {  // the sequence as seen from the range's first key
+    ctx -= KT * tile0;
+    seq_len -= KT * tile0;
+  }
   // qb numbers groups of nbpw blocks of CB columns (one block unless MB); the
   // work-group computes the group's blocks one after another, the last (most
   // keys) first. Every block of an MB group reads the same (at most two)
@@ -265,7 +283,9 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
   const int q_last = (min(n_cols, (blk + 1) * CB) - 1) / G;
   // (MB: the host checked that no sequence has more than two tiles' pages;
   // the clamp keeps an inconsistent seq_lens inside the staged tiles.)
-  const int hi = min(min(seq_len, ctx + q_last + 1), MB ? 2 * KT : 0x7fffffff);
+  const int hi_all = min(seq_len, ctx + q_last + 1);
+  const int hi = min(hi_all, MB ? 2 * KT : SPL ? KT * a.split_tiles : 0x7fffffff);
+  if (SPL && range > 0 && hi <= 0) return;
   const int n_tiles = hi > 0 ? (hi + KT - 1) / KT : 0;
 
   // The wave's columns: f = wave_f0 + 16·ct + n of the block's flat
@@ -764,6 +784,21 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
     wait_loads();
   }
 
+  if constexpr (SPL) {
+    if (range > 0 || hi_all > hi) {  // one of several ranges: fp32 partials
+      // Lane n + 16g holds dims 16c + 4g .. +3 of column n.
+#pragma unroll
+      for (int ct = 0; ct < QT; ++ct) {
+        if (!valid[ct]) continue;
+        const int64_t row = ((int64_t)range * a.num_tokens + q_start + qi[ct]) * a.num_heads + kvh * G + hl[ct];
+        float* po = a.part_out + row * D + 4 * g;
+#pragma unroll
+        for (int c = 0; c < VD; ++c) *reinterpret_cast<f32x4_t*>(po + 16 * c) = acc[ct][c];
+        if (g == 0) *reinterpret_cast<float2*>(a.part_ml + row * 2) = make_float2(m[ct], lsum[ct][0]);
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int ct = 0; ct < QT; ++ct) {
     const float lt = lsum[ct][0];
@@ -788,6 +823,76 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
   }
   if (!MB) break;
   } while (--blk >= b_first);
+}
+
+// Adds the key ranges' partials of every (token, head) whose block has more than one
+// range: out = Σ 2^(m_r − M)·o_r / Σ 2^(m_r − M)·l_r over the ranges r in order, M
+// the largest m_r among the ranges with a visible key (l_r ≠ 0), kept online over
+// batches of kMergeBatch ranges. One thread per 4 dims, the token uniform in a
+// work-group. Latency-bound at a few MB of partials: a batch's loads go out
+// together, and so does the search for the token's sequence (one load per 64
+// sequences and a ballot; a binary search and one load at a time per range took
+// 1 x (8000+64) in 16 ranges from 23 to 33 us).
+constexpr int kMergeBatch = 8;
+
+template <int D, int CB>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, int blocks_per_token) {
+  constexpr int TPR = D / 4;  // threads per (token, head)
+  const int t = (int)blockIdx.x / blocks_per_token;
+  const int it = ((int)blockIdx.x - t * blocks_per_token) * 256 + (int)threadIdx.x;
+  // The token's sequence: the number of sequences that start at or before it, less one.
+  int s = -1;
+  for (int s0 = 0; s0 < a.num_seqs; s0 += 64) {
+    const int i = s0 + lane_id();
+    const bool before = i < a.num_seqs && a.query_start_loc[i] <= t;
+    s += __popcll(__builtin_amdgcn_ballot_w64(before));
+  }
+  const int head = it / TPR, d = 4 * (it - head * TPR);
+  if (s < 0 || head >= a.num_heads) return;
+  s = uniform(s);
+  const int q_start = a.query_start_loc[s], q_len = a.query_start_loc[s + 1] - q_start;
+  const int seq_len = a.seq_lens[s], ctx = a.context_lens[s];
+  if (t >= q_start + q_len || (q_len == 1 && a.single_query_seqs != 0)) return;
+  const int G = a.num_heads / a.num_kv_heads;
+  const int blk = ((t - q_start) * G + head % G) / CB;
+  const int q_last = (min(q_len * G, (blk + 1) * CB) - 1) / G;
+  const int hi = min(seq_len, ctx + q_last + 1);
+  const int keys = 64 * a.split_tiles;
+  if (hi <= keys) return;  // a single range wrote the output itself
+  const int nr = min((hi + keys - 1) / keys, a.num_ranges);
+  const int64_t th = (int64_t)t * a.num_heads + head, step = (int64_t)a.num_tokens * a.num_heads;
+  const float* ml = a.part_ml + th * 2;
+  const float* po = a.part_out + th * D + d;
+  float M = kNegInf, den = 0.f;
+  f32x4_t num = {0.f, 0.f, 0.f, 0.f};
+  for (int r0 = 0; r0 < nr; r0 += kMergeBatch) {
+    float2 x[kMergeBatch];
+    f32x4_t o[kMergeBatch];
+#pragma unroll
+    for (int k = 0; k < kMergeBatch; ++k) {
+      const int r = min(r0 + k, nr - 1);
+      x[k] = *reinterpret_cast<const float2*>(ml + r * step * 2);
+      o[k] = *reinterpret_cast<const f32x4_t*>(po + r * step * D);
+    }
+    float Mb = M;
+#pragma unroll
+    for (int k = 0; k < kMergeBatch; ++k)
+      if (x[k].y != 0.f) Mb = fmax_prop(Mb, x[k].x);  // (a range taken twice changes no maximum)
+    const float alpha = M == kNegInf ? 0.f : fast_exp2(M - Mb);
+    den *= alpha;
+    num *= alpha;
+    M = Mb;
+#pragma unroll
+    for (int k = 0; k < kMergeBatch; ++k) {
+      const float wgt = r0 + k < nr && x[k].y != 0.f ? fast_exp2(x[k].x - M) : 0.f;
+      den = __builtin_fmaf(wgt, x[k].y, den);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) num[i] = __builtin_fmaf(wgt, o[k][i], num[i]);
+    }
+  }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  st8(reinterpret_cast<uint16_t*>(a.out) + (int64_t)t * a.o_st + (int64_t)head * a.o_sh + d,
+      make_uint2(pack_bf16x2_hw(num[0] * inv, num[1] * inv), pack_bf16x2_hw(num[2] * inv, num[3] * inv)));
 }
 
 // Decode view of a prefill batch: row b is sequence b; the decode work-group
@@ -888,6 +993,67 @@ static int prefill_blocks_per_wg(const PrefillArgs& a, const PrefillGrid& p1) {
   return (int)((p1.dense_qb + per_pair - 1) / per_pair);
 }
 
+// Key ranges: one work-group per (128-column block, range of a.split_tiles tiles),
+// then the merge.
+template <int D>
+static hipError_t launch_prefill_split(const PrefillArgs& a, hipStream_t stream) {
+  const PrefillGrid p = plan_prefill(a, 4 * 2 * 16);
+  const int64_t wgs = p.prefill_wgs * a.num_ranges;
+  if (wgs + p.dec_wgs == 0) return hipSuccess;
+  if (wgs + p.dec_wgs > 0x7ffffff0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((paged_prefill_kernel<D, 4, 2, false, 1, true>), dim3((unsigned)(p.dec_wgs + wgs)),
+                     dim3(4 * 64), 0, stream, a, (int)p.bound, p.dense_qb, p.xcd_group, (int)p.per_xcd,
+                     single_query_view(a), (int)p.dec_wgs, a.num_ranges);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  const int per_token = (a.num_heads * (D / 4) + 255) / 256;
+  const int64_t blocks = (int64_t)a.num_tokens * per_token;
+  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((prefill_merge_kernel<D, 4 * 2 * 16>), dim3((unsigned)blocks), dim3(256), 0, stream, a,
+                     per_token);
+  return hipGetLastError();
+}
+
+// Whether a batch's keys are cut into ranges, and how long. Only grids short of two
+// 128-column work-groups per CU are looked at. Times (us) as measured here:
+//   unsplit (64-column key split): 7 + 0.79 per tile of the longest walk with at
+//     most one work-group per CU, 1.1 beyond (107 tiles, 176 work-groups: 92;
+//     126 tiles, 28: 106; 71 tiles, 440: 89);
+//   split: 14 of start and merge, + the partials' bytes twice at 8 TB/s, + per tile
+//     1.07 to 1.4 with one work-group per CU, 1.75 with two (the rate of a full
+//     grid). Ranges shorter than 8 tiles gain nothing over their fixed cost.
+// The ranges are made as short as one round of work-groups allows: a second round
+// pays the fixed part again (4 sequences of 2-8 thousand cached + 30-200 new tokens:
+// 60 us at 13 tiles per range, 46 at 15, 51 at 20, 75 at 48; 92 unsplit). 0.86 of the
+// slots, since blocks fall unevenly on the XCDs; one work-group per CU beside decode
+// rows (100 new tokens behind 6000 + 20 rows: 44 us at 7 tiles, 34 at 15; 83 unsplit).
+int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles) {
+  const PrefillGrid p = plan_prefill(a, 4 * 2 * 16);
+  const double cus = device_cus(), hkv = a.num_kv_heads;
+  if (p.bound <= 0 || p.prefill_wgs >= 2 * (int64_t)cus) return 0;
+  const double longest = (a.max_blocks + 3) / 4;
+  const double steps = hkv * (key_tiles >= 0 ? (double)key_tiles : p.bound * longest);
+  const double blocks = hkv * p.bound;
+  const double walk = std::min(longest, std::max(steps / hkv, 1.0));
+  const double unsplit = 7.0 + (2.0 * blocks <= cus ? 0.79 : 1.1) * walk;
+  double best = 0.9 * unsplit;
+  int32_t tiles = 0;
+  for (int per_cu = 1; per_cu <= (p.dec_wgs > 0 ? 1 : 2); ++per_cu) {
+    const double slots = (per_cu == 1 ? 0.98 : 1.72) * cus - (double)p.dec_wgs - blocks / 2;
+    if (slots <= 0) continue;
+    const double c = std::max(8.0, std::ceil(steps / slots));
+    if (c >= longest) continue;
+    const double ranges = steps / (blocks * c) + 0.5;
+    const double bytes = (double)a.num_tokens * a.num_heads * (a.head_dim + 2) * 4 * ranges;
+    const double t = 14.0 + 2 * bytes / 8e6 + (per_cu == 1 ? 1.3 : 1.75) * c;
+    if (t < best) {
+      best = t;
+      tiles = (int32_t)c;
+    }
+  }
+  return tiles;
+}
+
 // Two column tiles per wave (128 columns per work-group) unless that grid
 // gives fewer than two prefill work-groups per CU (short batches, mixed
 // steps): then 64 columns per work-group, twice the work-groups, computed by
@@ -897,6 +1063,7 @@ static int prefill_blocks_per_wg(const PrefillArgs& a, const PrefillGrid& p1) {
 // kTunePrefillShortGrid; mixed 1 x 512 + 63 decodes: 29.3-30.0 us either way).
 template <int D>
 static hipError_t prefill_for_dim(const PrefillArgs& a, hipStream_t stream) {
+  if (a.split_tiles > 0) return launch_prefill_split<D>(a, stream);
   const PrefillGrid p2 = plan_prefill(a, 4 * 2 * 16);
   if (p2.prefill_wgs >= 2 * (int64_t)device_cus()) {
     const int bpw = prefill_blocks_per_wg(a, p2);

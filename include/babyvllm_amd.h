@@ -180,6 +180,37 @@ BVLLM_API int bvllm_paged_prefill(const void* q, int64_t q_stride_t, int64_t q_s
                         int32_t block_size, void* stream);
 
 /*
+ * The same, with each sequence's keys cut into ranges of split_tiles 64-key tiles,
+ * every (block, range) on a work-group of its own, and a second launch that adds the
+ * ranges' fp32 partials: for few new tokens behind long prefixes, where the plain
+ * launch leaves most of the chip idle. bvllm_prefill_split_tiles returns the
+ * split_tiles to use for a batch's shape, or 0 where the plain launch is the better one;
+ * key_tiles is the number of 64-key tiles the batch's blocks of 128 (query, head)
+ * pairs cover, per KV head, summed over its sequences of more than one query token
+ * (ceil(G * q_len / 128) * ceil(seq_len / 64)), or -1 if unknown; it steers the choice
+ * only, never what is computed. workspace holds bvllm_prefill_workspace_bytes() bytes.
+ * Results agree with bvllm_paged_prefill within the rounding of fp32 sums in another
+ * order. A sequence's keys end at its table's last page.
+ */
+BVLLM_API int32_t bvllm_prefill_split_tiles(int32_t num_seqs, int32_t num_tokens, int32_t max_query_len,
+                        int32_t single_query_seqs, int32_t num_heads, int32_t num_kv_heads,
+                        int32_t head_dim, int32_t max_blocks, int64_t key_tiles);
+BVLLM_API int64_t bvllm_prefill_workspace_bytes(int32_t num_tokens, int32_t num_heads, int32_t head_dim,
+                        int32_t max_blocks, int32_t split_tiles);
+BVLLM_API int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int64_t q_stride_h,
+                        const void* k_cache, const void* v_cache,
+                        int64_t cache_stride_block, int64_t cache_stride_tok, int64_t cache_stride_head,
+                        int32_t num_blocks,
+                        const int32_t* block_tables, int64_t bt_stride, int32_t max_blocks,
+                        const int32_t* query_start_loc, const int32_t* seq_lens,
+                        const int32_t* context_lens, float scale,
+                        void* out, int64_t out_stride_t, int64_t out_stride_h,
+                        int32_t num_seqs, int32_t num_tokens, int32_t max_query_len,
+                        int32_t single_query_seqs,
+                        int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                        int32_t block_size, void* workspace, int32_t split_tiles, void* stream);
+
+/*
  * Tuning switch for experiments and tests (no counterpart in the reference):
  * sets process-wide knob `knob` to `value` (0 = the library's default) and
  * returns the previous value, or -1 for an unknown knob. Knobs: 0 decode split

@@ -407,3 +407,50 @@ def test_gqa_groups_above_16(name, hkv, group, d):
     with tuned(_SHORT_GRID, 1):
         walk = _kernel()(q, kv_cache, md, d ** -0.5)
     assert_attn_close(walk, expected)
+
+
+# Key ranges (bvllm_paged_prefill_split), forced to a few tiles per range: a range's
+# edge inside the new tokens, ranges some columns of a block do not see, blocks of one
+# range beside blocks of many, more ranges than one merge batch, decode rows in the
+# same launch, and GQA groups whose blocks split a query's heads.
+SPLIT_CASES = {
+    "range_edges": [(63, 2), (64, 1), (0, 65), (127, 130), (1, 64)],
+    "short_beside_long": [(0, 5), (3000, 40), (0, 1), (700, 1), (1500, 300)],
+    "one_query_block_long_prefix": [(2500, 3)],
+    "fresh_long": [(0, 900)],
+}
+
+
+@pytest.mark.parametrize("tiles", [1, 2, 5])
+@pytest.mark.parametrize("case", list(SPLIT_CASES))
+@pytest.mark.parametrize("hkv,group,d", [(4, 7, 128), (2, 7, 64), (1, 33, 128)])
+def test_key_ranges_match_oracle(case, tiles, hkv, group, d, monkeypatch):
+    import babyvllm.kernels.paged_prefill as pp
+
+    q, kv_cache, md = build_prefill_case(SPLIT_CASES[case], hkv, group, d)
+    scale_keys_by_position(kv_cache, md.block_tables, md.seq_lens_cpu, lambda p: 1.0 + 0.002 * p)
+    expected = _oracle(q, kv_cache, md, group)
+    plain = _kernel()(q, kv_cache, md, d ** -0.5)
+    monkeypatch.setattr(pp, "_split_tiles", lambda *a: tiles)
+    actual = _kernel()(q, kv_cache, md, d ** -0.5)
+    assert_attn_close(actual, expected)
+    # No further from the oracle than the plain launch, up to the merge's fp32 rounding.
+    off = (actual.float().cpu() - expected).norm()
+    assert off <= 1.02 * (plain.float().cpu() - expected).norm() + 1e-4
+
+
+def test_key_ranges_chosen_for_short_turns_behind_long_prefixes():
+    import babyvllm.kernels.paged_prefill as pp
+
+    specs = [(2300, 40), (6000, 70), (4000, 150), (3000, 1)]
+    q, kv_cache, md = build_prefill_case(specs, 4, 7, 128)
+    width = md.block_tables.shape[1]
+    args = (md, len(specs), q.shape[0], 1, 28, 4, 128)
+    tiles = pp._split_tiles(*args, width)
+    assert 8 <= tiles < width // 4
+    assert_attn_close(_kernel()(q, kv_cache, md, 128 ** -0.5), _oracle(q, kv_cache, md, 7))
+    md.seq_lens_cpu = None  # no host lists: the table's width stands in
+    assert 8 <= pp._split_tiles(*args, width) <= width // 4
+    # Wide tables beside a full grid, and narrow tables, keep the plain launch.
+    assert pp._split_tiles(build_prefill_case([(2048, 2048)], 4, 7, 128)[2], 1, 2048, 0, 28, 4, 128, 256) == 0
+    assert pp._split_tiles(*args, 8) == 0
