@@ -48,6 +48,18 @@ SIGNATURES = {
         _i32, _i32, _i32, _i32, _i32, _i32,  # B, H, Hkv, D, block_size, waves
         _p,                         # stream
     ]),
+    "bvllm_decode_balanced_workspace_bytes": (ctypes.c_int64, [_i32, _i32, _i32, _i32]),
+    "bvllm_paged_decode_balanced": (ctypes.c_int, [
+        _p, _i64, _i64,             # q
+        _p, _p, _i64, _i64, _i64,   # caches + strides
+        _i32,                       # num_blocks
+        _p, _i64, _i32,             # block_tables, bt_stride, max_blocks
+        _p, _f32,                   # seq_lens, scale
+        _p, _i64, _i64,             # out
+        _p,                         # workspace
+        _i32, _i32, _i32, _i32, _i32,  # B, H, Hkv, D, block_size
+        _p,                         # stream
+    ]),
     "bvllm_paged_decode_noalloc": (ctypes.c_int, [
         _p, _i64, _i64,             # q
         _p, _p, _i64, _i64, _i64,   # caches + strides

@@ -16,11 +16,18 @@ no device-to-host read.
 from __future__ import annotations
 
 import functools
+import os
 
 import torch
 
 from babyvllm.kernels import _lib
-from babyvllm.kernels.decode_split import decode_split_plan
+from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV, decode_split_plan
+
+# A single-pass plan ("auto") sized for more pages than this runs the balanced launch
+# (bvllm_paged_decode_balanced). Shorter rows can lose less to each other than its second
+# launch costs equal ones (64 x 2048: 45.1 against 46.4 us; 64 rows of 200 to 2048: 30.2
+# against 27.1; 64 of 100 to 4096: 52 against 34; 64 x 4096: 86.7 against 87.7).
+BALANCE_MIN_PAGES = 128
 
 
 @functools.lru_cache(maxsize=None)
@@ -70,21 +77,28 @@ def paged_decode_attention(q, kv_cache, block_tables, seq_lens, scale,
     out = torch.empty(B, n_heads, head_dim, device=q.device, dtype=q.dtype)
     if B == 0:
         return out
-    workspace = None
-    nbytes = _lib.lib().bvllm_decode_workspace_bytes(B, n_heads, n_kv_heads, head_dim, num_splits,
-                                                     blocks_per_split)
-    if nbytes > 0:
-        workspace = torch.empty(nbytes // 4, device=q.device, dtype=torch.float32)
-    rc = _lib.lib().bvllm_paged_decode(
+    h = _lib.lib()
+    args = (
         q.data_ptr(), q.stride(0), q.stride(1),
         k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1), k_cache.stride(2),
         num_blocks,
         block_tables.data_ptr(), block_tables.stride(0), width,
         seq_lens.data_ptr(), float(scale),
         out.data_ptr(), out.stride(0), out.stride(1),
-        None if workspace is None else workspace.data_ptr(), num_splits, blocks_per_split,
-        B, n_heads, n_kv_heads, head_dim, block_size, 0,
-        _lib.stream_handle(q.device),
     )
+    balanced = num_splits == 1 and blocks_per_split > BALANCE_MIN_PAGES and partition_blocks is None \
+        and os.environ.get(DECODE_PARTITION_ENV, "auto") == "auto"
+    if balanced:
+        nbytes = h.bvllm_decode_balanced_workspace_bytes(B, n_heads, n_kv_heads, head_dim)
+    else:
+        nbytes = h.bvllm_decode_workspace_bytes(B, n_heads, n_kv_heads, head_dim, num_splits, blocks_per_split)
+    workspace = torch.empty(nbytes // 4, device=q.device, dtype=torch.float32) if nbytes > 0 else None
+    ws = None if workspace is None else workspace.data_ptr()
+    stream = _lib.stream_handle(q.device)
+    if balanced:
+        rc = h.bvllm_paged_decode_balanced(*args, ws, B, n_heads, n_kv_heads, head_dim, block_size, stream)
+    else:
+        rc = h.bvllm_paged_decode(*args, ws, num_splits, blocks_per_split,
+                                  B, n_heads, n_kv_heads, head_dim, block_size, 0, stream)
     _lib.check(rc, "bvllm_paged_decode")
     return out

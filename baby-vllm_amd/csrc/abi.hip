@@ -133,6 +133,50 @@ extern "C" int bvllm_paged_decode(const void* q, int64_t q_stride_b, int64_t q_s
   return (int)paged_decode(a, (hipStream_t)stream);
 }
 
+extern "C" int64_t bvllm_decode_balanced_workspace_bytes(int32_t batch, int32_t num_heads, int32_t num_kv_heads,
+                                                         int32_t head_dim) {
+  if (batch <= 0 || !valid_heads(num_heads, num_kv_heads) || head_dim <= 0) return 0;
+  return decode_chunk_slots(batch, num_heads, num_kv_heads) * num_heads * (head_dim + 1) * (int64_t)sizeof(float);
+}
+
+extern "C" int bvllm_paged_decode_balanced(const void* q, int64_t q_stride_b, int64_t q_stride_h,
+                                  const void* k_cache, const void* v_cache,
+                                  int64_t cache_stride_block, int64_t cache_stride_tok,
+                                  int64_t cache_stride_head, int32_t num_blocks,
+                                  const int32_t* block_tables, int64_t bt_stride, int32_t max_blocks,
+                                  const int32_t* seq_lens, float scale,
+                                  void* out, int64_t out_stride_b, int64_t out_stride_h,
+                                  void* workspace,
+                                  int32_t batch, int32_t num_heads, int32_t num_kv_heads,
+                                  int32_t head_dim, int32_t block_size, void* stream) {
+  if (batch < 0 || !valid_heads(num_heads, num_kv_heads)) return kBad;
+  if (head_dim != 64 && head_dim != 128) return kBad;
+  if (block_size != 16) return kBad;
+  if (batch == 0) return 0;
+  if (!q || !out || !block_tables || !seq_lens || !workspace || !aligned16(workspace)) return kBad;
+  if (!cache_ok(k_cache, v_cache, cache_stride_block, cache_stride_tok, cache_stride_head, num_blocks))
+    return kBad;
+  if (!aligned16(q) || !aligned16(out) || q_stride_b % 8 || q_stride_h % 8 || out_stride_b % 8 ||
+      out_stride_h % 8)
+    return kBad;
+  if (max_blocks < 1 || bt_stride < max_blocks) return kBad;
+  if ((int64_t)16 * cache_stride_tok > 0x7fffffff) return kBad;  // offsets inside one page are 32-bit
+  DecodeArgs a{};
+  a.q = q; a.q_sb = q_stride_b; a.q_sh = q_stride_h;
+  a.k_cache = k_cache; a.v_cache = v_cache;
+  a.c_sb = cache_stride_block; a.c_st = cache_stride_tok; a.c_sh = cache_stride_head;
+  a.num_pages = num_blocks;
+  a.block_tables = block_tables; a.bt_stride = bt_stride; a.max_blocks = max_blocks;
+  a.seq_lens = seq_lens;
+  a.scale_log2 = scale * kLog2e;
+  a.out = out; a.o_sb = out_stride_b; a.o_sh = out_stride_h;
+  a.part_out = reinterpret_cast<float*>(workspace);
+  a.part_lse = a.part_out + decode_chunk_slots(batch, num_heads, num_kv_heads) * num_heads * head_dim;
+  a.num_splits = 1; a.blocks_per_split = max_blocks;
+  a.batch = batch; a.num_heads = num_heads; a.num_kv_heads = num_kv_heads; a.head_dim = head_dim;
+  return (int)paged_decode_balanced(a, (hipStream_t)stream);
+}
+
 // Checks and packs a prefill call; `nothing` is set when there is nothing to compute.
 static int pack_prefill(PrefillArgs& a, bool& nothing, const void* q, int64_t q_stride_t, int64_t q_stride_h,
                         const void* k_cache, const void* v_cache,

@@ -26,20 +26,7 @@ constexpr int vec_chunk() { return kVecLoads * kArgmaxThreads * (16 / (int)sizeo
 
 // ------------------------------------------------------ wave reductions
 //
-// Wave-wide maximum / minimum by DPP and lane swaps (VALU only, no LDS round
-// trip): quad swaps (lanes l ^ 1, then l ^ 2), mirrors within 8 and within 16
-// lanes, then the 16- and 32-lane swaps. Each step combines a lane with a
-// partner holding the other half of its current group, so every lane ends
-// with the result for the whole wave.
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xf, 0xf, false);
-}
-constexpr int kQuadSwap1 = 0xB1;     // quad_perm [1, 0, 3, 2]
-constexpr int kQuadSwap2 = 0x4E;     // quad_perm [2, 3, 0, 1]
-constexpr int kRowHalfMirror = 0x141;
-constexpr int kRowMirror = 0x140;
-
+// The lane steps of wave_reduce.
 // NaN-propagating: the result is NaN if any lane holds a NaN.
 __device__ __forceinline__ float wave_maximum(float x) {
   x = fmax_prop(x, __uint_as_float(dpp<kQuadSwap1>(__float_as_uint(x))));
@@ -50,14 +37,7 @@ __device__ __forceinline__ float wave_maximum(float x) {
 }
 
 __device__ __forceinline__ int wave_min(int x) {
-  x = min(x, (int)dpp<kQuadSwap1>((uint32_t)x));
-  x = min(x, (int)dpp<kQuadSwap2>((uint32_t)x));
-  x = min(x, (int)dpp<kRowHalfMirror>((uint32_t)x));
-  x = min(x, (int)dpp<kRowMirror>((uint32_t)x));
-  const auto a = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
-  x = min((int)a[0], (int)a[1]);
-  const auto b = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
-  return min((int)b[0], (int)b[1]);
+  return wave_reduce(x, [](int a, int b) { return min(a, b); });
 }
 
 // Work-group maximum (NaN-propagating) and minimum over the 4 waves, through

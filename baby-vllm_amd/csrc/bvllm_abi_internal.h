@@ -41,6 +41,9 @@ struct DecodeArgs {
   int32_t num_partials;                    // partial states per (row, head) the launch writes
   int32_t ws_partials;                     // partial states per (row, head) the workspace holds
   int32_t item_order;                      // 0: KV head fastest in the wave numbering; 1: split unit fastest
+  // Balanced single pass (RowChunk): chunks aimed at per column group, rows an even
+  // share of which keeps every CU busy.
+  int32_t chunk_target, row_slots;
   // Prefill view (both null for a decode batch): row b is sequence b of a
   // varlen prefill batch. Only sequences with exactly one query token are
   // computed; their q / out row is query_start_loc[b] and they attend keys
@@ -128,6 +131,10 @@ hipError_t greedy_argmax(const ArgmaxArgs& a, hipStream_t stream);
 hipError_t fused_add_rms_norm(const NormArgs& a, hipStream_t stream);
 hipError_t silu_mul(const SiluArgs& a, hipStream_t stream);
 hipError_t paged_decode(const DecodeArgs& a, hipStream_t stream);
+// The single pass with long rows cut into chunks (paged_decode.hip). The partials hold
+// decode_chunk_slots() results per query head: [slots, H, D] and [slots, H].
+hipError_t paged_decode_balanced(const DecodeArgs& a, hipStream_t stream);
+int64_t decode_chunk_slots(int32_t batch, int32_t num_heads, int32_t num_kv_heads);
 
 // How a decode launch with the caller's split plan runs (paged_decode.hip).
 struct DecodePlan {

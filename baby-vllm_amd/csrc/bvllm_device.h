@@ -96,6 +96,32 @@ __device__ __forceinline__ float sum_across_groups(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// x of the lane that DPP control CTRL names, over the whole wave.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xf, 0xf, false);
+}
+constexpr int kQuadSwap1 = 0xB1;     // quad_perm [1, 0, 3, 2]
+constexpr int kQuadSwap2 = 0x4E;     // quad_perm [2, 3, 0, 1]
+constexpr int kRowHalfMirror = 0x141;
+constexpr int kRowMirror = 0x140;
+
+// Wave-wide reduction of a commutative, associative integer op by DPP and lane
+// swaps (VALU only, no LDS round trip): quad swaps (lanes l ^ 1, then l ^ 2),
+// mirrors within 8 and within 16 lanes, then the 16- and 32-lane swaps. Every lane
+// ends with the result for the whole wave.
+template <typename Op>
+__device__ __forceinline__ int wave_reduce(int x, Op op) {
+  x = op(x, (int)dpp<kQuadSwap1>((uint32_t)x));
+  x = op(x, (int)dpp<kQuadSwap2>((uint32_t)x));
+  x = op(x, (int)dpp<kRowHalfMirror>((uint32_t)x));
+  x = op(x, (int)dpp<kRowMirror>((uint32_t)x));
+  const auto a = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
+  x = op((int)a[0], (int)a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
+  return op((int)b[0], (int)b[1]);
+}
+
 __device__ __forceinline__ int wave_id() {
   return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }

@@ -20,6 +20,58 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(DecodeArgs a) {
   decode_work_group<D, NW, PF, EAGER>(a, blockIdx.x, smem);
 }
 
+__device__ __forceinline__ void store_reduced(const DecodeArgs& a, int64_t bh, int d, float4 num, float den);
+
+template <int D, int NW, int PF, bool EAGER>
+__global__ __launch_bounds__(NW * 64) void paged_decode_chunks_kernel(DecodeArgs a) {
+  extern __shared__ float smem[];
+  decode_work_group<D, NW, PF, EAGER, true>(a, blockIdx.x, smem);
+}
+
+// Merges the chunks of the rows that have several (RowChunk): with w_c =
+// 2^(lse_c − M), out = Σ w_c·o_c / Σ w_c in chunk order, M kept online over batches
+// of chunks whose loads go out together. One row per work-group column, one thread
+// per 4 dims; rows of one chunk were written by their work-group.
+template <int D>
+__global__ __launch_bounds__(256) void decode_chunks_merge_kernel(DecodeArgs a, int blocks_per_row) {
+  constexpr int BATCH = 8;
+  const int row = (int)blockIdx.x / blocks_per_row;
+  const int it = ((int)blockIdx.x - row * blocks_per_row) * 256 + (int)threadIdx.x;
+  const RowChunk ck = find_row_chunk(a, -1, row);
+  if (ck.count <= 1) return;
+  const int head = it / (D / 4), d = 4 * (it - head * (D / 4));
+  if (head >= a.num_heads) return;
+  const int64_t p0 = (int64_t)ck.index * a.num_heads + head;
+  float M = kNegInf, den = 0.f;
+  f32x4_t num = {0.f, 0.f, 0.f, 0.f};
+  for (int c0 = 0; c0 < ck.count; c0 += BATCH) {
+    float lse[BATCH];
+    f32x4_t o[BATCH];
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) {
+      const int64_t p = p0 + (int64_t)min(c0 + k, ck.count - 1) * a.num_heads;
+      lse[k] = a.part_lse[p];
+      o[k] = *reinterpret_cast<const f32x4_t*>(a.part_out + p * D + d);
+    }
+    float Mb = M;
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) Mb = fmaxf(Mb, lse[k]);
+    const float ref = Mb == kNegInf ? 0.f : Mb;
+    const float alpha = fast_exp2(M - ref);
+    den *= alpha;
+    num *= alpha;
+    M = Mb;
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) {
+      const float wgt = c0 + k < ck.count ? fast_exp2(lse[k] - ref) : 0.f;
+      den += wgt;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) num[i] = __builtin_fmaf(wgt, o[k][i], num[i]);
+    }
+  }
+  store_reduced(a, (int64_t)row * a.num_heads + head, d, make_float4(num[0], num[1], num[2], num[3]), den);
+}
+
 // One streaming wave per work-group, so that a short batch's splits spread
 // over every CU.
 template <int D, int PF, bool NT, bool GROUP>
@@ -434,6 +486,45 @@ static hipError_t launch_decode(const DecodeArgs& args, hipStream_t stream) {
   }
   if (err != hipSuccess || p.single_pass) return err;
   return launch_reduce<D>(a, p, stream);
+}
+
+// Chunks a balanced launch aims at, per column group: 1.5 per CU.
+static int32_t chunk_target(int64_t ncg) { return (int32_t)std::max<int64_t>(1, 3 * (int64_t)device_cus() / (2 * ncg)); }
+
+int64_t decode_chunk_slots(int32_t batch, int32_t num_heads, int32_t num_kv_heads) {
+  const int G = num_heads / num_kv_heads;
+  // Σ max(1, ceil(n_b / pages)) with pages >= Σ n_b / target.
+  return (int64_t)batch + chunk_target((int64_t)num_kv_heads * ((G + 15) / 16));
+}
+
+template <int D>
+static hipError_t launch_decode_balanced(const DecodeArgs& args, hipStream_t stream) {
+  DecodeArgs a = args;
+  const int64_t ncg = decode_col_groups(a);
+  a.chunk_target = chunk_target(ncg);
+  a.row_slots = (int32_t)std::max<int64_t>(1, device_cus() / ncg);
+  constexpr int NW = 4;
+  constexpr size_t smem = decode_lds_bytes<D, NW>();
+  static std::atomic<bool> done[64] = {};
+  hipError_t err = allow_lds(&paged_decode_chunks_kernel<D, NW, 1, true>, done, 160 * 1024);
+  if (err != hipSuccess) return err;
+  const int64_t wgs = decode_chunk_slots(a.batch, a.num_heads, a.num_kv_heads) * ncg;
+  const int per_row = (a.num_heads * (D / 4) + 255) / 256;
+  if (wgs > 0x7fffffff || (int64_t)a.batch * per_row > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((paged_decode_chunks_kernel<D, NW, 1, true>), dim3((unsigned)wgs), dim3(NW * 64), smem, stream, a);
+  err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL((decode_chunks_merge_kernel<D>), dim3((unsigned)(a.batch * per_row)), dim3(256), 0, stream, a,
+                     per_row);
+  return hipGetLastError();
+}
+
+hipError_t paged_decode_balanced(const DecodeArgs& a, hipStream_t stream) {
+  switch (a.head_dim) {
+    case 64: return launch_decode_balanced<64>(a, stream);
+    case 128: return launch_decode_balanced<128>(a, stream);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t paged_decode(const DecodeArgs& a, hipStream_t stream) {

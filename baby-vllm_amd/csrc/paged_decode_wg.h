@@ -292,9 +292,11 @@ __device__ __forceinline__ float split_lse(float M, float L) { return L > 0.f ? 
 // out by save_state), and writes those dims of the bf16 output rows of the G
 // heads head0 .. head0 + G - 1 (one column group): lane (n, g) writes head n,
 // dims VD·(4g + e) .. +VD-1.
+// part >= 0: one of several chunks of the row (RowChunk): the fp32 (o, lse) of the
+// chunk go to slot `part` of the partials instead.
 template <int D>
 __device__ __forceinline__ void merge_states(const DecodeArgs& a, const float* rec, int e, int G, int row,
-                                             int head0, int lane) {
+                                             int head0, int lane, int part = -1) {
   constexpr int VD = D / 16;
   const int n = lane & 15;
   const int g = lane >> 4;
@@ -323,6 +325,16 @@ __device__ __forceinline__ void merge_states(const DecodeArgs& a, const float* r
   const float inv = split_inv(L);
 #pragma unroll
   for (int c = 0; c < VD; ++c) o[c] = L == 0.f ? 0.f : o[c] * inv;
+  if (part >= 0) {  // uniform
+    if (n < G) {
+      const int64_t prow = (int64_t)part * a.num_heads + head0 + n;
+      float* dst = a.part_out + prow * D + VD * (4 * g + e);
+#pragma unroll
+      for (int c = 0; c < VD; c += 4) *reinterpret_cast<f32x4_t*>(dst + c) = f32x4_t{o[c], o[c + 1], o[c + 2], o[c + 3]};
+      if (g == 0 && e == 0) a.part_lse[prow] = split_lse(M, L);
+    }
+    return;
+  }
   if (n < G) {
     uint16_t* dst = reinterpret_cast<uint16_t*>(a.out) + (int64_t)row * a.o_sb + (int64_t)(head0 + n) * a.o_sh +
                     VD * (4 * g + e);
@@ -350,6 +362,89 @@ constexpr size_t decode_lds_bytes() {
   return (size_t)NW * kTileBytes<D> + (size_t)kMergeFloats<D> * sizeof(float);
 }
 
+// Row chunks of a balanced single pass. A batch whose plan is one split per row has
+// one work-group per (row, column group); when its rows are far from equal (or
+// fewer than the CUs serve at once) the longest rows run on while the rest of the
+// chip idles. The balanced launch cuts every row into chunks of whole pages, a
+// multiple of 4 (so that a page keeps its state), at most `pages` each: all pages of
+// the batch / a.chunk_target (1.5 per CU: 48 rows of 200 to 16384 tokens 182 -> 69 us;
+// one per CU 84, two 75, three 74), at least kMinChunkPages. No row is cut while the
+// longest is within 1.75 times an even share of a.row_slots, where the second pass
+// over partials costs more than it gives (36 equal rows of 4096: 1.78 shares, 63 -> 58
+// us cut; 40 of 2000: 1.6, 34 -> 37). Chunks are numbered row by row; a row of one chunk
+// is computed and written exactly as in the single pass, the others' fp32 (o, lse)
+// are merged by decode_chunks_merge_kernel. Finding the chunk and the empty merge
+// cost a batch that is not cut 1.1 us (64 x 4096: 86.7 -> 87.7).
+// Nor is any row cut while the longest has at most kCutMinPages pages, the size of
+// plan below which callers run the plain single pass: both give the same bits there.
+constexpr int kMinChunkPages = 32;
+constexpr int kCutMinPages = 128;
+
+struct RowChunk {
+  int pages;  // pages per chunk of the row
+  int row;    // the chunk's row (-1: no such chunk)
+  int index;  // which of the row's chunks
+  int count;  // chunks of the row
+};
+
+// Chunk number `item` (item >= 0), or the chunks of row `item_row` (item < 0: `row`
+// then is item_row and `index` the number of its first chunk). Every wave computes the
+// same answer from the batch's lengths, 64 rows per step.
+__device__ __forceinline__ RowChunk find_row_chunk(const DecodeArgs& a, int item, int item_row) {
+  const int lane = lane_id();
+  auto row_pages = [&](int b) {
+    const int len = b < a.batch ? a.seq_lens[b] : 0;
+    return min(len > 0 ? (len + 15) / 16 : 0, a.max_blocks);
+  };
+  const int n0 = row_pages(lane);
+  int total = 0, longest = 0;
+  for (int b0 = 0; b0 < a.batch; b0 += 64) {
+    const int n = b0 == 0 ? n0 : row_pages(b0 + lane);
+    total += wave_reduce(n, [](int x, int y) { return x + y; });
+    longest = max(longest, wave_reduce(n, [](int x, int y) { return max(x, y); }));
+  }
+  total = uniform(total);
+  longest = uniform(longest);
+  RowChunk r;
+  r.row = -1;
+  r.index = r.count = 0;
+  r.pages = (longest + 3) / 4 * 4;
+  if (longest <= kCutMinPages || 4 * (int64_t)longest * a.row_slots <= 7 * (int64_t)total) {  // no cut: chunk i is row i
+    r.row = item >= 0 ? (item < a.batch ? item : -1) : item_row;
+    r.index = item >= 0 ? 0 : item_row;
+    r.count = 1;
+    return r;
+  }
+  const int even = (total + a.chunk_target - 1) / a.chunk_target;
+  r.pages = max((even + 3) / 4 * 4, kMinChunkPages);
+  int before = 0;
+  for (int b0 = 0; b0 < a.batch; b0 += 64) {
+    const int b = b0 + lane;
+    const int n = b0 == 0 ? n0 : row_pages(b);
+    // (A row with no live token is one empty chunk: it writes zeros.)
+    const int chunks = b < a.batch ? max((n + r.pages - 1) / r.pages, 1) : 0;
+    int inc = chunks;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int t = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += t;
+    }
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(item >= 0 ? before + inc > item : b == item_row);
+    if (hit != 0) {
+      const int l = (int)__builtin_ctzll(hit);
+      const int first = before + __shfl(inc - chunks, l, 64);
+      r.row = uniform(b0 + l);
+      r.count = uniform(__shfl(chunks, l, 64));
+      r.index = uniform(item >= 0 ? item - first : first);
+      // The row's pages evenly over its chunks, in multiples of 4.
+      r.pages = (uniform(__shfl(n, l, 64)) + 4 * r.count - 1) / (4 * r.count) * 4;
+      return r;
+    }
+    before += __shfl(inc, 63, 64);
+  }
+  return r;
+}
+
 // One single-pass decode work-group: (sequence, column group) = wg (a column
 // group is a KV head when G <= 16), with NW waves and `smem` pointing at
 // decode_lds_bytes<D, NW>() bytes of LDS. Wave w walks the row's pages w,
@@ -358,7 +453,8 @@ constexpr size_t decode_lds_bytes() {
 // EAGER (PF = 1): page k+1 is requested as soon as page k has landed, before
 // page k is computed (two register sets), instead of after; the page order, so
 // the arithmetic, is the same either way.
-template <int D, int NW, int PF, bool EAGER = false>
+// CHUNKS: wg is (chunk number, column group) of a balanced launch (find_row_chunk).
+template <int D, int NW, int PF, bool EAGER = false, bool CHUNKS = false>
 __device__ __forceinline__ void decode_work_group(const DecodeArgs& a, const int wg, float* smem) {
   constexpr int KC = D / 32;
   constexpr int VD = D / 16;
@@ -367,7 +463,13 @@ __device__ __forceinline__ void decode_work_group(const DecodeArgs& a, const int
   const ColGroup cgp = col_group(a.num_heads / a.num_kv_heads, wg % ncg);
   const int G = cgp.cols;  // heads of this column group
   const int kvh = cgp.kvh;
-  const int b = wg / ncg;
+  RowChunk ck{};
+  if constexpr (CHUNKS) {
+    ck = find_row_chunk(a, wg / ncg, 0);
+    if (ck.row < 0) return;  // past the last chunk (uniform)
+  }
+  const int b = CHUNKS ? ck.row : wg / ncg;
+  const int page0 = CHUNKS ? ck.index * ck.pages : 0;  // first page of the chunk
 
   const int lane = lane_id();
   const int n = lane & 15;
@@ -385,6 +487,7 @@ __device__ __forceinline__ void decode_work_group(const DecodeArgs& a, const int
   }
   int n_blocks = seq_len > 0 ? (seq_len + 15) / 16 : 0;
   n_blocks = min(n_blocks, a.max_blocks);
+  if constexpr (CHUNKS) n_blocks = min(n_blocks, page0 + ck.pages);
 
   // Qᵀ operand: lane (n + 16g), chunk c -> q[b][head0 + n][8(4c+g) .. +8).
   uint4 qb[KC];
@@ -410,7 +513,7 @@ __device__ __forceinline__ void decode_work_group(const DecodeArgs& a, const int
   const uint16_t* vc = reinterpret_cast<const uint16_t*>(a.v_cache) + (int64_t)kvh * a.c_sh;
   const int32_t* bt = a.block_tables + (int64_t)b * a.bt_stride;
 
-  const int first = w;
+  const int first = page0 + w;
   const int cnt = (n_blocks > first) ? (n_blocks - first + NW - 1) / NW : 0;
   // Lane k holds the table entry of this wave's page number base + k. The first
   // slice is requested together with seq_len and q (its index is clamped into
@@ -489,7 +592,7 @@ __device__ __forceinline__ void decode_work_group(const DecodeArgs& a, const int
   float* merge = smem + NW * kTileBytes<D> / 4;
   save_state<D>(merge, st, w, lane);
   __syncthreads();
-  merge_states<D>(a, merge, w, G, row, cgp.head0, lane);
+  merge_states<D>(a, merge, w, G, row, cgp.head0, lane, CHUNKS && ck.count > 1 ? wg / ncg : -1);
 }
 
 }  // namespace bvllm

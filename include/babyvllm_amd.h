@@ -120,6 +120,28 @@ BVLLM_API int bvllm_paged_decode(const void* q, int64_t q_stride_b, int64_t q_st
                        int32_t head_dim, int32_t block_size, int32_t waves, void* stream);
 
 /*
+ * The single pass (one split per row) for batches whose rows may be far from equal:
+ * long rows are cut into chunks of whole pages, chosen on the device from seq_lens so
+ * that every CU has about the same number of pages, and a second launch merges the
+ * chunks' fp32 (o, lse). A row that stays whole has the single pass's bits; the cut
+ * depends on seq_lens and the head counts only, never on max_blocks, so a launch
+ * sized for a longer context gives the same bits. workspace holds
+ * bvllm_decode_balanced_workspace_bytes() bytes.
+ */
+BVLLM_API int64_t bvllm_decode_balanced_workspace_bytes(int32_t batch, int32_t num_heads, int32_t num_kv_heads,
+                                                        int32_t head_dim);
+BVLLM_API int bvllm_paged_decode_balanced(const void* q, int64_t q_stride_b, int64_t q_stride_h,
+                       const void* k_cache, const void* v_cache,
+                       int64_t cache_stride_block, int64_t cache_stride_tok, int64_t cache_stride_head,
+                       int32_t num_blocks,
+                       const int32_t* block_tables, int64_t bt_stride, int32_t max_blocks,
+                       const int32_t* seq_lens, float scale,
+                       void* out, int64_t out_stride_b, int64_t out_stride_h,
+                       void* workspace,
+                       int32_t batch, int32_t num_heads, int32_t num_kv_heads,
+                       int32_t head_dim, int32_t block_size, void* stream);
+
+/*
  * bvllm_paged_decode without a workspace argument, for callers that cannot
  * allocate device memory (code under hipGraph capture, tight serving loops,
  * harnesses that forbid hipMalloc). No counterpart in the reference: its

@@ -416,3 +416,72 @@ def test_reduce_sets_do_not_change_bits():
     graph = _kernel()(q, kv_cache, bt, seq_lens, scale, max_seq_len=1100 * BLOCK_SIZE, partition_blocks=1)
     assert torch.equal(eager, graph)
     assert_attn_close(graph, _oracle(q, kv_cache, bt, [600], scale))
+
+
+# ------------------------------------------- balanced single pass (rows cut into chunks)
+
+def _balanced_lens(name):
+    g = torch.Generator().manual_seed(9)
+    if name == "one_long_row":
+        return [9001] + [17] * 40
+    if name == "zeros_and_edges":  # empty rows, chunk ends inside and at the end of a page
+        return [0, 1, 16, 2049, 4096, 8191, 8192, 0] * 5
+    if name == "more_than_64_rows":
+        return torch.randint(1, 6000, (130,), generator=g).tolist()
+    return [3000] * 33  # equal rows, fewer than the CUs serve at once
+
+
+@pytest.mark.parametrize("name", ["one_long_row", "zeros_and_edges", "more_than_64_rows", "equal"])
+@pytest.mark.parametrize("hkv,group,d", [(4, 7, 128), (8, 2, 64), (4, 20, 128)])
+def test_balanced_single_pass_matches_oracle(name, hkv, group, d, monkeypatch):
+    from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV, decode_split_plan
+
+    monkeypatch.delenv(DECODE_PARTITION_ENV, raising=False)
+    lens = _balanced_lens(name)
+    q, kv_cache, bt, seq_lens = make_decode_inputs(lens, hkv=hkv, group=group, d=d, seed=31)
+    scale_keys_by_position(kv_cache, bt, lens, lambda p: 1.0 + 0.001 * p)
+    sms = torch.cuda.get_device_properties(0).multi_processor_count
+    assert decode_split_plan(len(lens), hkv, BLOCK_SIZE, bt.shape[1], max(lens), sms)[0] == 1
+    actual = _kernel()(q, kv_cache, bt, seq_lens, d ** -0.5, max_seq_len=max(lens))
+    expected = _oracle(q, kv_cache, bt, lens, d ** -0.5)
+    assert_attn_close(actual, expected, rows=_live(lens))
+    for i, n in enumerate(lens):
+        if n == 0:
+            assert actual[i].abs().max() == 0
+    # Rows that stay whole have the single pass's bits (32 pages are never cut), the
+    # others are no further from the oracle than it, up to the merge's fp32 rounding.
+    single = _kernel()(q, kv_cache, bt, seq_lens, d ** -0.5, max_seq_len=max(lens), partition_blocks=0)
+    short = [i for i, n in enumerate(lens) if 0 < n <= 512]
+    assert torch.equal(actual[short], single[short])
+    rows = _live(lens)
+    off, off1 = [(x.float().cpu()[rows] - expected[rows]).norm() for x in (actual, single)]
+    assert off <= 1.02 * off1 + 1e-4
+
+
+@pytest.mark.parametrize("longest", [2048, 5000])
+def test_balanced_bits_do_not_depend_on_the_bucket_or_other_columns(longest, monkeypatch):
+    from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV
+
+    monkeypatch.delenv(DECODE_PARTITION_ENV, raising=False)
+    lens = [longest, 100, 7] + [60] * 61
+    q, kv_cache, bt, seq_lens = make_decode_inputs(lens, width=700, seed=32)
+    scale = HEAD_DIM ** -0.5
+    live = _kernel()(q, kv_cache, bt, seq_lens, scale, max_seq_len=longest)
+    assert torch.equal(live, _kernel()(q, kv_cache, bt, seq_lens, scale, max_seq_len=700 * BLOCK_SIZE))
+    assert torch.equal(live, _kernel()(q, kv_cache, bt, seq_lens, scale))
+
+
+def test_balanced_launch_in_a_graph_follows_the_lengths(monkeypatch):
+    from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV
+
+    monkeypatch.delenv(DECODE_PARTITION_ENV, raising=False)
+    q, kv_cache, bt, seq_lens = make_decode_inputs([4000] * 40, seed=33)
+    scale = HEAD_DIM ** -0.5
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = _kernel()(q, kv_cache, bt, seq_lens, scale)
+    for lens in ([4000] * 40, [4000] + [30] * 39, [1] * 40, [3999, 0] * 20):
+        seq_lens.copy_(torch.tensor(lens, dtype=torch.int32))
+        graph.replay()
+        assert torch.equal(out, _kernel()(q, kv_cache, bt, seq_lens, scale))
+        assert_attn_close(out, _oracle(q, kv_cache, bt, lens, scale, 4000), rows=_live(lens))
