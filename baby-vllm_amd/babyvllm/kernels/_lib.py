@@ -154,6 +154,31 @@ def lib() -> ctypes.CDLL:
     return handle
 
 
+@functools.lru_cache(maxsize=None)
+def fast():
+    """The native host side of the wrappers' common calls (csrc/fast_calls.cpp), bound to ``lib()``.
+
+    Its functions return None for a call that is not plainly valid; the wrapper then
+    runs its own checks and path.
+    """
+    handle = lib()
+    try:
+        from babyvllm import _fast_calls
+    except ImportError as e:
+        raise KernelLibraryError("babyvllm._fast_calls not found or not loadable: build it with "
+                                 "`python baby-vllm_amd/build_lib.py`") from e
+    _fast_calls.bind({n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value for n in _fast_calls.names()})
+    return _fast_calls
+
+
+def current():
+    """(index, raw stream handle) of the current ROCm device and its current stream."""
+    from torch import _C
+
+    d = _C._cuda_getDevice()
+    return d, _C._cuda_getCurrentRawStream(d)
+
+
 def set_tuning(knob: int, value: int) -> int:
     """Sets a process-wide tuning knob (0 = default); returns its previous value."""
     prev = lib().bvllm_set_tuning(knob, value)

@@ -14,6 +14,10 @@ from babyvllm.kernels import _lib
 
 def fused_silu_mul(gate_up: torch.Tensor):
     """Fuses F.silu(gate) * up where gate_up is a concatenated tensor (..., 2 * D)."""
+    if gate_up.is_cuda:
+        out = _lib.fast().silu(gate_up, *_lib.current())
+        if out is not None:
+            return out
     assert gate_up.is_contiguous(), "gate_up tensor must be contiguous"
     _lib.require_rocm_tensor("gate_up", gate_up)
     if gate_up.dtype != torch.bfloat16:

@@ -21,7 +21,7 @@ import os
 import torch
 
 from babyvllm.kernels import _lib
-from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV, decode_split_plan
+from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV, MIN_PARTITION_BLOCKS, decode_split_plan
 
 # A single-pass plan ("auto") sized for more pages than this runs the balanced launch
 # (bvllm_paged_decode_balanced). Shorter rows can lose less to each other than its second
@@ -47,6 +47,12 @@ def paged_decode_attention(q, kv_cache, block_tables, seq_lens, scale,
     split count. ``partition_blocks`` overrides BABYVLLM_DECODE_PARTITION.
     Rows with ``seq_len == 0`` return zeros.
     """
+    if partition_blocks is None and q.is_cuda:
+        d, stream = _lib.current()
+        out = _lib.fast().decode(q, kv_cache, block_tables, seq_lens, scale, max_seq_len, _num_sms(d),
+                                 MIN_PARTITION_BLOCKS, BALANCE_MIN_PAGES, DECODE_PARTITION_ENV, d, stream)
+        if out is not None:
+            return out
     for name, t in (("q", q), ("kv_cache", kv_cache), ("block_tables", block_tables),
                     ("seq_lens", seq_lens)):
         _lib.require_rocm_tensor(name, t)

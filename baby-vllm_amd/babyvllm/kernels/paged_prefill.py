@@ -56,6 +56,12 @@ def paged_prefill_attention(q, kv_cache, md, scale):
     K/V of the step's tokens must already be in the cache (the RoPE + append
     kernel writes them first).
     """
+    if q.is_cuda:
+        out = _lib.fast().prefill(q, kv_cache, md.block_tables, md.query_start_loc, md.seq_lens, md.context_lens,
+                                  getattr(md, "query_start_loc_cpu", None), getattr(md, "seq_lens_cpu", None),
+                                  md.max_query_len, scale, _SPLIT_MIN_PAGES, *_lib.current())
+        if out is not None:
+            return out
     num_tokens, num_heads, head_dim = q.shape
     num_kv_heads = kv_cache.shape[3]
     page = kv_cache.shape[2]

@@ -32,6 +32,9 @@ def fused_rope_and_cache(
 
     cos/sin are ``[T, D]`` per-token rows (RotaryEmbedding output, duplicated halves).
     """
+    if q.is_cuda and kv_cache is not None and slot_mapping is not None:
+        if _lib.fast().rope(q, k, v, cos, sin, kv_cache, slot_mapping, *_lib.current()):
+            return q, k
     for name, t in (("q", q), ("k", k), ("cos", cos), ("sin", sin)):
         _lib.require_rocm_tensor(name, t)
     _check_rows("q", q, 3)

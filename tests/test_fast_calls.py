@@ -1,0 +1,132 @@
+"""The wrappers' native host side (csrc/fast_calls.cpp): its plan equals decode_split_plan, it declines
+what it must decline, and calls through it equal calls through the Python path."""
+
+import random
+
+import pytest
+import torch
+
+from tests._cases import build_prefill_case, make_decode_inputs
+
+
+
+def _fast():
+    from babyvllm.kernels import _lib
+
+    return _lib.fast()
+
+
+def test_auto_plan_equals_decode_split_plan(monkeypatch):
+    from babyvllm.kernels import decode_split as ds
+
+    monkeypatch.delenv(ds.DECODE_PARTITION_ENV, raising=False)
+    r = random.Random(4)
+    for _ in range(3000):
+        batch, hkv, width = r.randint(1, 300), r.choice([1, 2, 4, 8, 28]), r.choice([0, 1, 2, 129, r.randint(1, 5000)])
+        max_len = r.choice([None, 0, 1, 16, 17, r.randint(0, 90000)])
+        cus = r.choice([1, 132, 256, 304])
+        got = _fast().auto_plan(batch, hkv, 16, width, -1 if max_len is None else max_len, cus, ds.MIN_PARTITION_BLOCKS)
+        assert got == ds.decode_split_plan(batch, hkv, 16, width, max_len, cus), (batch, hkv, width, max_len, cus)
+
+
+def test_cpu_tensors_and_wrong_argument_counts_are_declined():
+    x = torch.zeros(2, 8, dtype=torch.bfloat16)
+    f = _fast()
+    assert f.norm(x, None, x[0], 1e-6, 0, 0) is None
+    assert f.silu(x, 0, 0) is None
+    assert f.linear(x, x, None, None, False, 0, 0) is None
+    assert f.norm() is None and f.decode(x) is None and f.prefill() is None and f.rope(x, x) is None
+
+
+class _Declining:
+    """Stands in for the native module: every call takes the Python path."""
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+def _python_path(monkeypatch):
+    from babyvllm.kernels import _lib
+
+    monkeypatch.setattr(_lib, "fast", lambda: _Declining())
+
+
+def _calls():
+    from babyvllm.kernels.activation import fused_silu_mul
+    from babyvllm.kernels.layernorm import fused_add_rms_norm
+    from babyvllm.kernels.paged_attn import paged_decode_attention
+    from babyvllm.kernels.paged_prefill import paged_prefill_attention
+    from babyvllm.kernels.rope import fused_rope_and_cache
+
+    def rand(*shape):
+        return torch.randn(*shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(sum(shape)))
+
+    x, res = rand(3, 5, 96).bfloat16(), rand(3, 5, 96).bfloat16()
+    out = {}
+    for w in (rand(96), rand(96).bfloat16()):
+        for r in (None, res.clone()):
+            out["norm", w.dtype, r is None] = (fused_add_rms_norm(x, r, w, 1e-5), r)
+    out["norm view"] = fused_add_rms_norm(rand(4, 200).bfloat16()[:, :96], None, rand(96), 1e-5)
+    out["silu"] = fused_silu_mul(x)
+    qkv = rand(7, 14 * 64 + 4 * 64).bfloat16()
+    q, k, v = qkv[:, :896].view(7, 14, 64), qkv[:, 896:1024].view(7, 2, 64), qkv[:, 1024:].view(7, 2, 64)
+    cache = rand(2, 4, 16, 2, 64).bfloat16()
+    slots = torch.tensor([3, 60, 17, 9, 31, -1, 40], device="cuda")
+    cos, sin = rand(7, 64).bfloat16(), rand(7, 64).bfloat16()
+    fused_rope_and_cache(q, k, v, cos, sin, cache, slots)
+    out["rope"] = (qkv, cache)
+    for lens in ([40, 700, 0], [3000] + [20] * 39):
+        dq, dc, bt, sl = make_decode_inputs(lens)
+        for bucket in (None, max(lens), 4096):
+            out["decode", len(lens), bucket] = paged_decode_attention(dq, dc, bt, sl, 0.1, max_seq_len=bucket)
+    for specs in ([(0, 20), (30, 1), (5, 70)], [(5000, 40), (3000, 7)]):
+        pq, pc, md = build_prefill_case(specs, 4, 7, 128)
+        out["prefill", len(specs)] = paged_prefill_attention(pq, pc, md, 0.1)
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a ROCm GPU")
+def test_calls_equal_the_python_path(monkeypatch):
+    native = _calls()
+    _python_path(monkeypatch)
+    python = _calls()
+    assert native.keys() == python.keys()
+    for name in native:
+        a, b = native[name], python[name]
+        for s, t in zip(a if isinstance(a, tuple) else (a,), b if isinstance(b, tuple) else (b,)):
+            assert (s is None) == (t is None), name
+            if s is not None:
+                assert s.shape == t.shape and s.dtype == t.dtype and s.stride() == t.stride(), name
+                assert torch.equal(s, t), name
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a ROCm GPU")
+def test_refused_calls_raise_as_before():
+    from babyvllm.kernels._lib import KernelLibraryError
+    from babyvllm.kernels.activation import fused_silu_mul
+    from babyvllm.kernels.layernorm import fused_add_rms_norm
+    from babyvllm.kernels.paged_attn import paged_decode_attention
+    from babyvllm.kernels.paged_prefill import paged_prefill_attention
+
+    x = torch.randn(4, 96, device="cuda", dtype=torch.bfloat16)
+    with pytest.raises(TypeError):
+        fused_add_rms_norm(x.float(), None, x[0], 1e-5)
+    with pytest.raises(TypeError):
+        fused_add_rms_norm(x, x[:, :8].contiguous(), x[0], 1e-5)
+    with pytest.raises(RuntimeError):  # .view of a non-contiguous input
+        fused_add_rms_norm(x.view(2, 2, 96).transpose(0, 1), None, x[0], 1e-5)
+    with pytest.raises(AssertionError):
+        fused_silu_mul(x[:, :32])
+    q, cache, bt, lens = make_decode_inputs([20, 30])
+    with pytest.raises(TypeError):
+        paged_decode_attention(q, cache, bt.long(), lens, 0.1)
+    with pytest.raises(ValueError):
+        paged_decode_attention(q, cache, bt[:1], lens, 0.1)
+    q96, cache96 = q[..., :96].contiguous(), cache[..., :96].contiguous()
+    with pytest.raises(KernelLibraryError):  # head_dim the library refuses
+        paged_decode_attention(q96, cache96, bt, lens, 0.1)
+    pq, pc, md = build_prefill_case([(0, 5)], 4, 7, 128)
+    with pytest.raises(AssertionError):
+        paged_prefill_attention(pq[..., :96].contiguous(), pc, md, 0.1)
