@@ -40,7 +40,8 @@ struct DecodeArgs {
   int32_t splits_per_item;                 // consecutive splits one streaming wave computes
   int32_t num_partials;                    // partial states per (row, head) the launch writes
   int32_t ws_partials;                     // partial states per (row, head) the workspace holds
-  int32_t item_order;                      // 0: KV head fastest in the wave numbering; 1: split unit fastest
+  int32_t item_order;                      // numbering: 0 KV head, row, unit (fastest first); 1 unit, KV head, row;
+                                           // 2 as 0 with each row's units together and the empty ones last
   // Balanced single pass (RowChunk): chunks aimed at per column group, rows an even
   // share of which keeps every CU busy.
   int32_t chunk_target, row_slots;
@@ -144,9 +145,11 @@ struct DecodePlan {
   int32_t partials;        // partial states per (row, head) in the workspace
   bool fold_in_reduce;     // the reduce folds the per-split partials into groups
   bool pair;               // one split or group per work-group of two waves (two states each)
-  bool quad;               // (with pair) one split of at most 32 pages per work-group of four waves
+  bool quad;               // (with pair) work-groups of four waves: splits of at most 64 pages, long groups
+  bool live_first;         // units with live pages before the empty ones (find_live_unit)
 };
-DecodePlan decode_plan(int32_t batch, int32_t num_kv_heads, int32_t num_splits, int32_t blocks_per_split);
+DecodePlan decode_plan(int32_t batch, int32_t num_kv_heads, int32_t head_dim, int32_t num_splits,
+                       int32_t blocks_per_split);
 // Column groups of a decode launch: its KV heads, each cut into ceil(G / 16)
 // groups of at most 16 query heads (one MFMA tile of columns) when G > 16.
 inline int64_t decode_col_groups(const DecodeArgs& a) {
@@ -161,9 +164,7 @@ int32_t decode_partials(int32_t batch, int32_t num_kv_heads, int32_t num_splits,
 enum TuneKnob {
   kTuneDecodeSplitMode = 0,         // 1: one wave per split, 2: one wave per group of splits, 3: two
                                     // waves per group, 4: two waves per split also for splits of at most
-                                    // 32 pages (same bits); by default single splits run on four waves
-                                    // (at most 32 pages) or two, groups on two waves when at most one
-                                    // group per CU
+                                    // 64 pages, 5: four waves per group (same bits); default: decode_plan
   kTunePrefillBlocksPerWg = 1,      // n > 0: prefill column blocks per work-group when the table allows it
   kTuneDecodeOrder = 2,             // 1: split units fastest in the streaming wave numbering (same bits)
   kTuneDecodeSinglePassStream = 3,  // 1: single-pass launches on streaming waves too (same bits)

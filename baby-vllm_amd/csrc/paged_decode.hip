@@ -307,7 +307,8 @@ int set_tuning(int knob, int value) {
 // stream); split mode folds at most kChain splits in the reduce. The default
 // takes group mode when there are more than kChain splits or enough groups to
 // fill the GPU (2 per CU of a 256-CU MI355X), split mode otherwise.
-DecodePlan decode_plan(int32_t batch, int32_t num_kv_heads, int32_t num_splits, int32_t blocks_per_split) {
+DecodePlan decode_plan(int32_t batch, int32_t num_kv_heads, int32_t head_dim, int32_t num_splits,
+                       int32_t blocks_per_split) {
   DecodePlan p{};
   if (num_splits <= 1) {
     p.single_pass = true;
@@ -319,20 +320,28 @@ DecodePlan decode_plan(int32_t batch, int32_t num_kv_heads, int32_t num_splits, 
   bool group_mode = p.group > 1 && (num_splits > kChain || (int64_t)batch * num_kv_heads * groups >= 512);
   const int forced = tuning(kTuneDecodeSplitMode);
   if (forced == 1 && (p.group == 1 || num_splits <= kChain)) group_mode = false;
-  if ((forced == 2 || forced == 3) && p.group > 1) group_mode = true;
+  if ((forced == 2 || forced == 3 || forced == 5) && p.group > 1) group_mode = true;
   p.splits_per_item = group_mode ? p.group : 1;
   p.partials = group_mode ? (int32_t)groups : num_splits;
   p.fold_in_reduce = !group_mode && p.group > 1;
-  // Two waves per work-group: for single splits unless knob 1; for groups of
-  // splits when there are at most two groups per CU (two waves per group, two
-  // pages in flight each, one wave per SIMD: 1 x 32768 and 2 x 16384, 512
-  // groups: 23.5 -> 21.5 and 24.1 -> 21.2 us; 4 x 4096, 256 groups: 22.0 ->
-  // 18.2 us), one wave per group beyond (8 x 16384, 1024 groups: 52.8 against
-  // 56.4 us on two waves; 4 x 32768, 2048 groups: 60.0 against 64.3 us).
+  // Waves per work-group. Single splits: four when a split has at most 64 pages (2 KV
+  // heads of 64, splits of 64 pages: 64 x 4000 29.8 -> 27 us against two waves, 50 rows of
+  // 100 to 2000 17.6 -> 14.4), else two. Groups of splits of 16 pages and more (64 pages
+  // per group: the walk of a group's pages sets the time): two, or four (see
+  // paged_decode_quad_group_kernel). Groups of shorter splits: two while there are at
+  // most two groups per CU (two pages in flight each, one wave per SIMD: 1 x 32768 and
+  // 2 x 16384, 512 groups: 23.5 -> 21.5 and 24.1 -> 21.2 us; 4 x 4096, 256 groups: 22.0
+  // -> 18.2 us), one beyond (8 x 16384, 1024 groups: 52.8 against 56.4 us on two waves;
+  // 4 x 32768, 2048 groups: 60.0 against 64.3 us).
   const int64_t group_items = (int64_t)batch * num_kv_heads * groups;
-  p.pair = group_mode ? (forced == 3 || (forced != 2 && group_items <= 2 * (int64_t)device_cus())) : forced != 1;
-  // Four waves per split when a split has at most 32 pages (at most 8 per wave), unless knob 4.
-  p.quad = p.pair && !group_mode && blocks_per_split <= 32 && forced != 4;
+  const bool long_groups = blocks_per_split >= 16;
+  p.pair = group_mode
+               ? (forced == 3 || forced == 5 || (forced != 2 && (long_groups || group_items <= 2 * (int64_t)device_cus())))
+               : forced != 1;
+  p.quad = group_mode ? forced == 5 || (forced != 2 && forced != 3 && long_groups &&
+                                        (head_dim == 64 || blocks_per_split >= 64))
+                      : p.pair && blocks_per_split <= 64 && forced != 4;
+  p.live_first = p.pair && group_mode && long_groups && batch > 1;
   return p;
 }
 
@@ -424,7 +433,7 @@ template <int D>
 static hipError_t launch_decode(const DecodeArgs& args, hipStream_t stream) {
   DecodeArgs a = args;
   const int64_t ncg = decode_col_groups(a);
-  const DecodePlan p = decode_plan(a.batch, (int32_t)ncg, a.num_splits, a.blocks_per_split);
+  const DecodePlan p = decode_plan(a.batch, (int32_t)ncg, a.head_dim, a.num_splits, a.blocks_per_split);
   a.item_order = tuning(kTuneDecodeOrder) == 1 ? 1 : 0;
   if (p.single_pass && tuning(kTuneDecodeSinglePassStream) == 0) {
     // One page in flight per wave, the next requested as soon as it has
@@ -448,11 +457,14 @@ static hipError_t launch_decode(const DecodeArgs& args, hipStream_t stream) {
   // The workspace holds decode_partials() states per (row, head); the plan
   // (one knob read above) never asks for more.
   if (!p.single_pass && (a.part_out == nullptr || p.partials > a.ws_partials)) return hipErrorInvalidValue;
+  if (p.live_first && a.item_order == 0) a.item_order = 2;
   const int64_t units = (a.num_splits + a.splits_per_item - 1) / a.splits_per_item;
   const int64_t items = (int64_t)a.batch * decode_col_groups(a) * units;
   if (items > 0x7ffffff0) return hipErrorInvalidValue;
   hipError_t err;
-  if (p.quad) {
+  if (p.quad && a.splits_per_item > 1) {
+    err = launch_quad_group_vgpr(a, items, tuning(kTuneDecodeCached) == 0, stream);
+  } else if (p.quad) {
     if constexpr (D == 64) {
       err = launch_quad_vgpr(a, items, tuning(kTuneDecodeCached) == 0, stream);
     } else {

@@ -82,7 +82,7 @@ __device__ __forceinline__ float group_lse(const GroupFold& f) { return f.L > 0.
 // LDS, twice that with GROUP), and wave w merges elements 2w and 2w + 1 of
 // every lane's accumulator vectors from the four, in order, as a single wave
 // would (and folds or writes those output dims).
-// QUAD (with PAIR, single splits of at most 32 pages): four waves; wave w holds
+// QUAD (with PAIR): four waves; wave w holds
 // state w (its pages 4k + w, two in flight), publishes
 // it at the split's end, and merges element w of every accumulator vector from
 // the four records: the same arithmetic in the same order, on a quarter of the
@@ -92,6 +92,52 @@ constexpr int kPairRecFloats = (2 + 4 * (D / 16)) * 64;  // m, l, accumulators o
 template <int D>
 constexpr int kPairLdsFloats = 4 * kPairRecFloats<D>;
 
+// Item order 2: the units with a live page first, row by row, then the empty ones (which
+// only write empty partials). Work-groups that end at once shift the dispatcher's
+// round, and it then puts two or three live ones on some CUs while others idle; with
+// the empty ones last the live ones are dealt evenly. For groups of long splits, where
+// a second group on a CU costs far more than the round trip of finding the unit (12
+// rows of 100 to 32768, two waves per group of 64 pages: 55 -> 40 us; two rows of 16000
+// among 18 of 16, four waves: 49 -> 32; equal rows lose about 1 us: 32 x 16000 169 -> 170).
+__device__ __forceinline__ void find_live_unit(const DecodeArgs& a, int t, int units, int unit_pages, int& b_out,
+                                               int& unit_out) {
+  const int lane = lane_id();
+  auto live_units = [&](int b) {
+    if (b >= a.batch) return 0;
+    const int len = a.seq_lens[b];
+    const int pages = min(len > 0 ? (len + 15) / 16 : 0, a.max_blocks);
+    return min((pages + unit_pages - 1) / unit_pages, units);
+  };
+  const int n0 = live_units(lane);
+  int total = 0;
+  for (int b0 = 0; b0 < a.batch; b0 += 64)
+    total += wave_reduce(b0 == 0 ? n0 : live_units(b0 + lane), [](int x, int y) { return x + y; });
+  const bool live = t < uniform(total);
+  int before = live ? 0 : uniform(total);
+  for (int b0 = 0; b0 < a.batch; b0 += 64) {
+    const int b = b0 + lane;
+    const int n = b0 == 0 ? n0 : live_units(b);
+    const int mine = b < a.batch ? (live ? n : units - n) : 0;
+    int inc = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int x = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += x;
+    }
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(before + inc > t);
+    if (hit != 0) {
+      const int l = (int)__builtin_ctzll(hit);
+      b_out = uniform(b0 + l);
+      const int k = t - before - __shfl(inc - mine, l, 64);
+      unit_out = uniform(live ? k : __shfl(n, l, 64) + k);
+      return;
+    }
+    before += __shfl(inc, 63, 64);
+  }
+  b_out = 0;  // not reached: every unit of every row is numbered
+  unit_out = 0;
+}
+
 template <int D, int PF, bool NT, bool GROUP, bool PAIR = false, bool QUAD = false>
 __device__ __forceinline__ void decode_stream_wave(const DecodeArgs& a, const int item, unsigned char* tile,
                                                    float* xs = nullptr) {
@@ -99,7 +145,7 @@ __device__ __forceinline__ void decode_stream_wave(const DecodeArgs& a, const in
   constexpr int VD = D / 16;
   constexpr int OPL = D / 4;  // output floats per lane: head n, dims VD·(4g+i) + c
   static_assert(PF == (PAIR && !GROUP && !QUAD ? 4 : 2), "pages in flight per wave");
-  static_assert(!QUAD || (PAIR && !GROUP), "four waves per item: single splits only");
+  static_assert(!QUAD || PAIR, "four waves share an item's states");
   const int w = PAIR ? wave_id() : 0;
 
   const int S = a.num_splits;
@@ -108,11 +154,21 @@ __device__ __forceinline__ void decode_stream_wave(const DecodeArgs& a, const in
   // Column groups: the KV heads, or their 16-head parts when G > 16 (ColGroup).
   const int ncg = a.num_kv_heads * col_groups_per_kv(a.num_heads / a.num_kv_heads);
   int cg, unit, b;
-  if (a.item_order == 0) {  // KV head fastest: the 4 head slices of a page are requested together
+  if (GROUP && a.item_order == 2) {
+    cg = item % ncg;
+    find_live_unit(a, item / ncg, units, spi * a.blocks_per_split, b, unit);
+  } else if (a.item_order == 0) {
+    // KV head fastest, then the row, then the unit: the first units of every row come
+    // first and units past the end of short rows last, so that the live work-groups
+    // are dealt evenly to the CUs (empty ones between them leave some CUs with two or
+    // three and others with none). The row is shifted by the unit, since work-groups
+    // go round-robin to the 8 XCDs and a row's units must not all meet on one (rows'
+    // units next to each other put the first unit of every row on the same XCDs: 64
+    // rows of 200 to 8192, 2 KV heads of 64: 33 -> 27.7 us).
     cg = item % ncg;
     const int rest = item / ncg;
-    unit = rest % units;
-    b = rest / units;
+    unit = rest / a.batch;
+    b = (rest - unit * a.batch + a.batch - unit % a.batch) % a.batch;
   } else {  // unit fastest
     unit = item % units;
     const int rest = item / units;
@@ -260,6 +316,8 @@ __device__ __forceinline__ void decode_stream_wave(const DecodeArgs& a, const in
   auto pair_finish = [&](int xb, int split) __attribute__((always_inline)) {
     float* xbase = xs + xb * kPairLdsFloats<D>;
     constexpr int SPW = QUAD ? 1 : 2;  // states per wave
+    // One buffer (QUAD groups): every wave has read the last split's records first.
+    if constexpr (QUAD && GROUP) __syncthreads();
 #pragma unroll
     for (int s2 = 0; s2 < SPW; ++s2) {
       float* rec = xbase + (SPW * w + s2) * kPairRecFloats<D>;
@@ -339,6 +397,52 @@ __device__ __forceinline__ void decode_stream_wave(const DecodeArgs& a, const in
     const int slot_ent = min(max(ent, 0), a.num_pages - 1);
     auto phys = [&](int k) -> int64_t { return (int64_t)__builtin_amdgcn_readlane(slot_ent, k); };
     PageRegs<D> r[PF];
+    // PAIR and QUAD groups: at a split's first page the split that ended is merged and
+    // folded.
+    auto new_split = [&](int quad) __attribute__((always_inline)) {
+      if (quad < here && base + quad == next_start) {
+        pair_finish(xb, cur);
+        if constexpr (!QUAD) xb ^= 1;
+        ++cur;
+        next_start = (cur + 1 < j1) ? next_start + bps : INT_MAX;
+        any = false;
+      }
+    };
+    if constexpr (QUAD && GROUP) {
+      // A group of splits on four waves: the wave's pages in order are q = 8j + 4i + w
+      // for ring slot i, all of state w, two in flight.
+#pragma unroll
+      for (int i = 0; i < PF; ++i) {
+        const int64_t p = phys(min(4 * i + w, here - 1)) * a.c_sb;
+        load_page<D, NT>(r[i], kc + p, vc + p, off);
+      }
+      int k = 0;
+      for (; k + 8 < here; k += 8) {
+#pragma unroll
+        for (int i = 0; i < PF; ++i) {
+          new_split(k + 4 * i);
+          wait_page<(PF - 1) * kLoadsPerPage, D>(r[i]);
+          const int q = k + 4 * i + w;
+          if (q < here)
+            process_page<D>(st[0], r[i], qb, tile, n, g, (p0 + base + q) * 16 + 4 * g, seq_len, a.scale_log2);
+          const int64_t pn = phys(min(q + 8, here - 1)) * a.c_sb;
+          load_page<D, NT>(r[i], kc + pn, vc + pn, off);
+          any = true;
+        }
+      }
+      // The last eight pages: no load past them, and slot i waits for itself only.
+      new_split(k);
+      wait_page<kLoadsPerPage, D>(r[0]);
+      if (k + w < here)
+        process_page<D>(st[0], r[0], qb, tile, n, g, (p0 + base + k + w) * 16 + 4 * g, seq_len, a.scale_log2);
+      any = true;
+      new_split(k + 4);
+      wait_page<0, D>(r[1]);
+      if (k + 4 + w < here)
+        process_page<D>(st[0], r[1], qb, tile, n, g, (p0 + base + k + 4 + w) * 16 + 4 * g, seq_len, a.scale_log2);
+      if (k + 4 < here) any = true;
+      continue;
+    }
     if constexpr (PAIR && GROUP) {
       // A group of splits on two waves: two pages in flight per wave, page
       // k + 4 requested once page k is computed. The wave's pages in order:
@@ -350,16 +454,6 @@ __device__ __forceinline__ void decode_stream_wave(const DecodeArgs& a, const in
         const int64_t p = phys(min(2 * w + i, here - 1)) * a.c_sb;
         load_page<D, NT>(r[i], kc + p, vc + p, off);
       }
-      // At a split's first page: the split that ended is merged and folded.
-      auto new_split = [&](int quad) __attribute__((always_inline)) {
-        if (quad < here && base + quad == next_start) {
-          pair_finish(xb, cur);
-          xb ^= 1;
-          ++cur;
-          next_start = (cur + 1 < j1) ? next_start + bps : INT_MAX;
-          any = false;
-        }
-      };
       int k = 0;
       for (; k + 4 < here; k += 4) {
         new_split(k);
@@ -524,7 +618,7 @@ __global__ __launch_bounds__(128) void paged_decode_pair_kernel(DecodeArgs a, in
   decode_stream_wave<D, GROUP ? 2 : 4, NT, GROUP, true>(a, item, tile + wave_id() * kTileBytes<D>, xs);
 }
 
-// Four waves per single split of at most 32 pages (one state each, two pages
+// Four waves per single split of at most 64 pages (one state each, two pages
 // in flight): B8 x 1920 (15 splits of 8 pages) 14.3 -> 13.9 us, config 1 (4 of
 // 8) 11.13 -> 10.85 us, B8 x 4096 (32 of 8) 25.0 -> 23.0 us, B16 x 1920 (8 of
 // 16) 19.3 -> 18.6 us, B16 x 4096 (16 of 16) 34.1 -> 31.5 us, B32 x 1920 (4 of
@@ -542,10 +636,27 @@ __global__ __launch_bounds__(256) void paged_decode_quad_kernel(DecodeArgs a, in
   decode_stream_wave<D, 2, NT, false, true, true>(a, item, tile + wave_id() * kTileBytes<D>, xs);
 }
 
+// Four waves per group of splits (one state each, two pages in flight): the groups
+// of long splits at D = 64, where one or two waves read too little at a time to keep
+// a CU's share of HBM busy (36 rows of 100 to 32000, groups of 256 pages: one wave 128
+// us, two 68, four 43; 16 x 16000: two 29.7, four 28.1), and of 64 pages and more.
+// At D = 128 two waves do as well (24 rows of 100 to 32768: one wave 94, two 67, four
+// 74; 20 of 200 to 16000: 89, 47, 40; 32 x 16000: 177, 170.6, 171.4).
+template <int D, bool NT>
+__global__ __launch_bounds__(256) void paged_decode_quad_group_kernel(DecodeArgs a, int items) {
+  __shared__ __attribute__((aligned(16))) unsigned char tile[4 * kTileBytes<D>];
+  __shared__ __attribute__((aligned(16))) float xs[kPairLdsFloats<D>];
+  const int item = (int)blockIdx.x;
+  if (item >= items) return;
+  decode_stream_wave<D, 2, NT, true, true, true>(a, item, tile + wave_id() * kTileBytes<D>, xs);
+}
+
 // Launches paged_decode_pair_kernel<D, nt, group> for the specializations
 // paged_decode_pair.hip holds (group walks, and split walks at D = 64).
 hipError_t launch_pair_vgpr(const DecodeArgs& a, int64_t items, bool group, bool nt, hipStream_t stream);
 // Launches paged_decode_quad_kernel<64, nt> (held by paged_decode_pair.hip).
 hipError_t launch_quad_vgpr(const DecodeArgs& a, int64_t items, bool nt, hipStream_t stream);
+// Launches paged_decode_quad_group_kernel<D, nt> (held by paged_decode_pair.hip).
+hipError_t launch_quad_group_vgpr(const DecodeArgs& a, int64_t items, bool nt, hipStream_t stream);
 
 }  // namespace bvllm

@@ -236,10 +236,10 @@ BVLLM_API int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int64
  * Tuning switch for experiments and tests (no counterpart in the reference):
  * sets process-wide knob `knob` to `value` (0 = the library's default) and
  * returns the previous value, or -1 for an unknown knob. Knobs: 0 decode split
- * mode (default: four waves per split of at most 32 pages, two per longer
- * split, or per group of 4 splits when the plan groups them, two only while
- * the groups are at most one per compute unit; 1 one wave per split, 2 one
- * wave per group, 3 two waves per group, 4 two waves per split), 1 prefill
+ * mode (default: four waves per split of at most 64 pages, two per longer
+ * split; per group of 4 splits, when the plan groups them, one, two or four by
+ * their number and length; 1 one wave per split, 2 one wave per group, 3 two
+ * waves per group, 4 two waves per split, 5 four waves per group), 1 prefill
  * column blocks per work-group (tables of at most 8 pages), 2 decode wave
  * order (1 split units fastest), 3 decode single pass on streaming waves (1),
  * 4 decode page loads of the streaming waves without the nontemporal hint

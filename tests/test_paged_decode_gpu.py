@@ -485,3 +485,21 @@ def test_balanced_launch_in_a_graph_follows_the_lengths(monkeypatch):
         graph.replay()
         assert torch.equal(out, _kernel()(q, kv_cache, bt, seq_lens, scale))
         assert_attn_close(out, _oracle(q, kv_cache, bt, lens, scale, 4000), rows=_live(lens))
+
+
+@pytest.mark.parametrize("partition", [16, 32, 64])
+@pytest.mark.parametrize("hkv,group,d", [(4, 7, 128), (2, 7, 64), (1, 20, 128)])
+def test_long_groups_agree_on_every_wave_count_and_order(partition, hkv, group, d):
+    """Groups of long splits (two or four waves, live units first) against one wave per
+    group and per split: the same bits, with empty rows, empty groups, rows that end
+    inside a group's first and last split, and more rows than a wave's lanes."""
+    lens = [9000, 0, 1, 16 * partition, 16 * partition + 1, 64 * partition + 17, 300] + [40, 0] * 30
+    q, kv_cache, bt, seq_lens = make_decode_inputs(lens, hkv=hkv, group=group, d=d, seed=41)
+    outs = {}
+    for mode in (0, 1, 2, 3, 5):
+        with tuned(0, mode):
+            outs[mode] = _kernel()(q, kv_cache, bt, seq_lens, d ** -0.5, max_seq_len=max(lens),
+                                   partition_blocks=partition)
+    for mode, out in outs.items():
+        assert torch.equal(out, outs[2]), mode
+    assert_attn_close(outs[0], _oracle(q, kv_cache, bt, lens, d ** -0.5), rows=_live(lens))
