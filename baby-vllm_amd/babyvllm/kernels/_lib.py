@@ -112,6 +112,11 @@ SIGNATURES = {
         _p,                         # stream
     ]),
     "bvllm_silu_mul": (ctypes.c_int, [_p, _i64, _i32, _p, _p]),
+    "bvllm_embed_rows": (ctypes.c_int, [
+        _p, _p, _i64, _p,           # ids, table, vocab, out
+        _p, _p, _p, _i64, _p, _p,   # positions, cos table, sin table, max_positions, cos out, sin out
+        _i32, _i32, _i32, _p,       # rows, hidden, head_dim, stream
+    ]),
     "bvllm_linear_workspace_bytes": (ctypes.c_int64, [_i32, _i32, _i32, _i32]),
     "bvllm_linear": (ctypes.c_int, [
         _p, _i64, _p, _p, _p, _i64,  # x, stride, w, bias, out, stride

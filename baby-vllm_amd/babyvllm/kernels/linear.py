@@ -19,7 +19,7 @@ from babyvllm.kernels import _lib
 MAX_ROWS = 64
 
 
-def _torch_must_see(*tensors) -> bool:
+def torch_must_see(*tensors) -> bool:
     """Whether something besides the values wants to see this operation."""
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
         return True
@@ -32,7 +32,7 @@ def _torch_must_see(*tensors) -> bool:
 
 def skinny_linear(x, weight, bias=None, out=None):
     """``x @ weight.T + bias`` for x [M ≤ 64, K] (into ``out`` if given), or None."""
-    if not x.is_cuda or x.dim() != 2 or x.shape[0] > MAX_ROWS or _torch_must_see(x, weight, bias, out):
+    if not x.is_cuda or x.dim() != 2 or x.shape[0] > MAX_ROWS or torch_must_see(x, weight, bias, out):
         return None
     return _lib.fast().linear(x, weight, bias, out, False, *_lib.current())
 
@@ -42,6 +42,6 @@ def gated_linear(x, weight):
 
     Gate and up stay fp32 up to the product (torch's two steps round them to bf16 first).
     """
-    if not x.is_cuda or x.dim() != 2 or x.shape[0] > MAX_ROWS or _torch_must_see(x, weight):
+    if not x.is_cuda or x.dim() != 2 or x.shape[0] > MAX_ROWS or torch_must_see(x, weight):
         return None
     return _lib.fast().linear(x, weight, None, None, True, *_lib.current())

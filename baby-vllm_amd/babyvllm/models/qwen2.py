@@ -18,6 +18,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from babyvllm.kernels.activation import fused_silu_mul
+from babyvllm.kernels.embed import embed_rows
 from babyvllm.kernels.linear import gated_linear, skinny_linear
 from babyvllm.kernels.rope import fused_rope_and_cache
 from babyvllm.layers.attention import Attention
@@ -103,9 +104,20 @@ class Qwen2Model(nn.Module):
         self.rotary_emb = RotaryEmbedding(cfg.head_dim, max_position_embeddings=cfg.max_position_embeddings,
                                           base=cfg.rope_theta)
 
+    def _input_rows(self, input_ids, positions):
+        embed, rope = self.embed_tokens, self.rotary_emb
+        # One launch for all three, skipping the modules' calls: only where nothing is
+        # attached to them and they are what this model builds.
+        if type(embed) is nn.Embedding and embed.max_norm is None and type(rope) is RotaryEmbedding \
+                and not _has_hooks(embed) and not _has_hooks(rope):
+            rows = embed_rows(input_ids, embed.weight, positions, rope.cos_cached[0, 0], rope.sin_cached[0, 0])
+            if rows is not None:
+                return rows
+        hidden = embed(input_ids)
+        return (hidden, *rope(positions, hidden.dtype))
+
     def forward(self, input_ids, positions):
-        hidden = self.embed_tokens(input_ids)
-        cos, sin = self.rotary_emb(positions, hidden.dtype)
+        hidden, cos, sin = self._input_rows(input_ids, positions)
         residual = None
         for layer in self.layers:
             hidden, residual = layer(hidden, residual, cos, sin)

@@ -369,3 +369,23 @@ extern "C" int bvllm_linear(const void* x, int64_t x_stride, const void* w, cons
   a.m = m; a.n = n; a.k = k;
   return (int)skinny_linear(a, gated != 0, (hipStream_t)stream);
 }
+
+extern "C" int bvllm_embed_rows(const int64_t* ids, const void* table, int64_t vocab, void* out,
+                                const int64_t* positions, const float* cos_table, const float* sin_table,
+                                int64_t max_positions, void* cos_out, void* sin_out, int32_t rows, int32_t hidden,
+                                int32_t head_dim, void* stream) {
+  if (rows < 0 || hidden < 8 || hidden % 8 || head_dim < 8 || head_dim % 8 || vocab < 1 || max_positions < 1)
+    return kBad;
+  if (rows == 0) return 0;
+  if (!ids || !positions || !table || !out || !cos_table || !sin_table || !cos_out || !sin_out) return kBad;
+  if (!aligned16(table) || !aligned16(out) || !aligned16(cos_table) || !aligned16(sin_table) || !aligned16(cos_out) ||
+      !aligned16(sin_out))
+    return kBad;
+  EmbedArgs a{};
+  a.ids = ids; a.table = table; a.out = out;
+  a.positions = positions; a.cos_table = cos_table; a.sin_table = sin_table;
+  a.cos_out = cos_out; a.sin_out = sin_out;
+  a.vocab = vocab; a.max_positions = max_positions;
+  a.rows = rows; a.hidden = hidden; a.head_dim = head_dim;
+  return (int)embed_rows(a, (hipStream_t)stream);
+}

@@ -115,6 +115,18 @@ struct LinearArgs {
   int32_t k_splits, row_groups, unit;
 };
 
+struct EmbedArgs {
+  const int64_t* ids;                      // [rows]
+  const void* table;                       // [vocab, hidden] bf16
+  void* out;                               // [rows, hidden] bf16
+  const int64_t* positions;                // [rows]
+  const float* cos_table; const float* sin_table;  // [max_positions, head_dim]
+  void* cos_out; void* sin_out;            // [rows, head_dim] bf16
+  int64_t vocab, max_positions;
+  int32_t rows, hidden, head_dim;
+};
+hipError_t embed_rows(const EmbedArgs& a, hipStream_t stream);
+
 // How a linear layer of a few tokens runs (skinny_linear.hip).
 struct LinearPlan {
   int32_t rw, kw;          // row waves x k slabs of a work-group; rw = 0: not a shape for this kernel

@@ -301,6 +301,18 @@ BVLLM_API int bvllm_linear(const void* x, int64_t x_stride, const void* w, const
                  int64_t out_stride, int32_t m, int32_t n, int32_t k, int32_t gated, void* workspace,
                  void* stream);
 
+/*
+ * A model's input rows (embed_tokens and rotary_emb of babyvllm/models/qwen2.py:109-118):
+ * out[r] = table[ids[r]] (bf16 [vocab, hidden]); cos_out[r], sin_out[r] = the fp32
+ * tables' rows positions[r], rounded to bf16. A negative position counts from the
+ * table's end; an id or position outside its table gives a row of NaN. hidden and
+ * head_dim multiples of 8, all but ids and positions (int64) 16-byte aligned.
+ */
+BVLLM_API int bvllm_embed_rows(const int64_t* ids, const void* table, int64_t vocab, void* out,
+                     const int64_t* positions, const float* cos_table, const float* sin_table,
+                     int64_t max_positions, void* cos_out, void* sin_out, int32_t rows, int32_t hidden,
+                     int32_t head_dim, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

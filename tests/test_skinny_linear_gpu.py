@@ -112,3 +112,47 @@ def test_module_keeps_autograd_hooks_and_other_types():
         hook.remove()
         assert len(seen) == 1 and seen[0].shape == (4, 256)
         assert gated_linear(x, mlp.gate_up_proj.weight) is not None
+
+
+# ------------------------------------------------------------------ input rows
+
+
+@pytest.mark.parametrize("rows,hidden,dim", [(1, 8, 8), (3, 896, 64), (16, 3584, 128), (65, 264, 72), (700, 3584, 128)])
+def test_embed_rows_equals_torch(rows, hidden, dim):
+    from babyvllm.kernels.embed import embed_rows
+
+    table = torch.randn(50, hidden, device="cuda", dtype=torch.bfloat16)
+    cos, sin = torch.randn(40, dim, device="cuda"), torch.randn(40, dim, device="cuda")
+    ids = torch.randint(0, 50, (rows,), device="cuda")
+    pos = torch.randint(-40, 40, (rows,), device="cuda")
+    with torch.no_grad():
+        got = embed_rows(ids, table, pos, cos, sin)
+    for a, b in zip(got, (table[ids], cos[pos].bfloat16(), sin[pos].bfloat16())):
+        assert torch.equal(a, b) and a.dtype == b.dtype
+    with torch.no_grad():  # outside the tables: NaN rows, the others untouched
+        ids[0], pos[-1] = 50, 40
+        h, c, s = embed_rows(ids, table, pos, cos, sin)
+    assert h[0].isnan().all() and c[-1].isnan().all() and s[-1].isnan().all()
+    assert torch.equal(h[1:], table[ids[1:]])
+
+
+def test_model_input_rows_keep_hooks_and_modules():
+    from babyvllm.config import ModelConfig
+    from babyvllm.models.qwen2 import Qwen2Model
+
+    cfg = ModelConfig(vocab_size=40, hidden_size=128, intermediate_size=256, num_hidden_layers=0,
+                      num_attention_heads=2, num_key_value_heads=1, rms_norm_eps=1e-6, max_position_embeddings=64,
+                      rope_theta=1e4, tie_word_embeddings=True)
+    model = Qwen2Model(cfg).to("cuda")
+    model.embed_tokens.to(torch.bfloat16)
+    ids, pos = torch.tensor([3, 39, 0], device="cuda"), torch.tensor([0, 63, 5], device="cuda")
+    with torch.no_grad():
+        one = model._input_rows(ids, pos)
+        seen = []
+        hook = model.embed_tokens.register_forward_hook(lambda m, i, o: seen.append(o))
+        two = model._input_rows(ids, pos)
+        hook.remove()
+    assert len(seen) == 1
+    for a, b in zip(one, two):
+        assert torch.equal(a, b) and a.dtype == b.dtype
+    assert model._input_rows(ids, pos)[0].requires_grad  # grad mode: torch's operations
