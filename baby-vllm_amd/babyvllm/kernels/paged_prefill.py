@@ -50,6 +50,15 @@ def _split_tiles(md, num_seqs, num_tokens, single, num_heads, num_kv_heads, head
                                                 num_kv_heads, head_dim, width, int(tiles))
 
 
+def _balance_rows(md, num_seqs, num_heads, num_kv_heads):
+    """Whether the single-query rows are cut into chunks (also a choice by the host lists)."""
+    qsl, seq = getattr(md, "query_start_loc_cpu", None), getattr(md, "seq_lens_cpu", None)
+    if qsl is None or seq is None or len(seq) != num_seqs or len(qsl) != num_seqs + 1:
+        return 0
+    pages = [(int(seq[i]) + 15) // 16 for i in range(num_seqs) if qsl[i + 1] - qsl[i] == 1]
+    return _lib.lib().bvllm_prefill_balance_rows(num_heads, num_kv_heads, max(pages), sum(pages)) if pages else 0
+
+
 def paged_prefill_attention(q, kv_cache, md, scale):
     """Causal attention for a flattened varlen batch, reading K/V from the paged cache.
 
@@ -107,10 +116,13 @@ def paged_prefill_attention(q, kv_cache, md, scale):
         num_heads, num_kv_heads, head_dim, page,
     )
     h = _lib.lib()
-    if split_tiles > 0:
-        nbytes = h.bvllm_prefill_workspace_bytes(num_tokens, num_heads, head_dim, bt.shape[1], split_tiles)
+    balance = _balance_rows(md, num_seqs, num_heads, num_kv_heads) if single > 0 else 0
+    if split_tiles > 0 or balance:
+        nbytes = h.bvllm_prefill_workspace_bytes(num_seqs, num_tokens, num_heads, num_kv_heads, head_dim,
+                                                 bt.shape[1], split_tiles, balance)
         workspace = torch.empty(nbytes // 4, device=q.device, dtype=torch.float32)
-        rc = h.bvllm_paged_prefill_split(*args, workspace.data_ptr(), split_tiles, _lib.stream_handle(q.device))
+        rc = h.bvllm_paged_prefill_split(*args, workspace.data_ptr(), split_tiles, balance,
+                                         _lib.stream_handle(q.device))
     else:
         rc = h.bvllm_paged_prefill(*args, _lib.stream_handle(q.device))
     _lib.check(rc, "bvllm_paged_prefill")

@@ -74,6 +74,9 @@ struct PrefillArgs {
   int32_t split_tiles, num_ranges;
   float* part_out;                         // [num_ranges, T, H, D], unnormalized
   float* part_ml;                          // [num_ranges, T, H, 2]: reference max (log2 units), row sum
+  // Balanced single-query rows (RowChunk), or null: decode_chunk_slots() results per head.
+  float* row_part_out;                     // [slots, H, D]
+  float* row_part_lse;                     // [slots, H]
 };
 
 struct ArgmaxArgs {
@@ -148,6 +151,12 @@ hipError_t paged_decode(const DecodeArgs& a, hipStream_t stream);
 // decode_chunk_slots() results per query head: [slots, H, D] and [slots, H].
 hipError_t paged_decode_balanced(const DecodeArgs& a, hipStream_t stream);
 int64_t decode_chunk_slots(int32_t batch, int32_t num_heads, int32_t num_kv_heads);
+// Sets the chunking fields of a launch, and merges its chunks (RowChunk).
+void decode_set_chunks(DecodeArgs& a);
+hipError_t decode_merge_chunks(const DecodeArgs& a, hipStream_t stream);
+// Whether a prefill batch's single-query rows (the longest and all of their pages) are
+// uneven enough that cutting them pays for the merge.
+bool prefill_balance_rows(int32_t num_heads, int32_t num_kv_heads, int64_t longest, int64_t total);
 
 // How a decode launch with the caller's split plan runs (paged_decode.hip).
 struct DecodePlan {

@@ -32,6 +32,7 @@ struct Entry {
   decltype(&bvllm_paged_decode_balanced) balanced = nullptr;
   decltype(&bvllm_paged_prefill) prefill = nullptr;
   decltype(&bvllm_prefill_split_tiles) split_tiles = nullptr;
+  decltype(&bvllm_prefill_balance_rows) balance_rows = nullptr;
   decltype(&bvllm_prefill_workspace_bytes) prefill_bytes = nullptr;
   decltype(&bvllm_paged_prefill_split) prefill_split = nullptr;
   decltype(&bvllm_fused_add_rms_norm) norm = nullptr;
@@ -52,6 +53,7 @@ const BindName kNames[] = {
     {"bvllm_paged_decode_balanced", (void**)&g.balanced},
     {"bvllm_paged_prefill", (void**)&g.prefill},
     {"bvllm_prefill_split_tiles", (void**)&g.split_tiles},
+    {"bvllm_prefill_balance_rows", (void**)&g.balance_rows},
     {"bvllm_prefill_workspace_bytes", (void**)&g.prefill_bytes},
     {"bvllm_paged_prefill_split", (void**)&g.prefill_split},
     {"bvllm_fused_add_rms_norm", (void**)&g.norm},
@@ -281,12 +283,13 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (tokens == 0 || seqs == 0 || c->size(4) != d || hkv == 0 || heads % hkv != 0 || (d & (d - 1)) != 0) return none();
   if (qsl->size(0) != seqs + 1 || ctx->size(0) != seqs || bt->size(0) < seqs) return none();
   if (!small(tokens) || !small(heads) || !small(seqs) || !small(width) || !small(c->size(2))) return none();
-  // Host lists: single-query sequences, and the key tiles of the others' blocks.
+  // Host lists: single-query sequences and their pages, and the key tiles of the
+  // others' blocks.
   if (!PyList_CheckExact(a[6]) || PyList_GET_SIZE(a[6]) != seqs + 1) return none();
   const bool lens_known = PyList_CheckExact(a[7]) && PyList_GET_SIZE(a[7]) == seqs;
   const int64_t split_min = PyLong_AsLongLong(a[10]);
-  const bool may_split = width >= split_min, want_tiles = may_split && lens_known;
-  int64_t single = 0, tiles = want_tiles ? 0 : -1, prev = 0;
+  const bool may_split = width >= split_min;
+  int64_t single = 0, tiles = may_split && lens_known ? 0 : -1, prev = 0, longest = 0, pages = 0;
   for (int64_t i = 0; i <= seqs; ++i) {
     PyObject* o = PyList_GET_ITEM(a[6], i);
     if (!PyLong_CheckExact(o)) return none();
@@ -294,12 +297,17 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (i > 0) {
       const int64_t m = v - prev;
       single += m == 1;
-      if (want_tiles && m > 1) {
+      if (lens_known) {
         PyObject* l = PyList_GET_ITEM(a[7], i - 1);
         if (!PyLong_CheckExact(l)) return none();
         const int64_t len = PyLong_AsLongLong(l);
         if (!small(m) || !small(len)) return none();
-        tiles += cdiv(m * (heads / hkv), 128) * cdiv(len, 64);
+        if (m == 1) {
+          longest = std::max(longest, cdiv(len, 16));
+          pages += cdiv(len, 16);
+        } else if (m > 1 && may_split) {
+          tiles += cdiv(m * (heads / hkv), 128) * cdiv(len, 64);
+        }
       }
     }
     prev = v;
@@ -313,19 +321,22 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int32_t split = !may_split ? 0
                                    : g.split_tiles((int32_t)seqs, (int32_t)tokens, (int32_t)max_q, (int32_t)single,
                                                    (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)width, tiles);
+  const int32_t balance = pages > 0 ? g.balance_rows((int32_t)heads, (int32_t)hkv, longest, pages) : 0;
   at::Tensor out = new_empty({tokens, heads, d}, *q, at::kBFloat16), ws;
-  if (split > 0)
-    ws = new_empty({g.prefill_bytes((int32_t)tokens, (int32_t)heads, (int32_t)d, (int32_t)width, split) / 4}, *q,
-                   at::kFloat);
+  if (split > 0 || balance)
+    ws = new_empty({g.prefill_bytes((int32_t)seqs, (int32_t)tokens, (int32_t)heads, (int32_t)hkv, (int32_t)d,
+                                    (int32_t)width, split, balance) /
+                    4},
+                   *q, at::kFloat);
   return launch(out, [&] {
     const int32_t *tables = bt->const_data_ptr<int32_t>(), *ql = qsl->const_data_ptr<int32_t>();
     const int32_t *sl = seq->const_data_ptr<int32_t>(), *cl = ctx->const_data_ptr<int32_t>();
-    if (split > 0)
+    if (split > 0 || balance)
       return g.prefill_split(ptr(*q), q->stride(0), q->stride(1), ptr(*c), v_half(*c), c->stride(1), c->stride(2),
                              c->stride(3), (int32_t)c->size(1), tables, bt->stride(0), (int32_t)width, ql, sl, cl,
                              scale, ptr(out), out.stride(0), out.stride(1), (int32_t)seqs, (int32_t)tokens,
                              (int32_t)max_q, (int32_t)single, (int32_t)heads, (int32_t)hkv, (int32_t)d,
-                             (int32_t)c->size(2), ptr(ws), split, stream);
+                             (int32_t)c->size(2), ptr(ws), split, balance, stream);
     return g.prefill(ptr(*q), q->stride(0), q->stride(1), ptr(*c), v_half(*c), c->stride(1), c->stride(2),
                      c->stride(3), (int32_t)c->size(1), tables, bt->stride(0), (int32_t)width, ql, sl, cl, scale,
                      ptr(out), out.stride(0), out.stride(1), (int32_t)seqs, (int32_t)tokens, (int32_t)max_q,

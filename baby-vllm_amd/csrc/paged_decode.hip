@@ -69,7 +69,8 @@ __global__ __launch_bounds__(256) void decode_chunks_merge_kernel(DecodeArgs a, 
       for (int i = 0; i < 4; ++i) num[i] = __builtin_fmaf(wgt, o[k][i], num[i]);
     }
   }
-  store_reduced(a, (int64_t)row * a.num_heads + head, d, make_float4(num[0], num[1], num[2], num[3]), den);
+  const int out_row = a.query_start_loc != nullptr ? a.query_start_loc[row] : row;
+  store_reduced(a, (int64_t)out_row * a.num_heads + head, d, make_float4(num[0], num[1], num[2], num[3]), den);
 }
 
 // One streaming wave per work-group, so that a short batch's splits spread
@@ -509,26 +510,36 @@ int64_t decode_chunk_slots(int32_t batch, int32_t num_heads, int32_t num_kv_head
   return (int64_t)batch + chunk_target((int64_t)num_kv_heads * ((G + 15) / 16));
 }
 
-template <int D>
-static hipError_t launch_decode_balanced(const DecodeArgs& args, hipStream_t stream) {
-  DecodeArgs a = args;
+void decode_set_chunks(DecodeArgs& a) {
   const int64_t ncg = decode_col_groups(a);
   a.chunk_target = chunk_target(ncg);
   a.row_slots = (int32_t)std::max<int64_t>(1, device_cus() / ncg);
+}
+
+hipError_t decode_merge_chunks(const DecodeArgs& a, hipStream_t stream) {
+  const int per_row = (a.num_heads * (a.head_dim / 4) + 255) / 256;
+  if ((int64_t)a.batch * per_row > 0x7fffffff) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(a.batch * per_row));
+  if (a.head_dim == 64) hipLaunchKernelGGL((decode_chunks_merge_kernel<64>), grid, dim3(256), 0, stream, a, per_row);
+  else if (a.head_dim == 128) hipLaunchKernelGGL((decode_chunks_merge_kernel<128>), grid, dim3(256), 0, stream, a, per_row);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+template <int D>
+static hipError_t launch_decode_balanced(const DecodeArgs& args, hipStream_t stream) {
+  DecodeArgs a = args;
+  decode_set_chunks(a);
   constexpr int NW = 4;
   constexpr size_t smem = decode_lds_bytes<D, NW>();
   static std::atomic<bool> done[64] = {};
   hipError_t err = allow_lds(&paged_decode_chunks_kernel<D, NW, 1, true>, done, 160 * 1024);
   if (err != hipSuccess) return err;
-  const int64_t wgs = decode_chunk_slots(a.batch, a.num_heads, a.num_kv_heads) * ncg;
-  const int per_row = (a.num_heads * (D / 4) + 255) / 256;
-  if (wgs > 0x7fffffff || (int64_t)a.batch * per_row > 0x7fffffff) return hipErrorInvalidValue;
+  const int64_t wgs = decode_chunk_slots(a.batch, a.num_heads, a.num_kv_heads) * decode_col_groups(a);
+  if (wgs > 0x7fffffff) return hipErrorInvalidValue;
   hipLaunchKernelGGL((paged_decode_chunks_kernel<D, NW, 1, true>), dim3((unsigned)wgs), dim3(NW * 64), smem, stream, a);
   err = hipGetLastError();
-  if (err != hipSuccess) return err;
-  hipLaunchKernelGGL((decode_chunks_merge_kernel<D>), dim3((unsigned)(a.batch * per_row)), dim3(256), 0, stream, a,
-                     per_row);
-  return hipGetLastError();
+  return err != hipSuccess ? err : decode_merge_chunks(a, stream);
 }
 
 hipError_t paged_decode_balanced(const DecodeArgs& a, hipStream_t stream) {

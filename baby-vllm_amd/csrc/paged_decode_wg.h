@@ -375,8 +375,11 @@ constexpr size_t decode_lds_bytes() {
 // is computed and written exactly as in the single pass, the others' fp32 (o, lse)
 // are merged by decode_chunks_merge_kernel. Finding the chunk and the empty merge
 // cost a batch that is not cut 1.1 us (64 x 4096: 86.7 -> 87.7).
-// Nor is any row cut while the longest has at most kCutMinPages pages, the size of
-// plan below which callers run the plain single pass: both give the same bits there.
+// Nor is any row cut while the longest has at most kCutMinPages pages: for a decode
+// batch the size of plan below which callers run the plain single pass (both give the
+// same bits there), and beside a prefill too little to pay for the merge (512 new
+// tokens + 63 rows of 500 to 2000: 36.9 us whole, 42.1 cut; + 9 rows of 4000 to 8000:
+// 106 whole, 42.5 cut).
 constexpr int kMinChunkPages = 32;
 constexpr int kCutMinPages = 128;
 
@@ -392,14 +395,20 @@ struct RowChunk {
 // same answer from the batch's lengths, 64 rows per step.
 __device__ __forceinline__ RowChunk find_row_chunk(const DecodeArgs& a, int item, int item_row) {
   const int lane = lane_id();
+  // Pages of row b; -1 for a row of a prefill batch that is not a single query.
   auto row_pages = [&](int b) {
-    const int len = b < a.batch ? a.seq_lens[b] : 0;
+    if (b >= a.batch) return -1;
+    int len = a.seq_lens[b];
+    if (a.query_start_loc != nullptr) {
+      if (a.query_start_loc[b + 1] - a.query_start_loc[b] != 1) return -1;
+      len = min(len, a.context_lens[b] + 1);
+    }
     return min(len > 0 ? (len + 15) / 16 : 0, a.max_blocks);
   };
   const int n0 = row_pages(lane);
   int total = 0, longest = 0;
   for (int b0 = 0; b0 < a.batch; b0 += 64) {
-    const int n = b0 == 0 ? n0 : row_pages(b0 + lane);
+    const int n = max(b0 == 0 ? n0 : row_pages(b0 + lane), 0);
     total += wave_reduce(n, [](int x, int y) { return x + y; });
     longest = max(longest, wave_reduce(n, [](int x, int y) { return max(x, y); }));
   }
@@ -422,7 +431,7 @@ __device__ __forceinline__ RowChunk find_row_chunk(const DecodeArgs& a, int item
     const int b = b0 + lane;
     const int n = b0 == 0 ? n0 : row_pages(b);
     // (A row with no live token is one empty chunk: it writes zeros.)
-    const int chunks = b < a.batch ? max((n + r.pages - 1) / r.pages, 1) : 0;
+    const int chunks = n < 0 ? 0 : max((n + r.pages - 1) / r.pages, 1);
     int inc = chunks;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {

@@ -136,7 +136,9 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
   const int n_pre_wgs = (int)gridDim.x - n_dec_wgs;
   if ((int)blockIdx.x >= n_pre_wgs) {
     const int dw = (int)blockIdx.x - n_pre_wgs;
-    if (dw < dec.batch * dec.num_kv_heads * col_groups_per_kv(dec.num_heads / dec.num_kv_heads))
+    if (dec.chunk_target > 0)  // uneven rows: cut into chunks (RowChunk)
+      decode_work_group<D, kDecodeWaves, kDecodeDepth, true, true>(dec, dw, reinterpret_cast<float*>(lds));
+    else if (dw < dec.batch * dec.num_kv_heads * col_groups_per_kv(dec.num_heads / dec.num_kv_heads))
       decode_work_group<D, kDecodeWaves, kDecodeDepth, true>(dec, dw, reinterpret_cast<float*>(lds));
     return;
   }
@@ -912,6 +914,11 @@ static DecodeArgs single_query_view(const PrefillArgs& p) {
   a.waves = kDecodeWaves;
   a.query_start_loc = p.query_start_loc;
   a.context_lens = p.context_lens;
+  if (p.row_part_out != nullptr) {
+    a.part_out = p.row_part_out;
+    a.part_lse = p.row_part_lse;
+    decode_set_chunks(a);
+  }
   return a;
 }
 
@@ -950,8 +957,9 @@ static PrefillGrid plan_prefill(const PrefillArgs& a, int64_t CB) {
   p.prefill_wgs = p.xcd_group > 0 ? 8 * ((p.bound + p.xcd_group - 1) / p.xcd_group)
                   : p.xcd_group < 0 ? 8 * p.per_xcd
                                     : p.bound * a.num_kv_heads;
-  // Decode work-groups: one per (sequence, column group), rounded up to whole XCD rounds.
-  p.dec_wgs = a.single_query_seqs != 0 ? ((int64_t)a.num_seqs * a.num_kv_heads * ((G + 15) / 16) + 7) / 8 * 8 : 0;
+  // Decode work-groups: one per (sequence or chunk, column group), rounded up to whole XCD rounds.
+  const int64_t rows = a.row_part_out != nullptr ? decode_chunk_slots(a.num_seqs, a.num_heads, a.num_kv_heads) : a.num_seqs;
+  p.dec_wgs = a.single_query_seqs != 0 ? (rows * a.num_kv_heads * ((G + 15) / 16) + 7) / 8 * 8 : 0;
   return p;
 }
 
@@ -1075,11 +1083,21 @@ static hipError_t prefill_for_dim(const PrefillArgs& a, hipStream_t stream) {
 }
 
 hipError_t paged_prefill(const PrefillArgs& a, hipStream_t stream) {
-  switch (a.head_dim) {
-    case 64: return prefill_for_dim<64>(a, stream);
-    case 128: return prefill_for_dim<128>(a, stream);
-    default: return hipErrorInvalidValue;
-  }
+  hipError_t err = hipErrorInvalidValue;
+  if (a.head_dim == 64) err = prefill_for_dim<64>(a, stream);
+  else if (a.head_dim == 128) err = prefill_for_dim<128>(a, stream);
+  if (err != hipSuccess || a.row_part_out == nullptr || a.single_query_seqs == 0) return err;
+  return decode_merge_chunks(single_query_view(a), stream);
+}
+
+// The device's own rule for the cut (find_row_chunk): no merge launch where it would
+// find nothing to do.
+bool prefill_balance_rows(int32_t num_heads, int32_t num_kv_heads, int64_t longest, int64_t total) {
+  DecodeArgs a{};
+  a.num_heads = num_heads;
+  a.num_kv_heads = num_kv_heads;
+  decode_set_chunks(a);
+  return longest > kCutMinPages && 4 * longest * a.row_slots > 7 * total;
 }
 
 }  // namespace bvllm

@@ -202,23 +202,32 @@ BVLLM_API int bvllm_paged_prefill(const void* q, int64_t q_stride_t, int64_t q_s
                         int32_t block_size, void* stream);
 
 /*
- * The same, with each sequence's keys cut into ranges of split_tiles 64-key tiles,
- * every (block, range) on a work-group of its own, and a second launch that adds the
- * ranges' fp32 partials: for few new tokens behind long prefixes, where the plain
- * launch leaves most of the chip idle. bvllm_prefill_split_tiles returns the
- * split_tiles to use for a batch's shape, or 0 where the plain launch is the better one;
- * key_tiles is the number of 64-key tiles the batch's blocks of 128 (query, head)
- * pairs cover, per KV head, summed over its sequences of more than one query token
- * (ceil(G * q_len / 128) * ceil(seq_len / 64)), or -1 if unknown; it steers the choice
- * only, never what is computed. workspace holds bvllm_prefill_workspace_bytes() bytes.
+ * The same with two ways of spreading uneven work over the chip, each paid for by a
+ * second launch that adds fp32 partials:
+ *   split_tiles > 0: each sequence's keys are cut into ranges of split_tiles 64-key
+ *     tiles, every (block, range) on a work-group of its own, for few new tokens
+ *     behind long prefixes;
+ *   balance_rows = 1: the single-query sequences' rows are cut into chunks chosen on
+ *     the device from their lengths (as bvllm_paged_decode_balanced does), for decode
+ *     rows far from equal or few.
+ * bvllm_prefill_split_tiles returns the split_tiles to use for a batch's shape, or 0
+ * where the plain launch is the better one; key_tiles is the number of 64-key tiles the
+ * batch's blocks of 128 (query, head) pairs cover, per KV head, summed over its
+ * sequences of more than one query token (ceil(G * q_len / 128) * ceil(seq_len / 64)),
+ * or -1 if unknown. bvllm_prefill_balance_rows returns whether cutting pays, from the
+ * pages of the longest single-query row and of all of them. Both steer the choice only,
+ * never what is computed. workspace holds bvllm_prefill_workspace_bytes() bytes.
  * Results agree with bvllm_paged_prefill within the rounding of fp32 sums in another
- * order. A sequence's keys end at its table's last page.
+ * order; a sequence's keys end at its table's last page.
  */
 BVLLM_API int32_t bvllm_prefill_split_tiles(int32_t num_seqs, int32_t num_tokens, int32_t max_query_len,
                         int32_t single_query_seqs, int32_t num_heads, int32_t num_kv_heads,
                         int32_t head_dim, int32_t max_blocks, int64_t key_tiles);
-BVLLM_API int64_t bvllm_prefill_workspace_bytes(int32_t num_tokens, int32_t num_heads, int32_t head_dim,
-                        int32_t max_blocks, int32_t split_tiles);
+BVLLM_API int32_t bvllm_prefill_balance_rows(int32_t num_heads, int32_t num_kv_heads, int64_t longest_pages,
+                        int64_t total_pages);
+BVLLM_API int64_t bvllm_prefill_workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t num_heads,
+                        int32_t num_kv_heads, int32_t head_dim, int32_t max_blocks,
+                        int32_t split_tiles, int32_t balance_rows);
 BVLLM_API int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                         const void* k_cache, const void* v_cache,
                         int64_t cache_stride_block, int64_t cache_stride_tok, int64_t cache_stride_head,
@@ -230,7 +239,8 @@ BVLLM_API int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int64
                         int32_t num_seqs, int32_t num_tokens, int32_t max_query_len,
                         int32_t single_query_seqs,
                         int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
-                        int32_t block_size, void* workspace, int32_t split_tiles, void* stream);
+                        int32_t block_size, void* workspace, int32_t split_tiles,
+                        int32_t balance_rows, void* stream);
 
 /*
  * Tuning switch for experiments and tests (no counterpart in the reference):

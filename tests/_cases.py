@@ -126,3 +126,15 @@ def tuned(knob: int, value: int):
         yield
     finally:
         _lib.set_tuning(knob, prev)
+
+
+class _Declining:
+    """Stands in for the wrappers' native host side: every call takes the Python path."""
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+def python_path(monkeypatch):
+    from babyvllm.kernels import _lib
+    monkeypatch.setattr(_lib, "fast", lambda: _Declining())

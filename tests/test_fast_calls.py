@@ -6,7 +6,7 @@ import random
 import pytest
 import torch
 
-from tests._cases import build_prefill_case, make_decode_inputs
+from tests._cases import build_prefill_case, make_decode_inputs, python_path
 
 
 
@@ -38,19 +38,6 @@ def test_cpu_tensors_and_wrong_argument_counts_are_declined():
     assert f.norm() is None and f.decode(x) is None and f.prefill() is None and f.rope(x, x) is None
 
 
-class _Declining:
-    """Stands in for the native module: every call takes the Python path."""
-
-    def __getattr__(self, name):
-        return lambda *a: None
-
-
-def _python_path(monkeypatch):
-    from babyvllm.kernels import _lib
-
-    monkeypatch.setattr(_lib, "fast", lambda: _Declining())
-
-
 def _calls():
     from babyvllm.kernels.activation import fused_silu_mul
     from babyvllm.kernels.layernorm import fused_add_rms_norm
@@ -79,9 +66,10 @@ def _calls():
         dq, dc, bt, sl = make_decode_inputs(lens)
         for bucket in (None, max(lens), 4096):
             out["decode", len(lens), bucket] = paged_decode_attention(dq, dc, bt, sl, 0.1, max_seq_len=bucket)
-    for specs in ([(0, 20), (30, 1), (5, 70)], [(5000, 40), (3000, 7)]):
+    for specs in ([(0, 20), (30, 1), (5, 70)], [(5000, 40), (3000, 7)], [(0, 50), (4000, 1), (9, 1), (20, 1)],
+                  [(6000, 40), (3000, 1), (40, 7), (70, 1), (9, 1)]):
         pq, pc, md = build_prefill_case(specs, 4, 7, 128)
-        out["prefill", len(specs)] = paged_prefill_attention(pq, pc, md, 0.1)
+        out["prefill", str(specs)] = paged_prefill_attention(pq, pc, md, 0.1)
     return out
 
 
@@ -89,7 +77,7 @@ def _calls():
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a ROCm GPU")
 def test_calls_equal_the_python_path(monkeypatch):
     native = _calls()
-    _python_path(monkeypatch)
+    python_path(monkeypatch)
     python = _calls()
     assert native.keys() == python.keys()
     for name in native:

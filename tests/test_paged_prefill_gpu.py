@@ -9,7 +9,8 @@ import pytest
 import torch
 
 from oracle import attention as oa
-from tests._cases import assert_attn_close, build_prefill_case, md_to_cpu, scale_keys_by_position, tuned
+from tests._cases import (assert_attn_close, build_prefill_case, md_to_cpu, python_path, scale_keys_by_position,
+                          tuned)
 
 _BPW = 1  # tuning knob: prefill column blocks per work-group (bvllm_set_tuning)
 _SHORT_GRID = 6  # tuning knob: 1 = short grids on the single key walk instead of the key split
@@ -431,6 +432,7 @@ def test_key_ranges_match_oracle(case, tiles, hkv, group, d, monkeypatch):
     scale_keys_by_position(kv_cache, md.block_tables, md.seq_lens_cpu, lambda p: 1.0 + 0.002 * p)
     expected = _oracle(q, kv_cache, md, group)
     plain = _kernel()(q, kv_cache, md, d ** -0.5)
+    python_path(monkeypatch)  # (the native side makes the choice itself)
     monkeypatch.setattr(pp, "_split_tiles", lambda *a: tiles)
     actual = _kernel()(q, kv_cache, md, d ** -0.5)
     assert_attn_close(actual, expected)
@@ -454,3 +456,38 @@ def test_key_ranges_chosen_for_short_turns_behind_long_prefixes():
     # Wide tables beside a full grid, and narrow tables, keep the plain launch.
     assert pp._split_tiles(build_prefill_case([(2048, 2048)], 4, 7, 128)[2], 1, 2048, 0, 28, 4, 128, 256) == 0
     assert pp._split_tiles(*args, 8) == 0
+
+
+@pytest.mark.parametrize("tiles", [0, 4])
+@pytest.mark.parametrize("hkv,group,d", [(4, 7, 128), (2, 7, 64), (1, 33, 128)])
+def test_uneven_decode_rows_of_a_mixed_step(tiles, hkv, group, d, monkeypatch):
+    """Decode rows cut into chunks beside prefill sequences (with and without key ranges):
+    against the oracle; a row short enough to stay whole keeps the plain launch's bits;
+    more sequences than a wave's lanes; an empty-context row and one query of a page."""
+    import babyvllm.kernels.paged_prefill as pp
+
+    specs = [(5000, 1), (0, 1), (0, 200), (15, 1), (700, 1), (300, 20), (2999, 1)] + [(60, 1)] * 70
+    q, kv_cache, md = build_prefill_case(specs, hkv, group, d)
+    scale_keys_by_position(kv_cache, md.block_tables, md.seq_lens_cpu, lambda p: 1.0 + 0.001 * p)
+    expected = _oracle(q, kv_cache, md, group)
+    assert pp._balance_rows(md, len(specs), hkv * group, hkv) == 1
+    assert_attn_close(_kernel()(q, kv_cache, md, d ** -0.5), expected)
+    python_path(monkeypatch)
+    monkeypatch.setattr(pp, "_split_tiles", lambda *a: tiles)
+    actual = _kernel()(q, kv_cache, md, d ** -0.5)
+    assert_attn_close(actual, expected)
+    monkeypatch.setattr(pp, "_balance_rows", lambda *a: 0)
+    plain = _kernel()(q, kv_cache, md, d ** -0.5)
+    whole = [md.query_start_loc_cpu[i] for i, (c, n) in enumerate(specs) if n == 1 and c < 512]
+    assert torch.equal(actual[whole], plain[whole])
+
+
+def test_even_decode_rows_keep_the_plain_launch():
+    import babyvllm.kernels.paged_prefill as pp
+
+    even = build_prefill_case([(0, 64)] + [(1000, 1)] * 63, 4, 7, 128)[2]
+    assert pp._balance_rows(even, 64, 28, 4) == 0
+    few = build_prefill_case([(0, 64)] + [(3000, 1)] * 9, 4, 7, 128)[2]
+    assert pp._balance_rows(few, 10, 28, 4) == 1
+    few.seq_lens_cpu = None
+    assert pp._balance_rows(few, 10, 28, 4) == 0
