@@ -4,7 +4,7 @@
 decode step's linear layers (and an MLP's fused gate/up projection with SiLU·mul)
 with ``bvllm_linear`` and return the result, or return ``None`` when the call is not
 one for that kernel; the caller then takes torch's own operations. The kernel takes
-plain bf16 tensors of at most 64 rows on the current ROCm device, outside autograd
+plain bf16 tensors of at most 64 rows (256 where K is long and N short) on the current ROCm device, outside autograd
 and outside every mode that has to see torch operations (tracing, compilation,
 functorch transforms, forward-mode AD, dispatch and function modes, autocast).
 """
@@ -16,7 +16,7 @@ from torch.autograd import forward_ad
 
 from babyvllm.kernels import _lib
 
-MAX_ROWS = 64
+MAX_ROWS = 256
 
 
 def torch_must_see(*tensors) -> bool:
@@ -31,14 +31,14 @@ def torch_must_see(*tensors) -> bool:
 
 
 def skinny_linear(x, weight, bias=None, out=None):
-    """``x @ weight.T + bias`` for x [M ≤ 64, K] (into ``out`` if given), or None."""
+    """``x @ weight.T + bias`` for x [M, K] (into ``out`` if given), or None."""
     if not x.is_cuda or x.dim() != 2 or x.shape[0] > MAX_ROWS or torch_must_see(x, weight, bias, out):
         return None
     return _lib.fast().linear(x, weight, bias, out, False, *_lib.current())
 
 
 def gated_linear(x, weight):
-    """``silu(x @ gate.T) * (x @ up.T)`` for weight = [gate; up], x [M ≤ 64, K], or None.
+    """``silu(x @ gate.T) * (x @ up.T)`` for weight = [gate; up], x [M, K], or None.
 
     Gate and up stay fp32 up to the product (torch's two steps round them to bf16 first).
     """

@@ -31,7 +31,8 @@
 // Measured against hipBLASLt (+ the SiLU·mul launch for gated), us, weights from
 // HBM, graph of back-to-back calls:
 //   gate/up 2·18944 x 3584: 1 token 56 + 3 -> 47, 16: 54 + 3 -> 50, 64: 60 + 3 -> 63
-//   down 3584 x 18944:      16 tokens 45.7 -> 29, 32: 109 -> 32, 64: 90 -> 35
+//   down 3584 x 18944:      16 tokens 48 -> 29, 32: 110 -> 32, 64: 91 -> 36, 128: 99 -> 47,
+//                           256 (two blocks of 128 side by side, weights shared in cache): 126 -> 83
 //   head 152064 x 3584:     1 token 228 -> 177, 16: 231 -> 188, 32: 250 -> 197
 //   qkv 4608 x 3584:        16 tokens 12.3 -> 10.4;  out 3584 x 3584: 11.9 -> 9.6
 #include "bvllm_device.h"
@@ -98,6 +99,7 @@ __global__ __launch_bounds__(RW * KW * 64) void skinny_linear_kernel(LinearArgs 
   const int lane = lane_id(), n = lane & 15, g = lane >> 4, w = wave_id();
   const int rw = w % RW, kw = w / RW;
   const int ks = (int)blockIdx.x % a.k_splits, rg = (int)blockIdx.x / a.k_splits;
+  const int m0 = (int)blockIdx.y * MT * 16, m_here = min(a.m - m0, MT * 16);  // the token block
   const int row0 = group_row(a.n, a.unit, rg, a.row_groups);
   const int row1 = group_row(a.n, a.unit, rg + 1, a.row_groups);
 
@@ -110,7 +112,8 @@ __global__ __launch_bounds__(RW * KW * 64) void skinny_linear_kernel(LinearArgs 
   for (int q = 0; q < KW; ++q) steps = max(steps, slab(ks * KW + q + 1) - slab(ks * KW + q));
 
   const uint32_t w_bytes = (GLU ? 2u : 1u) * (uint32_t)a.n * (uint32_t)a.k * 2u;
-  const uint32_t x_bytes = (uint32_t)a.m * (uint32_t)a.x_stride * 2u;
+  const uint32_t x_bytes = (uint32_t)m_here * (uint32_t)a.x_stride * 2u;
+  const uint16_t* x = reinterpret_cast<const uint16_t*>(a.x) + (int64_t)m0 * a.x_stride;
   const int col = row0 + 16 * (rw % CW) + n;
   const uint32_t w_row = (uint32_t)(col + (GLU && rw >= CW ? a.n : 0));
   const uint32_t w_off = col < row1 ? w_row * (uint32_t)a.k * 2u + 16u * g : kNoLoad;
@@ -119,7 +122,7 @@ __global__ __launch_bounds__(RW * KW * 64) void skinny_linear_kernel(LinearArgs 
   for (int i = 0; i < XL; ++i) {
     const int e = (i * RW + rw) * 64 + lane;  // row e / 16, chunk e mod 16; rows past m read as zeros
     const int r = e >> 4, c = e & 15;
-    x_off[i] = r < MT * 16 && r < a.m ? (uint32_t)r * (uint32_t)a.x_stride * 2u + 16u * c : kNoLoad;
+    x_off[i] = r < m_here ? (uint32_t)r * (uint32_t)a.x_stride * 2u + 16u * c : kNoLoad;
     x_dst[i] = (uint32_t)(kw * XB + r * 256 + 16 * (c ^ (r & 15)));
   }
 
@@ -128,7 +131,7 @@ __global__ __launch_bounds__(RW * KW * 64) void skinny_linear_kernel(LinearArgs 
   // (the counter retires in order) leaves the younger stages in flight.
   auto issue = [&](int d, int j) __attribute__((always_inline)) {
     const bool on = j < j1;
-    const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, on ? x_bytes : 0u, 0x00027000);
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, on ? x_bytes : 0u, 0x00027000);
     const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.w), 0, on ? w_bytes : 0u, 0x00027000);
     const uint32_t off = (uint32_t)j * (2u * kStageK);
 #pragma unroll
@@ -187,8 +190,8 @@ summed:
       return y;
     };
     // Lane n + 16g of a result tile: token 16t + n, columns 4g .. 4g + 3.
-    const int m = 16 * t + (l & 15), c = row0 + 16 * r + 4 * (l >> 4);
-    if (m >= a.m || c >= row1) continue;
+    const int mb = 16 * t + (l & 15), m = m0 + mb, c = row0 + 16 * r + 4 * (l >> 4);
+    if (mb >= m_here || c >= row1) continue;
     f32x4_t y = sum(r), u = y;
     if constexpr (GLU) u = sum(CW + r);
     if (a.k_splits > 1) {
@@ -242,7 +245,7 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(LinearArgs a) {
 
 template <int MT, int RW, int KW, int D, bool GLU>
 hipError_t launch_tiles(const LinearArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((skinny_linear_kernel<MT, RW, KW, D, GLU>), dim3((unsigned)(a.row_groups * a.k_splits)),
+  hipLaunchKernelGGL((skinny_linear_kernel<MT, RW, KW, D, GLU>), dim3((unsigned)(a.row_groups * a.k_splits), (unsigned)((a.m + MT * 16 - 1) / (MT * 16))),
                      dim3(RW * KW * 64), 0, s, a);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess || a.k_splits == 1) return err;
@@ -255,6 +258,11 @@ template <int RW, int KW, int D, bool GLU>
 hipError_t launch_waves(const LinearArgs& a, hipStream_t s) {
   if (a.m <= 16) return launch_tiles<1, RW, KW, D, GLU>(a, s);
   if (a.m <= 32) return launch_tiles<2, RW, KW, D, GLU>(a, s);
+  if constexpr (RW == 8 && !GLU) {  // beyond 64 tokens (linear_plan): blocks of at most 128, evenly
+    const int per_block = (a.m + (a.m + 127) / 128 - 1) / ((a.m + 127) / 128);
+    if (per_block > 96) return launch_tiles<8, RW, KW, D, GLU>(a, s);
+    if (per_block > 64) return launch_tiles<6, RW, KW, D, GLU>(a, s);
+  }
   return launch_tiles<4, RW, KW, D, GLU>(a, s);
 }
 
@@ -269,7 +277,9 @@ hipError_t launch_waves(const LinearArgs& a, hipStream_t s) {
 //     59.6 / 66.6; 152064 x 3584, 64 tokens: 216 / 201);
 //   long k (>= 64 stages, or >= 32 with few rows and more than 16 tokens): 4 row
 //     waves x 2 slabs, k cut over work-groups until tiles x splits reach about
-//     1000 (past 32 tokens and 64 stages 8 x 1, twice the splits);
+//     1000 (past 32 tokens and 64 stages 8 x 1, twice the splits). From 64 stages on
+//     up to 256 tokens, in blocks of at most 128 (3584 x 18944: 96 tokens 43 / 95, 128:
+//     50 / 99);
 //   the rest: 2 x 4 from 160 tiles, 1 x 4 below (each work-group then streams a
 //     few rows with 4 waves and no sum across work-groups). Past 32 tokens x
 //     outweighs the weights of so few rows per work-group: 3584 x 3584 stays with
@@ -277,9 +287,10 @@ hipError_t launch_waves(const LinearArgs& a, hipStream_t s) {
 LinearPlan linear_plan(int32_t m, int32_t n, int32_t k, bool gated) {
   LinearPlan p{};
   const int64_t rows = (gated ? 2 : 1) * (int64_t)n;
-  if (m < 1 || m > 64 || n < 64 || n % 4 != 0 || k < kStageK || k % kStageK != 0) return p;
+  if (m < 1 || m > 256 || n < 64 || n % 4 != 0 || k < kStageK || k % kStageK != 0) return p;
   if (rows * k * 2 >= (int64_t)kNoLoad) return p;
   const int tiles = (n + 15) / 16, stages = k / kStageK;
+  if (m > 64 && (gated || tiles >= 2048 || stages < 64)) return p;
   p.k_splits = 1;
   if (gated) {
     p.rw = n >= 8192 ? 8 : 4;

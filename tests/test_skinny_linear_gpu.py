@@ -15,6 +15,8 @@ SHAPES = [
     (33, 4608, 3584, False), (1, 32772, 256, False), (16, 33000, 896, False), (48, 32768, 1024, False),
     (2, 896, 8192, False), (16, 900, 18944, False), (33, 3584, 8320, False), (64, 260, 18944, False),
     (24, 896, 4864, False), (64, 896, 4864, False),
+    (65, 900, 8320, False), (128, 3584, 8192, False), (129, 260, 18944, False), (200, 896, 8192, False),
+    (256, 3584, 18944, False),
     (1, 64, 128, True), (16, 4864, 896, True), (33, 4868, 896, True), (64, 8196, 384, True),
     (16, 18944, 3584, True), (17, 9000, 640, True),
 ]
