@@ -95,7 +95,7 @@ SIGNATURES = {
         _i32, _i32, _i32, _i32,     # H, Hkv, D, block_size
         _p, _i32, _i32, _p,         # workspace, split_tiles, balance_rows, stream
     ]),
-    "bvllm_prefill_split_tiles": (ctypes.c_int32, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i64]),
+    "bvllm_prefill_split_tiles": (ctypes.c_int32, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i64, _i64]),
     "bvllm_prefill_balance_rows": (ctypes.c_int32, [_i32, _i32, _i64, _i64]),
     "bvllm_prefill_workspace_bytes": (ctypes.c_int64, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "bvllm_set_tuning": (ctypes.c_int, [_i32, _i32]),

@@ -38,16 +38,18 @@ def _split_tiles(md, num_seqs, num_tokens, single, num_heads, num_kv_heads, head
     """
     if width < _SPLIT_MIN_PAGES:
         return 0
-    tiles = -1
+    tiles = longest = -1
     qsl, seq = getattr(md, "query_start_loc_cpu", None), getattr(md, "seq_lens_cpu", None)
     if single >= 0 and qsl is not None and seq is not None and len(seq) == num_seqs and len(qsl) == num_seqs + 1:
-        group, tiles = num_heads // num_kv_heads, 0
+        group, tiles, longest = num_heads // num_kv_heads, 0, 0
         for i in range(num_seqs):
             n = qsl[i + 1] - qsl[i]
             if n > 1:
-                tiles += ((n * group + 127) >> 7) * ((seq[i] + 63) >> 6)
+                keys = (int(seq[i]) + 63) >> 6
+                tiles += ((int(n) * group + 127) >> 7) * keys
+                longest = max(longest, keys)
     return _lib.lib().bvllm_prefill_split_tiles(num_seqs, num_tokens, int(md.max_query_len), single, num_heads,
-                                                num_kv_heads, head_dim, width, int(tiles))
+                                                num_kv_heads, head_dim, width, tiles, longest)
 
 
 def _balance_rows(md, num_seqs, num_heads, num_kv_heads):

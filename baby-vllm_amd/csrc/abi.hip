@@ -245,7 +245,8 @@ extern "C" int bvllm_paged_prefill(const void* q, int64_t q_stride_t, int64_t q_
 
 extern "C" int32_t bvllm_prefill_split_tiles(int32_t num_seqs, int32_t num_tokens, int32_t max_query_len,
                                              int32_t single_query_seqs, int32_t num_heads, int32_t num_kv_heads,
-                                             int32_t head_dim, int32_t max_blocks, int64_t key_tiles) {
+                                             int32_t head_dim, int32_t max_blocks, int64_t key_tiles,
+                                             int64_t longest_tiles) {
   if (num_seqs < 1 || num_tokens < 1 || max_query_len < 1 || max_blocks < 1) return 0;
   if (!valid_heads(num_heads, num_kv_heads) || (head_dim != 64 && head_dim != 128)) return 0;
   if (single_query_seqs < -1 || single_query_seqs > num_seqs) return 0;
@@ -254,7 +255,7 @@ extern "C" int32_t bvllm_prefill_split_tiles(int32_t num_seqs, int32_t num_token
   a.single_query_seqs = single_query_seqs;
   a.num_heads = num_heads; a.num_kv_heads = num_kv_heads; a.head_dim = head_dim;
   a.max_blocks = max_blocks;
-  return prefill_split_tiles(a, key_tiles);
+  return prefill_split_tiles(a, key_tiles, longest_tiles);
 }
 
 extern "C" int32_t bvllm_prefill_balance_rows(int32_t num_heads, int32_t num_kv_heads, int64_t longest_pages,

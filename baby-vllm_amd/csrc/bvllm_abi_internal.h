@@ -191,15 +191,17 @@ enum TuneKnob {
   kTuneDecodeSinglePassStream = 3,  // 1: single-pass launches on streaming waves too (same bits)
   kTuneDecodeCached = 4,            // 1: streaming page loads without the nontemporal hint (same bits)
   kTuneAppendChunks = 5,            // 1: aligned appends on the per-chunk kernel (same bits, NaN payloads aside)
-  kTunePrefillShortGrid = 6,        // 1: short prefill grids on the single key walk instead of the key split
+  kTunePrefillShortGrid = 6,        // 1: short prefill grids on the single key walk instead of the key split;
+                                    // 2: on 64-column blocks also with at most one per CU
   kTuneKnobs = 7,
 };
 int tuning(int knob);
 int set_tuning(int knob, int value);
 hipError_t paged_prefill(const PrefillArgs& a, hipStream_t stream);
 // Key ranges of a prefill launch: tiles per range (0: no split) for the batch's shape
-// (key_tiles: 64-key tiles its 128-column blocks walk per KV head, or < 0 if unknown).
-int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles);
+// (key_tiles: 64-key tiles its 128-column blocks walk per KV head, longest_tiles: those of
+// its longest sequence of more than one query; < 0 if unknown).
+int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles, int64_t longest_tiles);
 inline int32_t prefill_ranges(int32_t max_blocks, int32_t split_tiles) {
   return ((max_blocks + 3) / 4 + split_tiles - 1) / split_tiles;
 }

@@ -290,6 +290,7 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t split_min = PyLong_AsLongLong(a[10]);
   const bool may_split = width >= split_min;
   int64_t single = 0, tiles = may_split && lens_known ? 0 : -1, prev = 0, longest = 0, pages = 0;
+  int64_t longest_tiles = tiles;
   for (int64_t i = 0; i <= seqs; ++i) {
     PyObject* o = PyList_GET_ITEM(a[6], i);
     if (!PyLong_CheckExact(o)) return none();
@@ -307,6 +308,7 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
           pages += cdiv(len, 16);
         } else if (m > 1 && may_split) {
           tiles += cdiv(m * (heads / hkv), 128) * cdiv(len, 64);
+          longest_tiles = std::max(longest_tiles, cdiv(len, 64));
         }
       }
     }
@@ -320,7 +322,8 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!small(max_q)) return none();
   const int32_t split = !may_split ? 0
                                    : g.split_tiles((int32_t)seqs, (int32_t)tokens, (int32_t)max_q, (int32_t)single,
-                                                   (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)width, tiles);
+                                                   (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)width, tiles,
+                                                   longest_tiles);
   const int32_t balance = pages > 0 ? g.balance_rows((int32_t)heads, (int32_t)hkv, longest, pages) : 0;
   at::Tensor out = new_empty({tokens, heads, d}, *q, at::kBFloat16), ws;
   if (split > 0 || balance)

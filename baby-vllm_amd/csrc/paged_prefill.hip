@@ -1024,9 +1024,9 @@ static hipError_t launch_prefill_split(const PrefillArgs& a, hipStream_t stream)
 
 // Whether a batch's keys are cut into ranges, and how long. Only grids short of two
 // 128-column work-groups per CU are looked at. Times (us) as measured here:
-//   unsplit (64-column key split): 7 + 0.79 per tile of the longest walk with at
-//     most one work-group per CU, 1.1 beyond (107 tiles, 176 work-groups: 92;
-//     126 tiles, 28: 106; 71 tiles, 440: 89);
+//   unsplit (key split): 5.5 + 0.6 per tile of the longest walk with at most one 64-
+//     column work-group per CU (7 + 0.79 beside decode rows), 7 + 1.1 beyond (25 tiles,
+//     28 work-groups: 19.6; 107 tiles, 176, as 64-column blocks: 92; 71 tiles, 440: 89);
 //   split: 14 of start and merge, + the partials' bytes twice at 8 TB/s, + per tile
 //     1.07 to 1.4 with one work-group per CU, 1.75 with two (the rate of a full
 //     grid). Ranges shorter than 8 tiles gain nothing over their fixed cost.
@@ -1035,15 +1035,15 @@ static hipError_t launch_prefill_split(const PrefillArgs& a, hipStream_t stream)
 // 60 us at 13 tiles per range, 46 at 15, 51 at 20, 75 at 48; 92 unsplit). 0.86 of the
 // slots, since blocks fall unevenly on the XCDs; one work-group per CU beside decode
 // rows (100 new tokens behind 6000 + 20 rows: 44 us at 7 tiles, 34 at 15; 83 unsplit).
-int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles) {
+int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles, int64_t longest_tiles) {
   const PrefillGrid p = plan_prefill(a, 4 * 2 * 16);
   const double cus = device_cus(), hkv = a.num_kv_heads;
   if (p.bound <= 0 || p.prefill_wgs >= 2 * (int64_t)cus) return 0;
-  const double longest = (a.max_blocks + 3) / 4;
+  const double longest = std::min<int64_t>((a.max_blocks + 3) / 4, longest_tiles >= 0 ? longest_tiles : INT32_MAX);
   const double steps = hkv * (key_tiles >= 0 ? (double)key_tiles : p.bound * longest);
   const double blocks = hkv * p.bound;
-  const double walk = std::min(longest, std::max(steps / hkv, 1.0));
-  const double unsplit = 7.0 + (2.0 * blocks <= cus ? 0.79 : 1.1) * walk;
+  const bool narrow = 2.0 * blocks <= cus && p.dec_wgs == 0;
+  const double unsplit = narrow ? 5.5 + 0.6 * longest : 7.0 + (2.0 * blocks <= cus ? 0.79 : 1.1) * longest;
   double best = 0.9 * unsplit;
   int32_t tiles = 0;
   for (int per_cu = 1; per_cu <= (p.dec_wgs > 0 ? 1 : 2); ++per_cu) {
@@ -1069,6 +1069,13 @@ int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles) {
 // every key tile; 8 x (1024 + 128): 29.4-29.9 us against 31.3-31.7 us for one
 // column tile per wave over every key, the choice behind the tuning switch
 // kTunePrefillShortGrid; mixed 1 x 512 + 63 decodes: 29.3-30.0 us either way).
+// With at most one such work-group per CU a tile step is one wave's dependency chain on
+// each SIMD (a third K/V tile in LDS, so that no step waits for its own loads, changed
+// nothing at D = 64), so each wave takes one column tile instead of two: half the chain
+// and twice the work-groups (1 x 64: 6.9 -> 5.5 us, 1 x 560: 14.1 -> 12.1, 40 behind 1500:
+// 25.1 -> 19.6, 0.5B 1 x 1000: 14.3 -> 11.8). Not with more (8 x 60-120 tokens, 316
+// work-groups of 64: 11.0 against 13.2; 800 tokens, 352: 19.1 either way), nor beside
+// decode rows, which the extra work-groups delay (1 x 512 + 63 x 1001: 28.3 against 41.4).
 template <int D>
 static hipError_t prefill_for_dim(const PrefillArgs& a, hipStream_t stream) {
   if (a.split_tiles > 0) return launch_prefill_split<D>(a, stream);
@@ -1079,7 +1086,10 @@ static hipError_t prefill_for_dim(const PrefillArgs& a, hipStream_t stream) {
     return launch_prefill<D, 4, 2>(a, plan_prefill(a, 4 * 2 * 16 * (int64_t)bpw), bpw, stream);
   }
   if (tuning(kTunePrefillShortGrid) == 1) return launch_prefill<D, 4, 1>(a, plan_prefill(a, 4 * 1 * 16), 1, stream);
-  return launch_prefill<D, 4, 2, 2>(a, plan_prefill(a, 4 / 2 * 2 * 16), 1, stream);
+  const PrefillGrid p1 = plan_prefill(a, 4 / 2 * 2 * 16);
+  if (tuning(kTunePrefillShortGrid) != 2 && p1.dec_wgs == 0 && p1.prefill_wgs <= (int64_t)device_cus())
+    return launch_prefill<D, 4, 1, 2>(a, plan_prefill(a, 4 / 2 * 1 * 16), 1, stream);
+  return launch_prefill<D, 4, 2, 2>(a, p1, 1, stream);
 }
 
 hipError_t paged_prefill(const PrefillArgs& a, hipStream_t stream) {

@@ -214,7 +214,7 @@ BVLLM_API int bvllm_paged_prefill(const void* q, int64_t q_stride_t, int64_t q_s
  * where the plain launch is the better one; key_tiles is the number of 64-key tiles the
  * batch's blocks of 128 (query, head) pairs cover, per KV head, summed over its
  * sequences of more than one query token (ceil(G * q_len / 128) * ceil(seq_len / 64)),
- * or -1 if unknown. bvllm_prefill_balance_rows returns whether cutting pays, from the
+ * longest_tiles the tiles of the longest of them (ceil(seq_len / 64)), each -1 if unknown. bvllm_prefill_balance_rows returns whether cutting pays, from the
  * pages of the longest single-query row and of all of them. Both steer the choice only,
  * never what is computed. workspace holds bvllm_prefill_workspace_bytes() bytes.
  * Results agree with bvllm_paged_prefill within the rounding of fp32 sums in another
@@ -222,7 +222,7 @@ BVLLM_API int bvllm_paged_prefill(const void* q, int64_t q_stride_t, int64_t q_s
  */
 BVLLM_API int32_t bvllm_prefill_split_tiles(int32_t num_seqs, int32_t num_tokens, int32_t max_query_len,
                         int32_t single_query_seqs, int32_t num_heads, int32_t num_kv_heads,
-                        int32_t head_dim, int32_t max_blocks, int64_t key_tiles);
+                        int32_t head_dim, int32_t max_blocks, int64_t key_tiles, int64_t longest_tiles);
 BVLLM_API int32_t bvllm_prefill_balance_rows(int32_t num_heads, int32_t num_kv_heads, int64_t longest_pages,
                         int64_t total_pages);
 BVLLM_API int64_t bvllm_prefill_workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t num_heads,
@@ -255,9 +255,10 @@ BVLLM_API int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int64
  * 4 decode page loads of the streaming waves without the nontemporal hint
  * (1), 5 aligned RoPE + append on the per-chunk kernel instead of the
  * per-row kernel (1), 6 short prefill grids on the single key walk instead of
- * the in-work-group key split (1). Knobs 0-5 change no result bit (a NaN's
- * payload aside); knob 6 changes the prefill's summation order (both paths
- * within the same tolerance of the reference).
+ * the in-work-group key split (1), or on it in blocks of 64 columns also where
+ * the grid has at most one per compute unit (2). Knobs 0-5 change no result bit
+ * (a NaN's payload aside); knob 6 changes the prefill's summation order (all
+ * paths within the same tolerance of the reference).
  */
 BVLLM_API int bvllm_set_tuning(int32_t knob, int32_t value);
 

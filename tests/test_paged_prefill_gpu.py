@@ -491,3 +491,17 @@ def test_even_decode_rows_keep_the_plain_launch():
     assert pp._balance_rows(few, 10, 28, 4) == 1
     few.seq_lens_cpu = None
     assert pp._balance_rows(few, 10, 28, 4) == 0
+
+
+@pytest.mark.parametrize("case", list(CASES) + list(SPLIT_CASES))
+@pytest.mark.parametrize("hkv,group,d", [(4, 7, 128), (2, 7, 64), (1, 33, 128), (8, 1, 128)])
+def test_narrow_blocks_of_short_grids(case, hkv, group, d):
+    """Short grids on 32-column blocks (the default with at most one 64-column block per CU)
+    and on 64-column ones, both against the oracle, with scores rising past the first max."""
+    specs = {**CASES, **SPLIT_CASES}[case]
+    q, kv_cache, md = build_prefill_case(specs, hkv, group, d, seed=3)
+    scale_keys_by_position(kv_cache, md.block_tables, md.seq_lens_cpu, lambda p: 1.0 + 0.002 * p)
+    expected = _oracle(q, kv_cache, md, group)
+    for knob in (0, 2):
+        with tuned(_SHORT_GRID, knob):
+            assert_attn_close(_kernel()(q, kv_cache, md, d ** -0.5), expected)
