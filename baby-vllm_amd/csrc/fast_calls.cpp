@@ -93,6 +93,8 @@ at::Tensor new_empty(at::IntArrayRef sizes, const at::Tensor& like, at::ScalarTy
 }
 
 void* ptr(const at::Tensor& t) { return const_cast<void*>(t.const_data_ptr()); }
+// What a kernel writes: a lazily cloned tensor gets its own storage here, as with data_ptr() in Python.
+void* out_ptr(const at::Tensor& t) { return t.mutable_data_ptr(); }
 
 // (input, residual | None, weight, eps, device, stream)
 PyObject* fast_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -117,8 +119,8 @@ PyObject* fast_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (PyErr_Occurred()) return nullptr;
   at::Tensor out = new_empty(x->sizes(), *x, at::kBFloat16);
   return launch(out, [&] {
-    return g.norm(ptr(*x), hidden, res ? ptr(*res) : nullptr, res ? hidden : 0, ptr(*w), w32 ? 1 : 0, ptr(out), hidden,
-                  (int32_t)rows, (int32_t)hidden, eps, stream);
+    return g.norm(ptr(*x), hidden, res ? out_ptr(*res) : nullptr, res ? hidden : 0, ptr(*w), w32 ? 1 : 0, ptr(out),
+                  hidden, (int32_t)rows, (int32_t)hidden, eps, stream);
   });
   END_HANDLE_TH_ERRORS
 }
@@ -168,10 +170,12 @@ PyObject* fast_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int rc;
   {
     pybind11::gil_scoped_release no_gil;
-    rc = g.rope(ptr(*q), q->stride(0), q->stride(1), ptr(*k), k->stride(0), k->stride(1), ptr(*v), v->stride(0),
-                v->stride(1), ptr(*cos), cos->stride(0), ptr(*sin), sin->stride(0), ptr(*c), (void*)v_half(*c),
-                c->stride(2), c->stride(3), c->size(1) * c->size(2), slots->const_data_ptr<int64_t>(),
-                (int32_t)tokens, (int32_t)heads, (int32_t)hkv, (int32_t)d, stream);
+    // The written ones first: where q and k are views of one storage, no pointer is read before it is settled.
+    void *qp = out_ptr(*q), *kp = out_ptr(*k), *cp = out_ptr(*c);
+    rc = g.rope(qp, q->stride(0), q->stride(1), kp, k->stride(0), k->stride(1), ptr(*v), v->stride(0), v->stride(1),
+                ptr(*cos), cos->stride(0), ptr(*sin), sin->stride(0), cp, (char*)cp + c->stride(0) * 2, c->stride(2),
+                c->stride(3), c->size(1) * c->size(2), slots->const_data_ptr<int64_t>(), (int32_t)tokens,
+                (int32_t)heads, (int32_t)hkv, (int32_t)d, stream);
   }
   if (rc != 0) return none();
   Py_RETURN_TRUE;
@@ -374,7 +378,7 @@ PyObject* fast_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int64_t out_stride = cols;
   if (a[3] != Py_None) {
     const at::Tensor* o = plain(a[3], at::kBFloat16, dev);
-    if (!o || o->dim() != 2 || o->size(0) != m || o->size(1) != cols || o->stride(1) != 1 || (uintptr_t)ptr(*o) % 8)
+    if (!o || o->dim() != 2 || o->size(0) != m || o->size(1) != cols || o->stride(1) != 1 || (uintptr_t)out_ptr(*o) % 8)
       return none();
     if (m > 1) out_stride = o->stride(0);
     if (out_stride < cols || out_stride % 4) return none();
@@ -384,7 +388,7 @@ PyObject* fast_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   if (bytes > 0) ws = new_empty({bytes / 4}, *x, at::kFloat);
   return launch(out, [&] {
-    return g.linear(ptr(*x), x_stride, ptr(*w), bias ? ptr(*bias) : nullptr, ptr(out), out_stride, (int32_t)m,
+    return g.linear(ptr(*x), x_stride, ptr(*w), bias ? ptr(*bias) : nullptr, out_ptr(out), out_stride, (int32_t)m,
                     (int32_t)cols, (int32_t)k, gated ? 1 : 0, bytes > 0 ? ptr(ws) : nullptr, stream);
   });
   END_HANDLE_TH_ERRORS

@@ -118,3 +118,34 @@ def test_refused_calls_raise_as_before():
     pq, pc, md = build_prefill_case([(0, 5)], 4, 7, 128)
     with pytest.raises(AssertionError):
         paged_prefill_attention(pq[..., :96].contiguous(), pc, md, 0.1)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a ROCm GPU")
+@pytest.mark.parametrize("op", ["norm", "rope"])
+def test_writes_to_a_lazy_clone_leave_its_source_alone(op):
+    from babyvllm.kernels.layernorm import fused_add_rms_norm
+    from babyvllm.kernels.rope import fused_rope_and_cache
+
+    def rand(*shape):
+        return torch.randn(*shape, device="cuda").bfloat16()
+
+    if op == "norm":
+        sources = [rand(4, 96)]
+        x, w = rand(4, 96), rand(96)
+    else:
+        sources = [rand(3, 4, 64), rand(3, 2, 64), rand(2, 4, 16, 2, 64)]
+        v, cos, sin, slots = rand(3, 2, 64), rand(3, 64), rand(3, 64), torch.tensor([5, 20, 40], device="cuda")
+
+    def call(written):
+        if op == "norm":
+            fused_add_rms_norm(x, written[0], w, 1e-5)
+        else:
+            fused_rope_and_cache(written[0], written[1], v, cos, sin, written[2], slots)
+        return written
+
+    expected = call([s.clone() for s in sources])
+    before = [s.clone() for s in sources]
+    got = call([torch._lazy_clone(s) for s in sources])
+    for s, b, g, e in zip(sources, before, got, expected):
+        assert torch.equal(s, b) and torch.equal(g, e) and not torch.equal(g, b)
