@@ -4,9 +4,10 @@
 decode step's linear layers (and an MLP's fused gate/up projection with SiLU·mul)
 with ``bvllm_linear`` and return the result, or return ``None`` when the call is not
 one for that kernel; the caller then takes torch's own operations. The kernel takes
-plain bf16 tensors of at most 64 rows (256 where K is long and N short) on the current ROCm device, outside autograd
-and outside every mode that has to see torch operations (tracing, compilation,
-functorch transforms, forward-mode AD, dispatch and function modes, autocast).
+plain bf16 tensors of at most 64 rows (up to 256 where it is the faster one, the
+library's rule) on the current ROCm device, outside autograd and outside every mode
+that has to see torch operations (tracing, compilation, functorch transforms,
+forward-mode AD, dispatch and function modes, autocast).
 """
 
 from __future__ import annotations

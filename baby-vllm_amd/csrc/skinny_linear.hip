@@ -258,7 +258,7 @@ template <int RW, int KW, int D, bool GLU>
 hipError_t launch_waves(const LinearArgs& a, hipStream_t s) {
   if (a.m <= 16) return launch_tiles<1, RW, KW, D, GLU>(a, s);
   if (a.m <= 32) return launch_tiles<2, RW, KW, D, GLU>(a, s);
-  if constexpr (RW == 8 && !GLU) {  // beyond 64 tokens (linear_plan): blocks of at most 128, evenly
+  if constexpr (RW == 8) {  // beyond 64 tokens (linear_plan): blocks of at most 128, evenly
     const int per_block = (a.m + (a.m + 127) / 128 - 1) / ((a.m + 127) / 128);
     if (per_block > 96) return launch_tiles<8, RW, KW, D, GLU>(a, s);
     if (per_block > 64) return launch_tiles<6, RW, KW, D, GLU>(a, s);
@@ -280,6 +280,17 @@ hipError_t launch_waves(const LinearArgs& a, hipStream_t s) {
 //     1000 (past 32 tokens and 64 stages 8 x 1, twice the splits). From 64 stages on
 //     up to 256 tokens, in blocks of at most 128 (3584 x 18944: 96 tokens 43 / 95, 128:
 //     50 / 99);
+//   beyond 64 tokens the library computes as fast or faster from HBM but costs its
+//     caller about 20 us of host time a call, in steps too large for a captured graph
+//     (MLP 896 x 4864, eager, 65 / 96 / 128 / 192 / 256 tokens: 54 / 53 / 53 / 53 / 53 us on the
+//     library, 22 / 23 / 26 / 33 / 44 here). So: gated with short k (at most 12 stages), 8 row
+//     waves in blocks of 65 to 128 tokens (2·4864 x 896: 65 tokens 11.1 / 14.2, 128: 14.1 / 15.0,
+//     192: 17.4 / 16.5; 2·8960 x 1536: 128 tokens 23.9 / 27.3, 192: 31.2 / 29.4; k = 3584 is the
+//     library's: 91 / 77 at 128); 28 to 63 stages with at most 320 tiles, 8 x 1 with k cut by 3
+//     stages or more until tiles x splits reach 1536 (896 x 4864: 65 tokens 12.3 / 13.2, 128:
+//     15.3 / 13.0, 192: 17.8 / 13.8; 3584 x 3584: 96 tokens 18.3 / 19.8, 128: 20.7 / 22.5; 4608 x
+//     3584: 17.9 / 19.2 and 22.6 / 22.9). Beyond 128 tokens only while the products are few
+//     enough to end within the library's host time;
 //   the rest: 2 x 4 from 160 tiles, 1 x 4 below (each work-group then streams a
 //     few rows with 4 waves and no sum across work-groups). Past 32 tokens x
 //     outweighs the weights of so few rows per work-group: 3584 x 3584 stays with
@@ -290,13 +301,20 @@ LinearPlan linear_plan(int32_t m, int32_t n, int32_t k, bool gated) {
   if (m < 1 || m > 256 || n < 64 || n % 4 != 0 || k < kStageK || k % kStageK != 0) return p;
   if (rows * k * 2 >= (int64_t)kNoLoad) return p;
   const int tiles = (n + 15) / 16, stages = k / kStageK;
-  if (m > 64 && (gated || tiles >= 2048 || stages < 64)) return p;
+  if (m > 64 && (gated || stages < 64)) {
+    const bool few = m <= 128 || (double)m * rows * k <= (gated ? 2.4e9 : 1.2e9);
+    if (!few || (gated ? stages > 12 : stages < 28 || tiles > 320)) return p;
+  }
+  if (m > 64 && tiles >= 2048) return p;
   p.k_splits = 1;
   if (gated) {
-    p.rw = n >= 8192 ? 8 : 4;
+    p.rw = n >= 8192 || m > 64 ? 8 : 4;
   } else if (tiles >= 2048) {
     if (m > 32 && stages > 8) return p;
     p.rw = 8;
+  } else if (m > 64 && stages < 64) {
+    p.rw = 8;
+    p.k_splits = std::max(1, std::min(stages / 3, 1536 / tiles));
   } else if (stages >= 64 || (stages >= 32 && tiles < 160 && m > 16)) {
     const bool wide = m > 32 && stages >= 64;
     p.rw = wide ? 8 : 4;

@@ -301,9 +301,9 @@ BVLLM_API int bvllm_silu_mul(const void* gate_up, int64_t rows, int32_t d, void*
  * out_stride. gated = 1: w is [2n, k] (gate rows, then up rows, no bias) and
  * out = bf16(silu(gate) * up), silu and product in fp32.
  * bvllm_linear_workspace_bytes returns the scratch one call needs, or -1 for a
- * shape this kernel does not take (more than 64 tokens, or 256 where k is long and
- * n short, k not a multiple of 128, n not of 4, ...): the caller then uses a library GEMM. Pointers of x and w
- * are 16-byte aligned, x_stride a multiple of 8 elements, out 8-byte aligned with a
+ * shape this kernel does not take (more than 64 tokens, or up to 256 where a call to it
+ * ends sooner; k not a multiple of 128, n not of 4, ...): the caller then uses a
+ * library GEMM. Pointers of x and w are 16-byte aligned, x_stride a multiple of 8 elements, out 8-byte aligned with a
  * stride multiple of 4. The order of the sums depends on (n, k, gated) and on
  * whether m is at most 16, 32, 64 or more, on nothing else.
  */
