@@ -165,7 +165,7 @@ def fast():
     """The native host side of the wrappers' common calls (csrc/fast_calls.cpp), bound to ``lib()``.
 
     Its functions return None for a call that is not plainly valid; the wrapper then
-    runs its own checks and path.
+    runs its own checks and path. A return code of the library raises (``check``).
     """
     handle = lib()
     try:
@@ -173,7 +173,7 @@ def fast():
     except ImportError as e:
         raise KernelLibraryError("babyvllm._fast_calls not found or not loadable: build it with "
                                  "`python baby-vllm_amd/build_lib.py`") from e
-    _fast_calls.bind({n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value for n in _fast_calls.names()})
+    _fast_calls.bind({n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value for n in _fast_calls.names()}, check)
     return _fast_calls
 
 

@@ -6,7 +6,9 @@
 // Every function returns None for a call that is not plainly valid (other types,
 // layouts, devices, shapes, tensor subclasses, empty inputs): the Python wrapper then
 // runs its own checks and path, so what is accepted, what is refused and with which
-// error stays in one place. Nothing is kept between calls. The GIL is released
+// error stays in one place. A call is declined only before the library is called: a
+// code the library returns raises here, since the kernel may have run and the in-place
+// ones must not run twice. Nothing is kept between calls. The GIL is released
 // around allocation and launch, as ctypes and torch's own bindings do.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -62,7 +64,16 @@ const BindName kNames[] = {
     {"bvllm_linear", (void**)&g.linear},
 };
 
+// The wrappers' own error for a return code (babyvllm.kernels._lib.check), bound with the addresses.
+PyObject* g_check = nullptr;
+
 PyObject* none() { Py_RETURN_NONE; }
+
+PyObject* failed(int rc, const char* what) {
+  PyObject* r = PyObject_CallFunction(g_check, "is", rc, what);
+  Py_XDECREF(r);
+  return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_RuntimeError, "%s failed (code %d)", what, rc);
+}
 
 // A plain tensor (or parameter) on ROCm device `dev` of type `t`, or nullptr.
 const at::Tensor* plain(PyObject* o, at::ScalarType t, int64_t dev) {
@@ -77,14 +88,13 @@ const at::Tensor* plain(PyObject* o, at::ScalarType t, int64_t dev) {
 bool small(int64_t v) { return v >= 0 && v <= INT32_MAX; }
 
 template <typename F>
-PyObject* launch(const at::Tensor& out, F&& call) {
+PyObject* launch(const at::Tensor& out, const char* what, F&& call) {
   int rc;
   {
     pybind11::gil_scoped_release no_gil;
     rc = call();
   }
-  // A refused launch: the wrapper repeats it and raises with the library's text.
-  return rc == 0 ? THPVariable_Wrap(out) : none();
+  return rc == 0 ? THPVariable_Wrap(out) : failed(rc, what);
 }
 
 at::Tensor new_empty(at::IntArrayRef sizes, const at::Tensor& like, at::ScalarType t) {
@@ -118,7 +128,7 @@ PyObject* fast_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* stream = PyLong_AsVoidPtr(a[5]);
   if (PyErr_Occurred()) return nullptr;
   at::Tensor out = new_empty(x->sizes(), *x, at::kBFloat16);
-  return launch(out, [&] {
+  return launch(out, "bvllm_fused_add_rms_norm", [&] {
     return g.norm(ptr(*x), hidden, res ? out_ptr(*res) : nullptr, res ? hidden : 0, ptr(*w), w32 ? 1 : 0, ptr(out),
                   hidden, (int32_t)rows, (int32_t)hidden, eps, stream);
   });
@@ -138,7 +148,7 @@ PyObject* fast_silu(PyObject*, PyObject* const* a, Py_ssize_t n) {
   std::vector<int64_t> sizes = x->sizes().vec();
   sizes.back() = d;
   at::Tensor out = new_empty(sizes, *x, at::kBFloat16);
-  return launch(out, [&] { return g.silu(ptr(*x), rows, (int32_t)d, ptr(out), stream); });
+  return launch(out, "bvllm_silu_mul", [&] { return g.silu(ptr(*x), rows, (int32_t)d, ptr(out), stream); });
   END_HANDLE_TH_ERRORS
 }
 
@@ -177,7 +187,7 @@ PyObject* fast_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
                 c->stride(3), c->size(1) * c->size(2), slots->const_data_ptr<int64_t>(), (int32_t)tokens,
                 (int32_t)heads, (int32_t)hkv, (int32_t)d, stream);
   }
-  if (rc != 0) return none();
+  if (rc != 0) return failed(rc, "bvllm_rope_kv_append");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -251,7 +261,7 @@ PyObject* fast_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   at::Tensor out = new_empty({batch, heads, d}, *q, at::kBFloat16), ws;
   if (bytes > 0) ws = new_empty({bytes / 4}, *q, at::kFloat);
   void* wp = bytes > 0 ? ptr(ws) : nullptr;
-  return launch(out, [&] {
+  return launch(out, "bvllm_paged_decode", [&] {
     const int32_t* tables = bt->const_data_ptr<int32_t>();
     const int32_t* l = lens->const_data_ptr<int32_t>();
     if (balanced)
@@ -335,7 +345,7 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                     (int32_t)width, split, balance) /
                     4},
                    *q, at::kFloat);
-  return launch(out, [&] {
+  return launch(out, "bvllm_paged_prefill", [&] {
     const int32_t *tables = bt->const_data_ptr<int32_t>(), *ql = qsl->const_data_ptr<int32_t>();
     const int32_t *sl = seq->const_data_ptr<int32_t>(), *cl = ctx->const_data_ptr<int32_t>();
     if (split > 0 || balance)
@@ -364,7 +374,8 @@ PyObject* fast_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t m = x->size(0), k = x->size(1), rows = w->size(0), cols = gated ? rows / 2 : rows;
   if (m < 1 || w->size(1) != k || (gated && rows % 2) || !small(m) || !small(k) || !small(rows)) return none();
   const int64_t x_stride = m > 1 ? x->stride(0) : k;
-  if (x_stride < k || x_stride % 8 || ((uintptr_t)ptr(*x) | (uintptr_t)ptr(*w)) % 16) return none();
+  // (Rows further apart than the kernel's 32-bit offsets reach are the library's.)
+  if (x_stride < k || x_stride % 8 || m * x_stride * 2 >= ((int64_t)1 << 31) || ((uintptr_t)ptr(*x) | (uintptr_t)ptr(*w)) % 16) return none();
   const at::Tensor* bias = nullptr;
   if (a[2] != Py_None) {
     bias = plain(a[2], at::kBFloat16, dev);
@@ -387,21 +398,25 @@ PyObject* fast_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     out = new_empty({m, cols}, *x, at::kBFloat16);
   }
   if (bytes > 0) ws = new_empty({bytes / 4}, *x, at::kFloat);
-  return launch(out, [&] {
+  return launch(out, "bvllm_linear", [&] {
     return g.linear(ptr(*x), x_stride, ptr(*w), bias ? ptr(*bias) : nullptr, out_ptr(out), out_stride, (int32_t)m,
                     (int32_t)cols, (int32_t)k, gated ? 1 : 0, bytes > 0 ? ptr(ws) : nullptr, stream);
   });
   END_HANDLE_TH_ERRORS
 }
 
-// ({name: address}): binds the library's entry points.
-PyObject* bind(PyObject*, PyObject* names) {
+// ({name: address}, check): binds the library's entry points and what raises for a return code.
+PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 2 || !PyDict_Check(a[0]) || !PyCallable_Check(a[1]))
+    return PyErr_Format(PyExc_TypeError, "bind({name: address}, check)");
   for (const BindName& b : kNames) {
-    PyObject* v = PyDict_Check(names) ? PyDict_GetItemString(names, b.name) : nullptr;
+    PyObject* v = PyDict_GetItemString(a[0], b.name);
     if (v == nullptr) return PyErr_Format(PyExc_KeyError, "no address for %s", b.name);
     *b.slot = PyLong_AsVoidPtr(v);
     if (PyErr_Occurred()) return nullptr;
   }
+  Py_INCREF(a[1]);
+  Py_XSETREF(g_check, a[1]);
   Py_RETURN_NONE;
 }
 
@@ -424,7 +439,7 @@ PyObject* names(PyObject*, PyObject*) {
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))fast_##name, METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {
     FAST(norm), FAST(silu), FAST(rope), FAST(auto_plan), FAST(decode), FAST(prefill), FAST(linear),
-    {"bind", bind, METH_O, nullptr}, {"names", names, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr},
+    {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, nullptr}, {"names", names, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_fast_calls", nullptr, -1, kMethods};
 

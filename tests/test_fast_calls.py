@@ -149,3 +149,64 @@ def test_writes_to_a_lazy_clone_leave_its_source_alone(op):
     got = call([torch._lazy_clone(s) for s in sources])
     for s, b, g, e in zip(sources, before, got, expected):
         assert torch.equal(s, b) and torch.equal(g, e) and not torch.equal(g, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a ROCm GPU")
+@pytest.mark.parametrize("op", ["norm", "silu", "rope", "decode", "prefill", "linear"])
+def test_an_error_code_after_the_launch_raises_and_nothing_runs_twice(op, monkeypatch):
+    """A code left behind by an earlier failed call comes back from a launch that ran:
+    the call raises, the in-place kernels have run once and no other path is taken."""
+    import ctypes
+
+    from babyvllm.kernels import _lib
+    from babyvllm.kernels.activation import fused_silu_mul
+    from babyvllm.kernels.layernorm import fused_add_rms_norm
+    from babyvllm.kernels.paged_attn import paged_decode_attention
+    from babyvllm.kernels.paged_prefill import paged_prefill_attention
+    from babyvllm.kernels.rope import fused_rope_and_cache
+    from babyvllm.layers.linear import Linear
+
+    def rand(*shape):
+        return torch.randn(*shape, device="cuda").bfloat16()
+
+    x, w = rand(4, 256), rand(256)
+    if op == "norm":
+        name, state = "bvllm_fused_add_rms_norm", [rand(4, 256)]
+        call = lambda s: fused_add_rms_norm(x, s[0], w, 1e-5)
+    elif op == "silu":
+        name, state, call = "bvllm_silu_mul", [], lambda s: fused_silu_mul(x)
+    elif op == "rope":
+        v, cos, sin, slots = rand(3, 2, 64), rand(3, 64), rand(3, 64), torch.tensor([5, 20, 40], device="cuda")
+        name, state = "bvllm_rope_kv_append", [rand(3, 4, 64), rand(3, 2, 64), rand(2, 4, 16, 2, 64)]
+        call = lambda s: fused_rope_and_cache(s[0], s[1], v, cos, sin, s[2], slots)
+    elif op == "decode":
+        args = make_decode_inputs([20, 30])
+        name, state, call = "bvllm_paged_decode", [], lambda s: paged_decode_attention(*args, 0.1)
+    elif op == "prefill":
+        args = build_prefill_case([(0, 5)], 4, 7, 128)
+        name, state, call = "bvllm_paged_prefill", [], lambda s: paged_prefill_attention(*args, 0.1)
+    else:
+        lin = Linear(256, 64).to("cuda", torch.bfloat16)
+        name, state, call = "bvllm_linear", [], lambda s: lin(x)
+    with torch.no_grad():
+        once = [t.clone() for t in state]
+        call(once)
+        fast, handle = _lib.fast(), _lib.lib()
+        real, calls = getattr(handle, name), []
+
+        def runs_and_fails(*a):
+            calls.append(real(*a))
+            return 1
+
+        stub = ctypes.CFUNCTYPE(real.restype, *real.argtypes)(runs_and_fails)
+        addresses = {n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value for n in fast.names()}
+        try:
+            fast.bind({**addresses, name: ctypes.cast(stub, ctypes.c_void_p).value}, _lib.check)
+            with pytest.raises(_lib.KernelLibraryError, match=name):
+                call(state)
+        finally:
+            fast.bind(addresses, _lib.check)
+        assert calls == [0]
+        for got, want in zip(state, once):
+            assert torch.equal(got, want)
