@@ -93,11 +93,12 @@ SIGNATURES = {
         _i32, _i32, _i32,           # num_seqs, num_tokens, max_query_len
         _i32,                       # single_query_seqs (-1 = unknown)
         _i32, _i32, _i32, _i32,     # H, Hkv, D, block_size
-        _p, _i32, _i32, _p,         # workspace, split_tiles, balance_rows, stream
+        _p, _i32, _i32, _i32, _p,   # workspace, split_tiles, num_ranges, balance_rows, stream
     ]),
     "bvllm_prefill_split_tiles": (ctypes.c_int32, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i64, _i64]),
     "bvllm_prefill_balance_rows": (ctypes.c_int32, [_i32, _i32, _i64, _i64]),
-    "bvllm_prefill_workspace_bytes": (ctypes.c_int64, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "bvllm_prefill_ranges": (ctypes.c_int32, [_i32, _i32, _i64]),
+    "bvllm_prefill_workspace_bytes": (ctypes.c_int64, [_i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "bvllm_set_tuning": (ctypes.c_int, [_i32, _i32]),
     "bvllm_argmax_workspace_bytes": (ctypes.c_int64, [_i32, _i32]),
     "bvllm_greedy_argmax": (ctypes.c_int, [
@@ -126,7 +127,7 @@ SIGNATURES = {
     ]),
 }
 
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 
 # Knobs of bvllm_set_tuning (include/babyvllm_amd.h).

@@ -30,6 +30,22 @@ def _single_query_seqs(md, num_seqs):
 _SPLIT_MIN_PAGES = 32
 
 
+def _key_tiles(md, num_seqs, num_heads, num_kv_heads):
+    """(64-key tiles that the blocks of the sequences of several queries cover, tiles of the
+    longest of them) from the host lists, -1 for each if those are absent or of another length."""
+    qsl, seq = getattr(md, "query_start_loc_cpu", None), getattr(md, "seq_lens_cpu", None)
+    if qsl is None or seq is None or len(seq) != num_seqs or len(qsl) != num_seqs + 1:
+        return -1, -1
+    group, tiles, longest = num_heads // num_kv_heads, 0, 0
+    for i in range(num_seqs):
+        n = qsl[i + 1] - qsl[i]
+        if n > 1:
+            keys = (int(seq[i]) + 63) >> 6
+            tiles += ((int(n) * group + 127) >> 7) * keys
+            longest = max(longest, keys)
+    return tiles, longest
+
+
 def _split_tiles(md, num_seqs, num_tokens, single, num_heads, num_kv_heads, head_dim, width):
     """Key tiles per range of a split launch, 0 for the plain one.
 
@@ -38,16 +54,7 @@ def _split_tiles(md, num_seqs, num_tokens, single, num_heads, num_kv_heads, head
     """
     if width < _SPLIT_MIN_PAGES:
         return 0
-    tiles = longest = -1
-    qsl, seq = getattr(md, "query_start_loc_cpu", None), getattr(md, "seq_lens_cpu", None)
-    if single >= 0 and qsl is not None and seq is not None and len(seq) == num_seqs and len(qsl) == num_seqs + 1:
-        group, tiles, longest = num_heads // num_kv_heads, 0, 0
-        for i in range(num_seqs):
-            n = qsl[i + 1] - qsl[i]
-            if n > 1:
-                keys = (int(seq[i]) + 63) >> 6
-                tiles += ((int(n) * group + 127) >> 7) * keys
-                longest = max(longest, keys)
+    tiles, longest = _key_tiles(md, num_seqs, num_heads, num_kv_heads)
     return _lib.lib().bvllm_prefill_split_tiles(num_seqs, num_tokens, int(md.max_query_len), single, num_heads,
                                                 num_kv_heads, head_dim, width, tiles, longest)
 
@@ -120,10 +127,14 @@ def paged_prefill_attention(q, kv_cache, md, scale):
     h = _lib.lib()
     balance = _balance_rows(md, num_seqs, num_heads, num_kv_heads) if single > 0 else 0
     if split_tiles > 0 or balance:
-        nbytes = h.bvllm_prefill_workspace_bytes(num_seqs, num_tokens, num_heads, num_kv_heads, head_dim,
-                                                 bt.shape[1], split_tiles, balance)
+        ranges = 0
+        if split_tiles > 0:
+            longest = _key_tiles(md, num_seqs, num_heads, num_kv_heads)[1]
+            ranges = h.bvllm_prefill_ranges(bt.shape[1], split_tiles, longest)
+        nbytes = h.bvllm_prefill_workspace_bytes(num_seqs, num_tokens, num_heads, num_kv_heads, head_dim, ranges,
+                                                 balance)
         workspace = torch.empty(nbytes // 4, device=q.device, dtype=torch.float32)
-        rc = h.bvllm_paged_prefill_split(*args, workspace.data_ptr(), split_tiles, balance,
+        rc = h.bvllm_paged_prefill_split(*args, workspace.data_ptr(), split_tiles, ranges, balance,
                                          _lib.stream_handle(q.device))
     else:
         rc = h.bvllm_paged_prefill(*args, _lib.stream_handle(q.device))

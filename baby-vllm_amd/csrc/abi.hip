@@ -264,19 +264,17 @@ extern "C" int32_t bvllm_prefill_balance_rows(int32_t num_heads, int32_t num_kv_
   return prefill_balance_rows(num_heads, num_kv_heads, longest_pages, total_pages) ? 1 : 0;
 }
 
-static int64_t range_floats(int32_t num_tokens, int32_t num_heads, int32_t head_dim, int32_t max_blocks,
-                            int32_t split_tiles) {
-  return split_tiles < 1 ? 0
-                         : (int64_t)prefill_ranges(max_blocks, split_tiles) * num_tokens * num_heads * (head_dim + 2);
+extern "C" int32_t bvllm_prefill_ranges(int32_t max_blocks, int32_t split_tiles, int64_t longest_tiles) {
+  return max_blocks < 1 || split_tiles < 1 ? 0 : prefill_ranges(max_blocks, split_tiles, longest_tiles);
 }
 
 extern "C" int64_t bvllm_prefill_workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t num_heads,
-                                                 int32_t num_kv_heads, int32_t head_dim, int32_t max_blocks,
-                                                 int32_t split_tiles, int32_t balance_rows) {
-  if (num_seqs < 1 || num_tokens < 1 || !valid_heads(num_heads, num_kv_heads) || head_dim < 1 || max_blocks < 1)
+                                                 int32_t num_kv_heads, int32_t head_dim, int32_t num_ranges,
+                                                 int32_t balance_rows) {
+  if (num_seqs < 1 || num_tokens < 1 || !valid_heads(num_heads, num_kv_heads) || head_dim < 1 || num_ranges < 0)
     return 0;
   // (Each part a multiple of 16 bytes.)
-  const int64_t ranges = (range_floats(num_tokens, num_heads, head_dim, max_blocks, split_tiles) + 3) / 4 * 4;
+  const int64_t ranges = (prefill_range_floats(num_ranges, num_tokens, num_heads, head_dim) + 3) / 4 * 4;
   const int64_t rows =
       balance_rows ? decode_chunk_slots(num_seqs, num_heads, num_kv_heads) * num_heads * (head_dim + 1) : 0;
   return (ranges + rows) * (int64_t)sizeof(float);
@@ -294,7 +292,7 @@ extern "C" int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int6
                                    int32_t single_query_seqs,
                                    int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
                                    int32_t block_size, void* workspace, int32_t split_tiles,
-                                   int32_t balance_rows, void* stream) {
+                                   int32_t num_ranges, int32_t balance_rows, void* stream) {
   PrefillArgs a{};
   bool nothing;
   const int rc = pack_prefill(a, nothing, q, q_stride_t, q_stride_h, k_cache, v_cache, cache_stride_block, cache_stride_tok,
@@ -304,13 +302,15 @@ extern "C" int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int6
                               head_dim, block_size);
   if (rc != 0 || nothing) return rc;
   if (split_tiles < 0 || split_tiles > (1 << 20) || !workspace || !aligned16(workspace)) return kBad;
+  // Every range starts inside the table.
+  if (split_tiles > 0 && (num_ranges < 1 || num_ranges > prefill_ranges(max_blocks, split_tiles, -1))) return kBad;
   float* ws = reinterpret_cast<float*>(workspace);
   if (split_tiles > 0) {
     a.split_tiles = split_tiles;
-    a.num_ranges = prefill_ranges(max_blocks, split_tiles);
+    a.num_ranges = num_ranges;
     a.part_out = ws;
     a.part_ml = ws + (int64_t)a.num_ranges * num_tokens * num_heads * head_dim;
-    ws += (range_floats(num_tokens, num_heads, head_dim, max_blocks, split_tiles) + 3) / 4 * 4;
+    ws += (prefill_range_floats(num_ranges, num_tokens, num_heads, head_dim) + 3) / 4 * 4;
   }
   if (balance_rows) {
     a.row_part_out = ws;

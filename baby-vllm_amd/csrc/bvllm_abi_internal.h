@@ -69,8 +69,8 @@ struct PrefillArgs {
   // Sequences with exactly one query token: -1 = unknown, 0 = none. When not 0
   // those sequences run on the decode kernel and the prefill kernel skips them.
   int32_t single_query_seqs;
-  // Key ranges (split_tiles > 0): 64-key tiles per range, ranges of the longest
-  // sequence the table holds, and the ranges' fp32 partials.
+  // Key ranges (split_tiles > 0): 64-key tiles per range, the number of ranges (the last
+  // one runs to the row's end) and their fp32 partials.
   int32_t split_tiles, num_ranges;
   float* part_out;                         // [num_ranges, T, H, D], unnormalized
   float* part_ml;                          // [num_ranges, T, H, 2]: reference max (log2 units), row sum
@@ -202,8 +202,16 @@ hipError_t paged_prefill(const PrefillArgs& a, hipStream_t stream);
 // (key_tiles: 64-key tiles its 128-column blocks walk per KV head, longest_tiles: those of
 // its longest sequence of more than one query; < 0 if unknown).
 int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles, int64_t longest_tiles);
-inline int32_t prefill_ranges(int32_t max_blocks, int32_t split_tiles) {
-  return ((max_blocks + 3) / 4 + split_tiles - 1) / split_tiles;
+// Ranges of split_tiles tiles that hold keys: those of the longest sequence of more than one
+// query, or of the table where its length is unknown (longest_tiles < 0).
+inline int32_t prefill_ranges(int32_t max_blocks, int32_t split_tiles, int64_t longest_tiles) {
+  int64_t tiles = ((int64_t)max_blocks + 3) / 4;
+  if (longest_tiles >= 0 && longest_tiles < tiles) tiles = longest_tiles > 0 ? longest_tiles : 1;
+  return (int32_t)((tiles + split_tiles - 1) / split_tiles);
+}
+// fp32 values of the partials of num_ranges ranges.
+inline int64_t prefill_range_floats(int32_t num_ranges, int32_t num_tokens, int32_t num_heads, int32_t head_dim) {
+  return (int64_t)num_ranges * num_tokens * num_heads * (head_dim + 2);
 }
 // Compute units of the current device (cached per device).
 int device_cus();

@@ -35,6 +35,7 @@ struct Entry {
   decltype(&bvllm_paged_prefill) prefill = nullptr;
   decltype(&bvllm_prefill_split_tiles) split_tiles = nullptr;
   decltype(&bvllm_prefill_balance_rows) balance_rows = nullptr;
+  decltype(&bvllm_prefill_ranges) ranges = nullptr;
   decltype(&bvllm_prefill_workspace_bytes) prefill_bytes = nullptr;
   decltype(&bvllm_paged_prefill_split) prefill_split = nullptr;
   decltype(&bvllm_fused_add_rms_norm) norm = nullptr;
@@ -56,6 +57,7 @@ const BindName kNames[] = {
     {"bvllm_paged_prefill", (void**)&g.prefill},
     {"bvllm_prefill_split_tiles", (void**)&g.split_tiles},
     {"bvllm_prefill_balance_rows", (void**)&g.balance_rows},
+    {"bvllm_prefill_ranges", (void**)&g.ranges},
     {"bvllm_prefill_workspace_bytes", (void**)&g.prefill_bytes},
     {"bvllm_paged_prefill_split", (void**)&g.prefill_split},
     {"bvllm_fused_add_rms_norm", (void**)&g.norm},
@@ -339,10 +341,11 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                                    (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)width, tiles,
                                                    longest_tiles);
   const int32_t balance = pages > 0 ? g.balance_rows((int32_t)heads, (int32_t)hkv, longest, pages) : 0;
+  const int32_t ranges = split > 0 ? g.ranges((int32_t)width, split, longest_tiles) : 0;
   at::Tensor out = new_empty({tokens, heads, d}, *q, at::kBFloat16), ws;
   if (split > 0 || balance)
-    ws = new_empty({g.prefill_bytes((int32_t)seqs, (int32_t)tokens, (int32_t)heads, (int32_t)hkv, (int32_t)d,
-                                    (int32_t)width, split, balance) /
+    ws = new_empty({g.prefill_bytes((int32_t)seqs, (int32_t)tokens, (int32_t)heads, (int32_t)hkv, (int32_t)d, ranges,
+                                    balance) /
                     4},
                    *q, at::kFloat);
   return launch(out, "bvllm_paged_prefill", [&] {
@@ -353,7 +356,7 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
                              c->stride(3), (int32_t)c->size(1), tables, bt->stride(0), (int32_t)width, ql, sl, cl,
                              scale, ptr(out), out.stride(0), out.stride(1), (int32_t)seqs, (int32_t)tokens,
                              (int32_t)max_q, (int32_t)single, (int32_t)heads, (int32_t)hkv, (int32_t)d,
-                             (int32_t)c->size(2), ptr(ws), split, balance, stream);
+                             (int32_t)c->size(2), ptr(ws), split, ranges, balance, stream);
     return g.prefill(ptr(*q), q->stride(0), q->stride(1), ptr(*c), v_half(*c), c->stride(1), c->stride(2),
                      c->stride(3), (int32_t)c->size(1), tables, bt->stride(0), (int32_t)width, ql, sl, cl, scale,
                      ptr(out), out.stride(0), out.stride(1), (int32_t)seqs, (int32_t)tokens, (int32_t)max_q,

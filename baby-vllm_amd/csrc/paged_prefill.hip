@@ -161,8 +161,7 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
   const int range = SPL ? (int)blockIdx.x / grid_wgs : 0;
   const int id = SPL ? (int)blockIdx.x - range * grid_wgs : (int)blockIdx.x;
   const int tile0 = SPL ? range * a.split_tiles : 0;  // first key tile of the range
-  const int max_blocks = SPL ? a.max_blocks - 4 * tile0 : a.max_blocks;
-  if (SPL && max_blocks <= 0) return;
+  const int max_blocks = SPL ? a.max_blocks - 4 * tile0 : a.max_blocks;  // > 0: ranges start inside the table
   // The arguments that address the metadata and table loads below, read
   // with the mapping's own: otherwise their wait splits those loads' round trip.
   asm volatile("" ::"s"(a.block_tables), "s"(a.bt_stride), "s"(a.max_blocks), "s"(a.query_start_loc),
@@ -286,7 +285,9 @@ __global__ __launch_bounds__(NW * 64, 2) void paged_prefill_kernel(PrefillArgs a
   // (MB: the host checked that no sequence has more than two tiles' pages;
   // the clamp keeps an inconsistent seq_lens inside the staged tiles.)
   const int hi_all = min(seq_len, ctx + q_last + 1);
-  const int hi = min(hi_all, MB ? 2 * KT : SPL ? KT * a.split_tiles : 0x7fffffff);
+  // (SPL: the last range takes the rest of the row, so a row longer than the host's
+  // lists say is slower but no key of it is left out and no partial is out of range.)
+  const int hi = min(hi_all, MB ? 2 * KT : SPL && range < bpw - 1 ? KT * a.split_tiles : 0x7fffffff);
   if (SPL && range > 0 && hi <= 0) return;
   const int n_tiles = hi > 0 ? (hi + KT - 1) / KT : 0;
 
@@ -860,7 +861,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, int b
   const int q_last = (min(q_len * G, (blk + 1) * CB) - 1) / G;
   const int hi = min(seq_len, ctx + q_last + 1);
   const int keys = 64 * a.split_tiles;
-  if (hi <= keys) return;  // a single range wrote the output itself
+  if (hi <= keys || a.num_ranges == 1) return;  // a single range wrote the output itself
   const int nr = min((hi + keys - 1) / keys, a.num_ranges);
   const int64_t th = (int64_t)t * a.num_heads + head, step = (int64_t)a.num_tokens * a.num_heads;
   const float* ml = a.part_ml + th * 2;
@@ -1035,6 +1036,11 @@ static hipError_t launch_prefill_split(const PrefillArgs& a, hipStream_t stream)
 // 60 us at 13 tiles per range, 46 at 15, 51 at 20, 75 at 48; 92 unsplit). 0.86 of the
 // slots, since blocks fall unevenly on the XCDs; one work-group per CU beside decode
 // rows (100 new tokens behind 6000 + 20 rows: 44 us at 7 tiles, 34 at 15; 83 unsplit).
+// The partials hold every token of the step for every range: at most kMaxRangeBytes (the
+// choices above stay under 50 MB over steps of 2 to 4096 new tokens behind up to 16 thousand;
+// a few tokens on a long prefix beside fresh prompts would take ten times that).
+constexpr int64_t kMaxRangeBytes = 64ll << 20;
+
 int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles, int64_t longest_tiles) {
   const PrefillGrid p = plan_prefill(a, 4 * 2 * 16);
   const double cus = device_cus(), hkv = a.num_kv_heads;
@@ -1045,11 +1051,13 @@ int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles, int64_t lon
   const bool narrow = 2.0 * blocks <= cus && p.dec_wgs == 0;
   const double unsplit = narrow ? 5.5 + 0.6 * longest : 7.0 + (2.0 * blocks <= cus ? 0.79 : 1.1) * longest;
   double best = 0.9 * unsplit;
+  const int64_t max_ranges = kMaxRangeBytes / (prefill_range_floats(1, a.num_tokens, a.num_heads, a.head_dim) * 4);
+  if (max_ranges < 2) return 0;
   int32_t tiles = 0;
   for (int per_cu = 1; per_cu <= (p.dec_wgs > 0 ? 1 : 2); ++per_cu) {
     const double slots = (per_cu == 1 ? 0.98 : 1.72) * cus - (double)p.dec_wgs - blocks / 2;
     if (slots <= 0) continue;
-    const double c = std::max(8.0, std::ceil(steps / slots));
+    const double c = std::max({8.0, std::ceil(steps / slots), std::ceil(longest / (double)max_ranges)});
     if (c >= longest) continue;
     const double ranges = steps / (blocks * c) + 0.5;
     const double bytes = (double)a.num_tokens * a.num_heads * (a.head_dim + 2) * 4 * ranges;

@@ -40,7 +40,7 @@ extern "C" {
 #endif
 
 /* ABI version of this header; bumped on any signature change. */
-#define BVLLM_ABI_VERSION 7
+#define BVLLM_ABI_VERSION 8
 
 #if defined(__GNUC__)
 #define BVLLM_API __attribute__((visibility("default")))
@@ -214,20 +214,26 @@ BVLLM_API int bvllm_paged_prefill(const void* q, int64_t q_stride_t, int64_t q_s
  * where the plain launch is the better one; key_tiles is the number of 64-key tiles the
  * batch's blocks of 128 (query, head) pairs cover, per KV head, summed over its
  * sequences of more than one query token (ceil(G * q_len / 128) * ceil(seq_len / 64)),
- * longest_tiles the tiles of the longest of them (ceil(seq_len / 64)), each -1 if unknown. bvllm_prefill_balance_rows returns whether cutting pays, from the
- * pages of the longest single-query row and of all of them. Both steer the choice only,
- * never what is computed. workspace holds bvllm_prefill_workspace_bytes() bytes.
- * Results agree with bvllm_paged_prefill within the rounding of fp32 sums in another
- * order; a sequence's keys end at its table's last page.
+ * longest_tiles the tiles of the longest of them (ceil(seq_len / 64)), each -1 if
+ * unknown. bvllm_prefill_ranges returns the number of ranges those sequences have
+ * (of the table's width if longest_tiles is -1); the last range of a launch runs to the
+ * row's end, so any num_ranges from 1 to that of the width computes every key.
+ * bvllm_prefill_balance_rows returns whether cutting pays, from the pages of the longest
+ * single-query row and of all of them. All three steer the choice only, never what is
+ * computed. workspace holds bvllm_prefill_workspace_bytes() bytes (num_ranges 0 without
+ * key ranges; partials of the ranges that bvllm_prefill_split_tiles chooses are at most
+ * 64 MiB). Results agree with bvllm_paged_prefill within the rounding of fp32 sums in
+ * another order.
  */
 BVLLM_API int32_t bvllm_prefill_split_tiles(int32_t num_seqs, int32_t num_tokens, int32_t max_query_len,
                         int32_t single_query_seqs, int32_t num_heads, int32_t num_kv_heads,
                         int32_t head_dim, int32_t max_blocks, int64_t key_tiles, int64_t longest_tiles);
 BVLLM_API int32_t bvllm_prefill_balance_rows(int32_t num_heads, int32_t num_kv_heads, int64_t longest_pages,
                         int64_t total_pages);
+BVLLM_API int32_t bvllm_prefill_ranges(int32_t max_blocks, int32_t split_tiles, int64_t longest_tiles);
 BVLLM_API int64_t bvllm_prefill_workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t num_heads,
-                        int32_t num_kv_heads, int32_t head_dim, int32_t max_blocks,
-                        int32_t split_tiles, int32_t balance_rows);
+                        int32_t num_kv_heads, int32_t head_dim, int32_t num_ranges,
+                        int32_t balance_rows);
 BVLLM_API int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                         const void* k_cache, const void* v_cache,
                         int64_t cache_stride_block, int64_t cache_stride_tok, int64_t cache_stride_head,
@@ -240,7 +246,7 @@ BVLLM_API int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int64
                         int32_t single_query_seqs,
                         int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
                         int32_t block_size, void* workspace, int32_t split_tiles,
-                        int32_t balance_rows, void* stream);
+                        int32_t num_ranges, int32_t balance_rows, void* stream);
 
 /*
  * Tuning switch for experiments and tests (no counterpart in the reference):

@@ -73,6 +73,37 @@ def test_workspace_bytes_formula():
     assert h.bvllm_decode_workspace_bytes(1, 28, 4, 128, 512, 6) == 28 * 512 * 129 * 4
 
 
+def test_key_range_scratch_follows_the_sequences_not_the_table():
+    h = _lib().lib()
+
+    def scratch(specs, width, decode_rows=0):
+        """Bytes of the partials that a step of (context, new) sequences and decode rows takes."""
+        tokens, longest = sum(n for _, n in specs) + decode_rows, max(-(-(c + n) // 64) for c, n in specs)
+        tiles = sum(-(-7 * n // 128) * -(-(c + n) // 64) for c, n in specs)
+        seqs = len(specs) + decode_rows
+        split = h.bvllm_prefill_split_tiles(seqs, tokens, max(n for _, n in specs), decode_rows, 28, 4, 128, width,
+                                            tiles, longest)
+        ranges = h.bvllm_prefill_ranges(width, split, longest) if split else 0
+        return split, ranges, h.bvllm_prefill_workspace_bytes(seqs, tokens, 28, 4, 128, ranges, 0)
+
+    # 200 new tokens behind 4000: the same ranges for a table of any width.
+    split, ranges, nbytes = scratch([(4000, 200)], 263)
+    assert split > 0 and ranges == -(-66 // split) and nbytes == ranges * 200 * 28 * 130 * 4
+    for width in (264, 2048, 8192):
+        assert scratch([(4000, 200)], width) == (split, ranges, nbytes)
+    # A short turn and fresh prompts beside decode rows of up to 31 thousand tokens.
+    assert scratch([(1331, 30)] + [(0, 146)] * 4, 1938, 9)[2] <= 3 * 623 * 28 * 130 * 4
+    # A few tokens on a long prefix beside fresh prompts: bounded, with longer ranges or none.
+    for prompts in ([(0, 700)] * 2, [(0, 300)], [(0, 1000)], []):
+        split, ranges, nbytes = scratch([(28000, 5)] + prompts, 1751)
+        assert nbytes <= 64 << 20 and (ranges == 0 or ranges >= 2)
+    # Without lengths the table stands in for them, within the same bound.
+    for width in (64, 500, 2048, 1 << 20):
+        split = h.bvllm_prefill_split_tiles(4, 400, 200, -1, 28, 4, 128, width, -1, -1)
+        if split:
+            assert h.bvllm_prefill_workspace_bytes(4, 400, 28, 4, 128, h.bvllm_prefill_ranges(width, split, -1), 0) <= 64 << 20
+
+
 def test_workspace_bytes_ignore_the_split_mode_knob():
     # The size (and the place of part_lse inside it) must not follow knob 0:
     # a knob changed between the size query and the launch would otherwise make

@@ -458,6 +458,46 @@ def test_key_ranges_chosen_for_short_turns_behind_long_prefixes():
     assert pp._split_tiles(*args, 8) == 0
 
 
+def test_key_ranges_of_a_table_wider_than_its_rows():
+    """The ranges and their scratch are those of the sequences: a table 32 times as wide (or a
+    far longer decode row beside them) changes neither the bits nor the memory taken."""
+    import babyvllm.kernels.paged_prefill as pp
+
+    specs = [(4000, 200), (1000, 40)]
+    q, kv_cache, md = build_prefill_case(specs, 4, 7, 128)
+    assert pp._split_tiles(md, 2, 240, 0, 28, 4, 128, md.block_tables.shape[1]) > 0
+
+    def call():
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_stats()["requested_bytes.all.current"]
+        out = _kernel()(q, kv_cache, md, 128 ** -0.5)
+        return out, torch.cuda.memory_stats()["requested_bytes.all.peak"] - before
+
+    tight, tight_bytes = call()
+    assert_attn_close(tight, _oracle(q, kv_cache, md, 7))
+    table = torch.zeros(2, 32 * md.block_tables.shape[1], dtype=torch.int32, device="cuda")
+    table[:, :md.block_tables.shape[1]] = md.block_tables
+    md.block_tables = table
+    wide, wide_bytes = call()
+    assert torch.equal(tight, wide)
+    assert wide_bytes == tight_bytes
+
+
+@pytest.mark.parametrize("path", ["native", "python"])
+def test_key_ranges_cover_rows_longer_than_the_host_lists_say(path, monkeypatch):
+    """The last range runs to the row's end, so the host lists steer the choice only."""
+    specs = [(6000, 40), (3000, 70), (200, 9)]
+    q, kv_cache, md = build_prefill_case(specs, 4, 7, 128)
+    scale_keys_by_position(kv_cache, md.block_tables, md.seq_lens_cpu, lambda p: 1.0 + 0.001 * p)
+    expected = _oracle(q, kv_cache, md, 7)
+    if path == "python":
+        python_path(monkeypatch)
+    for listed in ([6040, 3070, 209], [2500, 3070, 209], [700, 600, 209], [6040, 100000, 209]):
+        md.seq_lens_cpu = listed
+        assert_attn_close(_kernel()(q, kv_cache, md, 128 ** -0.5), expected)
+
+
 @pytest.mark.parametrize("tiles", [0, 4])
 @pytest.mark.parametrize("hkv,group,d", [(4, 7, 128), (2, 7, 64), (1, 33, 128)])
 def test_uneven_decode_rows_of_a_mixed_step(tiles, hkv, group, d, monkeypatch):
