@@ -168,12 +168,17 @@ def fast():
     Its functions return None for a call that is not plainly valid; the wrapper then
     runs its own checks and path. A return code of the library raises (``check``).
     """
+    import torch  # noqa: F401  (its libraries, which the module links to)
+
     handle = lib()
     try:
         from babyvllm import _fast_calls
     except ImportError as e:
         raise KernelLibraryError("babyvllm._fast_calls not found or not loadable: build it with "
                                  "`python baby-vllm_amd/build_lib.py`") from e
+    got = getattr(_fast_calls, "ABI_VERSION", None)
+    if got != ABI_VERSION:  # it would call the library with another version's arguments
+        raise KernelLibraryError(f"{_fast_calls.__file__} was built for ABI {got}, expected {ABI_VERSION}: rebuild it")
     _fast_calls.bind({n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value for n in _fast_calls.names()}, check)
     return _fast_calls
 

@@ -448,4 +448,9 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_fast_calls", nullptr, -1, kMetho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__fast_calls() { return PyModule_Create(&kModule); }
+// ABI_VERSION: that of the header the calls above were compiled against.
+PyMODINIT_FUNC PyInit__fast_calls() {
+  PyObject* m = PyModule_Create(&kModule);
+  if (m != nullptr && PyModule_AddIntConstant(m, "ABI_VERSION", BVLLM_ABI_VERSION) != 0) Py_CLEAR(m);
+  return m;
+}

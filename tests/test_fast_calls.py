@@ -38,6 +38,35 @@ def test_cpu_tensors_and_wrong_argument_counts_are_declined():
     assert f.norm() is None and f.decode(x) is None and f.prefill() is None and f.rope(x, x) is None
 
 
+@pytest.mark.parametrize("version", [None, 1])
+def test_a_module_of_another_abi_is_refused(version, monkeypatch):
+    import types
+
+    import babyvllm
+    from babyvllm.kernels import _lib
+
+    assert _fast().ABI_VERSION == _lib.ABI_VERSION
+    bound = []
+    stale = types.SimpleNamespace(__file__="stale.so", names=_fast().names, bind=lambda *a: bound.append(a))
+    if version is not None:
+        stale.ABI_VERSION = version
+    monkeypatch.setattr(babyvllm, "_fast_calls", stale)
+    with pytest.raises(_lib.KernelLibraryError, match="rebuild"):
+        _lib.fast.__wrapped__()
+    assert not bound
+
+
+def test_the_module_loads_in_a_process_that_has_not_imported_torch():
+    import subprocess
+    import sys
+    from pathlib import Path
+
+    pkg = Path(__file__).resolve().parents[1] / "baby-vllm_amd"
+    code = f"import sys; sys.path.insert(0, {str(pkg)!r}); from babyvllm.kernels import _lib; _lib.fast()"
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stderr
+
+
 def _calls():
     from babyvllm.kernels.activation import fused_silu_mul
     from babyvllm.kernels.layernorm import fused_add_rms_norm
