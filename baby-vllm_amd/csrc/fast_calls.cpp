@@ -194,7 +194,13 @@ PyObject* fast_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+int64_t cdiv(int64_t a, int64_t b) { return a / b + (a % b > 0); }  // a >= 0: no sum to overflow
+// An int of any size: past 64 bits the nearest one, which means the same for a length.
+int64_t clamped(PyObject* o) {
+  int overflow = 0;
+  const long long v = PyLong_AsLongLongAndOverflow(o, &overflow);
+  return overflow > 0 ? INT64_MAX : overflow < 0 ? INT64_MIN : v;
+}
 int64_t pow2_at_least(int64_t n) {
   int64_t p = 1;
   while (p < n) p <<= 1;
@@ -219,7 +225,7 @@ Plan auto_plan(int64_t batch, int64_t hkv, int64_t page, int64_t width, int64_t 
 PyObject* fast_auto_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 7) return none();
   int64_t v[7];
-  for (int i = 0; i < 7; ++i) v[i] = PyLong_AsLongLong(a[i]);
+  for (int i = 0; i < 7; ++i) v[i] = clamped(a[i]);
   if (PyErr_Occurred()) return nullptr;
   const Plan p = auto_plan(v[0], v[1], v[2], v[3], v[4], v[5], v[6]);
   return Py_BuildValue("LL", (long long)p.splits, (long long)p.pages);
@@ -243,7 +249,7 @@ PyObject* fast_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int64_t max_seq_len = -1;
   if (a[5] != Py_None) {
     if (!PyLong_CheckExact(a[5])) return none();
-    max_seq_len = std::max<int64_t>(PyLong_AsLongLong(a[5]), 0);
+    max_seq_len = std::max<int64_t>(clamped(a[5]), 0);
   }
   if (!PyFloat_CheckExact(a[4])) return none();
   const float scale = (float)PyFloat_AsDouble(a[4]);
@@ -310,14 +316,15 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   for (int64_t i = 0; i <= seqs; ++i) {
     PyObject* o = PyList_GET_ITEM(a[6], i);
     if (!PyLong_CheckExact(o)) return none();
-    const int64_t v = PyLong_AsLongLong(o);
+    const int64_t v = clamped(o);
+    if (!small(v)) return none();
     if (i > 0) {
       const int64_t m = v - prev;
       single += m == 1;
       if (lens_known) {
         PyObject* l = PyList_GET_ITEM(a[7], i - 1);
         if (!PyLong_CheckExact(l)) return none();
-        const int64_t len = PyLong_AsLongLong(l);
+        const int64_t len = clamped(l);
         if (!small(m) || !small(len)) return none();
         if (m == 1) {
           longest = std::max(longest, cdiv(len, 16));
@@ -331,7 +338,7 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     prev = v;
   }
   if (!PyLong_CheckExact(a[8]) || !PyFloat_CheckExact(a[9])) return none();
-  const int64_t max_q = PyLong_AsLongLong(a[8]);
+  const int64_t max_q = clamped(a[8]);
   const float scale = (float)PyFloat_AsDouble(a[9]);
   void* stream = PyLong_AsVoidPtr(a[12]);
   if (PyErr_Occurred()) return nullptr;

@@ -29,6 +29,18 @@ def test_auto_plan_equals_decode_split_plan(monkeypatch):
         assert got == ds.decode_split_plan(batch, hkv, 16, width, max_len, cus), (batch, hkv, width, max_len, cus)
 
 
+def test_auto_plan_at_the_ends_of_the_integers(monkeypatch):
+    import sys
+
+    from babyvllm.kernels import decode_split as ds
+
+    monkeypatch.delenv(ds.DECODE_PARTITION_ENV, raising=False)
+    for batch, width in ((1, 2048), (8, 130), (64, 300), (3, 1)):
+        for max_len in (sys.maxsize - 15, sys.maxsize - 14, sys.maxsize, 2 ** 63, 2 ** 80):
+            want = ds.decode_split_plan(batch, 4, 16, width, max_len, 256)
+            assert _fast().auto_plan(batch, 4, 16, width, max_len, 256, ds.MIN_PARTITION_BLOCKS) == want, (batch, max_len)
+
+
 def test_cpu_tensors_and_wrong_argument_counts_are_declined():
     x = torch.zeros(2, 8, dtype=torch.bfloat16)
     f = _fast()
@@ -116,6 +128,18 @@ def test_calls_equal_the_python_path(monkeypatch):
             if s is not None:
                 assert s.shape == t.shape and s.dtype == t.dtype and s.stride() == t.stride(), name
                 assert torch.equal(s, t), name
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a ROCm GPU")
+@pytest.mark.parametrize("max_len", [-5, 2 ** 63 - 1, 2 ** 63, 2 ** 70, -2 ** 70])
+def test_decode_takes_a_bucket_of_any_size_as_the_python_path_does(max_len, monkeypatch):
+    from babyvllm.kernels.paged_attn import paged_decode_attention
+
+    args = make_decode_inputs([900, 40, 0])
+    native = paged_decode_attention(*args, 0.1, max_seq_len=max_len)
+    python_path(monkeypatch)
+    assert torch.equal(native, paged_decode_attention(*args, 0.1, max_seq_len=max_len))
 
 
 @pytest.mark.gpu
