@@ -154,10 +154,13 @@ PyObject* fast_silu(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// [2, NB, 16, Hkv, D] whose halves share a layout with a unit last stride.
+// [2, NB, page, Hkv, D] whose halves share a layout with a unit last stride.
 bool plain_cache(const at::Tensor* c) {
   return c && c->dim() == 5 && c->size(0) == 2 && c->stride(4) == 1 && small(c->size(1)) && small(c->size(3));
 }
+// The attention kernels' page size; others (0 among them, which the plan would divide by)
+// are for the wrapper to refuse.
+constexpr int64_t kPage = 16;
 const char* v_half(const at::Tensor& c) { return (const char*)c.const_data_ptr() + c.stride(0) * 2; }
 
 bool rows_of(const at::Tensor* t, int64_t dim) { return t && t->dim() == dim && t->stride(dim - 1) == 1; }
@@ -227,6 +230,7 @@ PyObject* fast_auto_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int64_t v[7];
   for (int i = 0; i < 7; ++i) v[i] = clamped(a[i]);
   if (PyErr_Occurred()) return nullptr;
+  if (v[2] < 1) return none();
   const Plan p = auto_plan(v[0], v[1], v[2], v[3], v[4], v[5], v[6]);
   return Py_BuildValue("LL", (long long)p.splits, (long long)p.pages);
 }
@@ -245,7 +249,7 @@ PyObject* fast_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t batch = q->size(0), heads = q->size(1), d = q->size(2), hkv = c->size(3), width = bt->size(1);
   if (batch == 0 || c->size(4) != d || bt->size(0) < batch) return none();
   if (!lens || lens->dim() != 1 || lens->size(0) < batch || !lens->is_contiguous()) return none();
-  if (!small(batch) || !small(heads) || !small(width) || !small(c->size(2))) return none();
+  if (!small(batch) || !small(heads) || !small(width) || c->size(2) != kPage) return none();
   int64_t max_seq_len = -1;
   if (a[5] != Py_None) {
     if (!PyLong_CheckExact(a[5])) return none();
@@ -304,7 +308,7 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t width = bt->size(1);
   if (tokens == 0 || seqs == 0 || c->size(4) != d || hkv == 0 || heads % hkv != 0 || (d & (d - 1)) != 0) return none();
   if (qsl->size(0) != seqs + 1 || ctx->size(0) != seqs || bt->size(0) < seqs) return none();
-  if (!small(tokens) || !small(heads) || !small(seqs) || !small(width) || !small(c->size(2))) return none();
+  if (!small(tokens) || !small(heads) || !small(seqs) || !small(width) || c->size(2) != kPage) return none();
   // Host lists: single-query sequences and their pages, and the key tiles of the
   // others' blocks.
   if (!PyList_CheckExact(a[6]) || PyList_GET_SIZE(a[6]) != seqs + 1) return none();

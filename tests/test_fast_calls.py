@@ -41,6 +41,18 @@ def test_auto_plan_at_the_ends_of_the_integers(monkeypatch):
             assert _fast().auto_plan(batch, 4, 16, width, max_len, 256, ds.MIN_PARTITION_BLOCKS) == want, (batch, max_len)
 
 
+def test_auto_plan_declines_a_page_size_it_cannot_divide_by():
+    import subprocess
+    import sys
+    from pathlib import Path
+
+    pkg = Path(__file__).resolve().parents[1] / "baby-vllm_amd"
+    code = (f"import sys; sys.path.insert(0, {str(pkg)!r}); from babyvllm.kernels import _lib\n"
+            "assert _lib.fast().auto_plan(1, 4, 0, 8, 100, 256, 4) is None")
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, (out.returncode, out.stderr)
+
+
 def test_cpu_tensors_and_wrong_argument_counts_are_declined():
     x = torch.zeros(2, 8, dtype=torch.bfloat16)
     f = _fast()
@@ -171,6 +183,12 @@ def test_refused_calls_raise_as_before():
     pq, pc, md = build_prefill_case([(0, 5)], 4, 7, 128)
     with pytest.raises(AssertionError):
         paged_prefill_attention(pq[..., :96].contiguous(), pc, md, 0.1)
+    for page, buckets in ((0, (None, 40)), (8, (None, 40))):  # pages of another size than 16 tokens
+        for bucket in buckets:
+            with pytest.raises((KernelLibraryError, ZeroDivisionError)):
+                paged_decode_attention(q, cache[:, :, :page].contiguous(), bt, lens, 0.1, max_seq_len=bucket)
+        with pytest.raises(KernelLibraryError):
+            paged_prefill_attention(pq, pc[:, :, :page].contiguous(), md, 0.1)
 
 
 @pytest.mark.gpu
