@@ -22,13 +22,14 @@ MAX_ROWS = 256
 
 def torch_must_see(*tensors) -> bool:
     """Whether something besides the values wants to see this operation."""
+    if torch.compiler.is_compiling():  # first: the questions below are none the compiler can trace
+        return True
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
         return True
     c = torch._C
     return (c._len_torch_dispatch_stack() > 0 or c._len_torch_function_stack() > 0
             or c._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0
-            or c._get_tracing_state() is not None or torch.compiler.is_compiling()
-            or torch.is_autocast_enabled("cuda"))
+            or c._get_tracing_state() is not None or torch.is_autocast_enabled("cuda"))
 
 
 def skinny_linear(x, weight, bias=None, out=None):
