@@ -407,6 +407,9 @@ PyObject* fast_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return none();
     if (m > 1) out_stride = o->stride(0);
     if (out_stride < cols || out_stride % 4) return none();
+    // An in-place write to autograd, as torch's out= is: what was saved of the old values is
+    // stale, and an inference tensor is refused outside inference mode.
+    o->unsafeGetTensorImpl()->bump_version();
     out = *o;
   } else {
     out = new_empty({m, cols}, *x, at::kBFloat16);

@@ -73,6 +73,32 @@ def test_same_bits_for_any_batch_of_a_token_tile_count_and_in_a_graph():
             assert torch.equal(out, skinny_linear(x, w))
 
 
+def test_out_is_an_in_place_write_to_autograd():
+    """As torch.mm(..., out=): the version moves, a backward through overwritten values and a
+    write to an inference tensor outside inference mode raise."""
+    from babyvllm.kernels.linear import skinny_linear
+
+    x = torch.randn(4, 256, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(64, 256, device="cuda", dtype=torch.bfloat16)
+    out = torch.randn(4, 64, device="cuda", dtype=torch.bfloat16)
+    scale = torch.ones(64, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    loss = (out * scale).sum()
+    version = out._version
+    with torch.no_grad():
+        assert skinny_linear(x, w, None, out) is not None
+    assert out._version == version + 1
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        loss.backward()
+    with torch.inference_mode():
+        inference = torch.zeros(4, 64, device="cuda", dtype=torch.bfloat16)
+        assert skinny_linear(x, w, None, inference) is not None
+        kept = inference.clone()
+        assert skinny_linear(x, w, None, out) is not None
+    with torch.no_grad(), pytest.raises(RuntimeError, match="inference tensor"):
+        skinny_linear(x + 1, w, None, inference)
+    assert torch.equal(inference, kept)
+
+
 def test_non_finite_weights_and_inputs_stay_in_their_row_and_column():
     from babyvllm.kernels.linear import skinny_linear
 
