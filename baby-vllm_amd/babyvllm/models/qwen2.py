@@ -13,6 +13,8 @@ SiLU·mul in its epilogue; the others on hipBLASLt through torch, with the HIP S
 
 from __future__ import annotations
 
+import sys
+
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
@@ -103,6 +105,12 @@ class Qwen2Model(nn.Module):
         self.norm = RMSNorm(cfg.hidden_size, eps=cfg.rms_norm_eps)
         self.rotary_emb = RotaryEmbedding(cfg.head_dim, max_position_embeddings=cfg.max_position_embeddings,
                                           base=cfg.rope_theta)
+
+    def table_sizes(self) -> tuple[int, int]:
+        """Ids and positions must stay below these (no bound for a replaced module's own)."""
+        embed, rope = self.embed_tokens, self.rotary_emb
+        return (embed.num_embeddings if type(embed) is nn.Embedding else sys.maxsize,
+                rope.cos_cached.shape[2] if type(rope) is RotaryEmbedding else sys.maxsize)
 
     def _input_rows(self, input_ids, positions):
         embed, rope = self.embed_tokens, self.rotary_emb

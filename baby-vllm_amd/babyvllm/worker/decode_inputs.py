@@ -56,9 +56,22 @@ def _layout(max_batch: int, max_blocks: int) -> dict[str, tuple[int, tuple[int, 
 _TORCH = {np.dtype(np.int64): torch.int64, np.dtype(np.int32): torch.int32}
 
 
+def check_inputs(ids, last_position: int, table_sizes: tuple[int, int]) -> None:
+    """IndexError for ids or positions outside the model's tables, as nn.Embedding's on the CPU is:
+    asked on the host, since neither a captured step nor the input-row kernel (NaN rows) raises."""
+    low, high = min(ids), max(ids)
+    if low < 0 or high >= table_sizes[0]:
+        raise IndexError(f"token id {low if low < 0 else high} is outside the embedding table of "
+                         f"{table_sizes[0]} rows")
+    if last_position >= table_sizes[1]:
+        raise IndexError(f"position {last_position} is past the model's {table_sizes[1]} positions")
+
+
 class DecodeInputs:
-    def __init__(self, max_batch: int, max_blocks: int, block_size: int, dummy_block: int, pin: bool):
+    def __init__(self, max_batch: int, max_blocks: int, block_size: int, dummy_block: int, pin: bool,
+                 table_sizes: tuple[int, int] | None = None):
         self.max_batch = max_batch
+        self.table_sizes = table_sizes  # of the tables the captured steps read, or None: not checked
         self.max_blocks = max_blocks
         self.block_size = block_size
         self.dummy_block = dummy_block
@@ -103,8 +116,12 @@ class DecodeInputs:
         if not n <= bucket <= self.max_batch:
             raise ValueError(f"{n} sequences do not fit a bucket of {bucket} rows (staging holds {self.max_batch})")
         pos = np.fromiter((s.num_computed_tokens for s in seqs), dtype=np.int64, count=n)
+        positions = pos.tolist()
+        ids = [s.token_ids[p] for s, p in zip(seqs, positions)]
+        if n and self.table_sizes is not None:
+            check_inputs(ids, max(positions), self.table_sizes)
         self.positions[:n] = pos
-        self.input_ids[:n] = [s.token_ids[p] for s, p in zip(seqs, pos.tolist())]
+        self.input_ids[:n] = ids
         self.context_lens[:n] = pos
         self.seq_lens[:n] = pos + 1
 

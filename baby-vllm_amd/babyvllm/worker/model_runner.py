@@ -31,7 +31,7 @@ from babyvllm.kernels.argmax import greedy_argmax
 from babyvllm.layers.attention import Attention
 from babyvllm.models.qwen2 import Qwen2ForCausalLM
 from babyvllm.worker.context import AttentionMetadata, set_forward_context
-from babyvllm.worker.decode_inputs import DecodeInputs
+from babyvllm.worker.decode_inputs import DecodeInputs, check_inputs
 
 BATCH_BUCKETS = [1, 2, 4, 8, 16, 32, 64]
 CTX_BUCKETS = [256, 2048]
@@ -133,6 +133,8 @@ class ModelRunner:
             qsl.append(qsl[-1] + n)
             seq_lens.append(ctx + n)
             ctx_lens.append(ctx)
+        if ids:
+            check_inputs(ids, max(seq_lens) - 1, self.model.model.table_sizes())
         width = max(len(t) for t in tables)
         dev = self.device
         md = AttentionMetadata(
@@ -215,7 +217,8 @@ class ModelRunner:
     def _host_inputs(self) -> DecodeInputs:
         if self._decode_inputs is None:
             self._decode_inputs = DecodeInputs(max(BATCH_BUCKETS), self.max_blocks_per_seq, self.block_size,
-                                               self._dummy_block, pin=self.device.type == "cuda")
+                                               self._dummy_block, pin=self.device.type == "cuda",
+                                               table_sizes=self.model.model.table_sizes())
         return self._decode_inputs
 
     def prepare_decode_inputs(self, seqs, block_tables, batch_bucket: int, ctx_bucket: int) -> StaticBuffers:

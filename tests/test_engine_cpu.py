@@ -697,3 +697,44 @@ def test_static_decode_buffers_on_cpu():
     runner = ModelRunner(cfg, cache_config=CacheConfig(), device="cpu")
     buf = runner._ensure_static_buffers(batch_bucket=4, ctx_bucket=256)
     assert buf.block_tables.shape == (4, 2048 // 16 + 1) and buf.logits.shape == (4, 100)
+
+
+def _index_runner():
+    from babyvllm.config import CacheConfig, ModelConfig
+    from babyvllm.worker.model_runner import ModelRunner
+
+    cfg = ModelConfig(vocab_size=100, hidden_size=128, intermediate_size=256, num_hidden_layers=1,
+                      num_attention_heads=2, num_key_value_heads=1, rms_norm_eps=1e-6,
+                      max_position_embeddings=64, rope_theta=10000.0, tie_word_embeddings=True)
+    runner = ModelRunner(cfg, cache_config=CacheConfig(num_gpu_blocks=8), device="cpu")
+    runner.allocate_kv_cache()
+    return runner
+
+
+@pytest.mark.parametrize("tokens,word", [([1, 100, 2], "100"), ([1, -1, 2], "-1"), ([0, 99, 99], None),
+                                         ([5] * 64, None), ([5] * 65, "position 64")])
+def test_ids_and_positions_outside_the_tables_raise_before_the_step(tokens, word):
+    """A prefill step and the staging of a captured decode step: an id outside the vocabulary or
+    a position past the tables is an IndexError, as nn.Embedding's is on the CPU."""
+    from babyvllm.scheduler import SchedulerOutput
+
+    runner = _index_runner()
+    seq = Sequence(tokens, SamplingParams(temperature=0.0))
+    n = len(tokens)
+    table = list(range(-(-n // 16)))
+    step = SchedulerOutput([seq], {seq.seq_id: n}, {seq.seq_id: table}, {seq.seq_id: list(range(n))}, [])
+    decode = Sequence(tokens[:1] + tokens[2:] + [tokens[1]], SamplingParams(temperature=0.0))
+    decode.num_computed_tokens = n - 1
+
+    def stage():
+        runner._decode_inputs = None
+        runner.prepare_decode_inputs([decode], {decode.seq_id: table}, 1, 256)
+
+    if word is None:
+        assert runner.prepare_inputs(step)[0].tolist() == tokens
+        stage()
+    else:
+        with pytest.raises(IndexError, match=word):
+            runner.prepare_inputs(step)
+        with pytest.raises(IndexError, match=word):
+            stage()
