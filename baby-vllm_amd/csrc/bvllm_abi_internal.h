@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "bvllm_fast_div.h"
+
 namespace bvllm {
 
 struct RopeArgs {
@@ -45,6 +47,7 @@ struct DecodeArgs {
   // Balanced single pass (RowChunk): chunks aimed at per column group, rows an even
   // share of which keeps every CU busy.
   int32_t chunk_target, row_slots;
+  FastDiv by_col_groups, by_batch;         // of item orders 0 and 2
   // Prefill view (both null for a decode batch): row b is sequence b of a
   // varlen prefill batch. Only sequences with exactly one query token are
   // computed; their q / out row is query_start_loc[b] and they attend keys

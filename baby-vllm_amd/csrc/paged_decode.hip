@@ -462,6 +462,8 @@ static hipError_t launch_decode(const DecodeArgs& args, hipStream_t stream) {
   const int64_t units = (a.num_splits + a.splits_per_item - 1) / a.splits_per_item;
   const int64_t items = (int64_t)a.batch * decode_col_groups(a) * units;
   if (items > 0x7ffffff0) return hipErrorInvalidValue;
+  a.by_col_groups = fast_div((int32_t)ncg);
+  a.by_batch = fast_div(a.batch);
   hipError_t err;
   if (p.quad && a.splits_per_item > 1) {
     err = launch_quad_group_vgpr(a, items, tuning(kTuneDecodeCached) == 0, stream);
