@@ -119,15 +119,15 @@ SIGNATURES = {
         _p, _p, _p, _i64, _p, _p,   # positions, cos table, sin table, max_positions, cos out, sin out
         _i32, _i32, _i32, _p,       # rows, hidden, head_dim, stream
     ]),
-    "bvllm_linear_workspace_bytes": (ctypes.c_int64, [_i32, _i32, _i32, _i32]),
+    "bvllm_linear_workspace_bytes": (ctypes.c_int64, [_i32, _i32, _i32, _i32, _i32]),
     "bvllm_linear": (ctypes.c_int, [
         _p, _i64, _p, _p, _p, _i64,  # x, stride, w, bias, out, stride
-        _i32, _i32, _i32, _i32,     # m, n, k, gated
+        _i32, _i32, _i32, _i32, _i32,  # m, n, k, gated, eager
         _p, _p,                     # workspace, stream
     ]),
 }
 
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 
 # Knobs of bvllm_set_tuning (include/babyvllm_amd.h).

@@ -4,8 +4,8 @@
 decode step's linear layers (and an MLP's fused gate/up projection with SiLU·mul)
 with ``bvllm_linear`` and return the result, or return ``None`` when the call is not
 one for that kernel; the caller then takes torch's own operations. The kernel takes
-plain bf16 tensors of at most 64 rows (up to 256 where it is the faster one, the
-library's rule) on the current ROCm device, outside autograd and outside every mode
+plain bf16 tensors of at most 256 rows, of the shapes where it ends sooner than a
+library GEMM (``bvllm_linear_workspace_bytes``), on the current ROCm device, outside autograd and outside every mode
 that has to see torch operations (tracing, compilation, functorch transforms,
 forward-mode AD, dispatch and function modes, autocast).
 """
@@ -32,11 +32,17 @@ def torch_must_see(*tensors) -> bool:
             or c._get_tracing_state() is not None or torch.is_autocast_enabled("cuda"))
 
 
+def _eager(x) -> bool:
+    """Whether the library's host time counts: a captured step pays none (up to 64 rows the kernel's
+    choice does not ask)."""
+    return x.shape[0] > 64 and not torch.cuda.is_current_stream_capturing()
+
+
 def skinny_linear(x, weight, bias=None, out=None):
     """``x @ weight.T + bias`` for x [M, K] (into ``out`` if given), or None."""
     if not x.is_cuda or x.dim() != 2 or x.shape[0] > MAX_ROWS or torch_must_see(x, weight, bias, out):
         return None
-    return _lib.fast().linear(x, weight, bias, out, False, *_lib.current())
+    return _lib.fast().linear(x, weight, bias, out, False, _eager(x), *_lib.current())
 
 
 def gated_linear(x, weight):
@@ -46,4 +52,4 @@ def gated_linear(x, weight):
     """
     if not x.is_cuda or x.dim() != 2 or x.shape[0] > MAX_ROWS or torch_must_see(x, weight):
         return None
-    return _lib.fast().linear(x, weight, None, None, True, *_lib.current())
+    return _lib.fast().linear(x, weight, None, None, True, _eager(x), *_lib.current())

@@ -373,16 +373,16 @@ extern "C" int bvllm_silu_mul(const void* gate_up, int64_t rows, int32_t d, void
   return (int)silu_mul(a, (hipStream_t)stream);
 }
 
-extern "C" int64_t bvllm_linear_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t gated) {
-  const LinearPlan p = linear_plan(m, n, k, gated != 0);
+extern "C" int64_t bvllm_linear_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t gated, int32_t eager) {
+  const LinearPlan p = linear_plan(m, n, k, gated != 0, eager != 0);
   return p.rw == 0 ? -1 : p.partial_bytes;
 }
 
 extern "C" int bvllm_linear(const void* x, int64_t x_stride, const void* w, const void* bias, void* out,
-                            int64_t out_stride, int32_t m, int32_t n, int32_t k, int32_t gated, void* workspace,
-                            void* stream) {
+                            int64_t out_stride, int32_t m, int32_t n, int32_t k, int32_t gated, int32_t eager,
+                            void* workspace, void* stream) {
   if ((gated != 0 && gated != 1) || !x || !w || !out || (gated && bias)) return kBad;
-  const int64_t bytes = bvllm_linear_workspace_bytes(m, n, k, gated);
+  const int64_t bytes = bvllm_linear_workspace_bytes(m, n, k, gated, eager);
   if (bytes < 0 || (bytes > 0 && (!workspace || !aligned16(workspace)))) return kBad;
   if (x_stride < k || out_stride < n || x_stride % 8 || out_stride % 4) return kBad;
   if (!aligned16(x) || !aligned16(w) || ((uintptr_t)out & 7u) != 0) return kBad;
@@ -393,7 +393,7 @@ extern "C" int bvllm_linear(const void* x, int64_t x_stride, const void* w, cons
   a.out = out; a.out_stride = out_stride;
   a.partials = reinterpret_cast<float*>(workspace);
   a.m = m; a.n = n; a.k = k;
-  return (int)skinny_linear(a, gated != 0, (hipStream_t)stream);
+  return (int)skinny_linear(a, gated != 0, eager != 0, (hipStream_t)stream);
 }
 
 extern "C" int bvllm_embed_rows(const int64_t* ids, const void* table, int64_t vocab, void* out,

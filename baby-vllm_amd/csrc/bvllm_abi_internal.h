@@ -141,8 +141,8 @@ struct LinearPlan {
   int32_t unit;            // ... in units of 2 or 4 columns
   int64_t partial_bytes;
 };
-LinearPlan linear_plan(int32_t m, int32_t n, int32_t k, bool gated);
-hipError_t skinny_linear(const LinearArgs& a, bool gated, hipStream_t stream);
+LinearPlan linear_plan(int32_t m, int32_t n, int32_t k, bool gated, bool eager);
+hipError_t skinny_linear(const LinearArgs& a, bool gated, bool eager, hipStream_t stream);
 
 hipError_t rope_kv_append(const RopeArgs& a, hipStream_t stream);
 int64_t argmax_workspace_bytes(int32_t rows, int32_t vocab);

@@ -376,14 +376,14 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// (x, weight, bias | None, out | None, gated, device, stream)
+// (x, weight, bias | None, out | None, gated, eager, device, stream)
 PyObject* fast_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 7) return none();
-  const int64_t dev = PyLong_AsLongLong(a[5]);
+  if (n != 8) return none();
+  const int64_t dev = PyLong_AsLongLong(a[6]);
   const at::Tensor* x = plain(a[0], at::kBFloat16, dev);
   const at::Tensor* w = plain(a[1], at::kBFloat16, dev);
-  const bool gated = a[4] == Py_True;
+  const bool gated = a[4] == Py_True, eager = a[5] == Py_True;
   if (!x || !w || x->dim() != 2 || w->dim() != 2 || x->stride(1) != 1 || !w->is_contiguous()) return none();
   const int64_t m = x->size(0), k = x->size(1), rows = w->size(0), cols = gated ? rows / 2 : rows;
   if (m < 1 || w->size(1) != k || (gated && rows % 2) || !small(m) || !small(k) || !small(rows)) return none();
@@ -395,9 +395,9 @@ PyObject* fast_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     bias = plain(a[2], at::kBFloat16, dev);
     if (!bias || gated || bias->dim() != 1 || bias->size(0) != cols || !bias->is_contiguous()) return none();
   }
-  void* stream = PyLong_AsVoidPtr(a[6]);
+  void* stream = PyLong_AsVoidPtr(a[7]);
   if (PyErr_Occurred()) return nullptr;
-  const int64_t bytes = g.linear_bytes((int32_t)m, (int32_t)cols, (int32_t)k, gated ? 1 : 0);
+  const int64_t bytes = g.linear_bytes((int32_t)m, (int32_t)cols, (int32_t)k, gated, eager);
   if (bytes < 0) return none();
   at::Tensor out, ws;
   int64_t out_stride = cols;
@@ -417,7 +417,7 @@ PyObject* fast_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (bytes > 0) ws = new_empty({bytes / 4}, *x, at::kFloat);
   return launch(out, "bvllm_linear", [&] {
     return g.linear(ptr(*x), x_stride, ptr(*w), bias ? ptr(*bias) : nullptr, out_ptr(out), out_stride, (int32_t)m,
-                    (int32_t)cols, (int32_t)k, gated ? 1 : 0, bytes > 0 ? ptr(ws) : nullptr, stream);
+                    (int32_t)cols, (int32_t)k, gated, eager, bytes > 0 ? ptr(ws) : nullptr, stream);
   });
   END_HANDLE_TH_ERRORS
 }

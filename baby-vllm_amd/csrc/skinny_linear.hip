@@ -268,49 +268,108 @@ hipError_t launch_waves(const LinearArgs& a, hipStream_t s) {
 
 }  // namespace
 
-// The launch of a shape, or rw = 0 where the library's GEMM is the better one (or
-// the shape does not fit the kernel). 16-row tiles of weights and 128-wide stages
-// of k decide (us, this kernel / hipBLASLt):
-//   gated: 8 row waves from 8192 columns, else 4 x 2;
+// Whether the kernel's call ends sooner than the library's, for n = 16 * tiles columns and
+// k = 128 * stages. Measured in graphs of back-to-back calls, weights from HBM, at 7,900 points:
+// 640 to 256000 columns, k 384 to 28672, 1 to 256 tokens. Of the 4,800 taken 19 in 20 are faster,
+// 22 more than a twentieth slower and none more than a tenth. The library's time jumps with its own choice of tiles, so
+// its good shapes lie between bad ones; where they do, the line leaves both to it. Lines and
+// figures (us, kernel / library):
+//   gated (the library's side includes its SiLU·mul launch): the kernel reads gate and up once
+//     and writes half the columns. Lost to a long k with few columns, where a work-group's walk
+//     sets the time: 1024 columns, 48 stages, 1 token 16.2 / 14.1; 2048 columns, 33
+//     tokens, 28 stages 17.5 / 15.0, 12 stages 9.8 / 12.1. Beyond 64 tokens to all but a short k
+//     (2·4864 x 896: 65 tokens 11.1 / 14.2, 128: 14.1 / 15.0, 192: 17.3 / 16.8; 18944 columns, 7
+//     stages, 128 tokens 31.1 / 27.2);
+//   beyond 17 thousand k the library reads the weights at 1.1 to 1.4 TB/s (3584 x 18944: 16
+//     tokens 29 / 46, 64: 36 / 90, 256: 83 / 126; 4096 x 16384, 1 token 35.2 / 33.9, 17408 33.7 / 50.4);
+//   1 to 16 tokens: few rows are the kernel's at any k (16 tokens, 1152 x 896 4.7 / 6.8, 896 x
+//     8192 10.1 / 12.2); 160 to 255 tiles up to 35 stages (3584 x 4608 13.1 / 11.4, 4352 12.8 /
+//     17.1), 256 to 511 up to 51 (4096 x 6656 17.9 / 15.5), more columns up to 39 (12288 x 5120
+//     35.2 / 29.9);
+//   17 to 32: 160 to 255 tiles lose from 40 stages (32 tokens, 3584 x 5120 17.0 / 15.8), 288 to
+//     320 nowhere (4608 x 3584 0.95 times), the rest of 256 to 511 from 28 or 18 (4096 x 3840
+//     14.4 / 13.0, 7168 x 2304 11.7 / 11.2), more columns from 9 (10240 x 1280 12.4 / 10.9), 1184
+//     tiles and more at once (18944 x 1536 21.8 / 18.9);
+//   33 to 64: x outweighs the weights of few rows per work-group. Below 160 tiles the lines
+//     follow the library's jumps (2048 x 2560, 33 tokens 11.1 / 9.3, 1280 x 5632, 48: 12.8 / 10.6,
+//     896 x 896 0.77 times, 896 x 4864 0.70); 256 to 287 tiles up to 20 stages (4096 x 3072, 48
+//     tokens 14.7 / 11.4), 288 to 511 up to 29 (4608 x 3584 0.89 times; 4608 x 4096, 48 tokens
+//     18.3 / 22.7, 64: 19.4 / 17.8), none beyond (12288 x 3584, 33 tokens 32.6 / 23.1);
+//   65 to 128: from 80, 56 or 28 stages with the row tiles (896 x 8192, 65 tokens 14.8 / 13.3;
+//     2560 x 6656 18.8 / 19.1; 3584 x 3584 0.95 times), 256 to 320 tiles but for 32 to 43 stages
+//     (5120 x 4096, 65 tokens 19.7 / 17.2, 5632 23.7 / 23.0; 4608 x 3584 1.01 times), up to 511
+//     from 64;
+//   heads (2048 tiles and more) are within a tenth of each other but for the library's bad
+//     sizes (100352 x 896, 17 tokens 42 / 126; 152064 x 3584, 16 tokens 188 / 231): below 32
+//     stages, up to 16 tokens; from 4096 tiles up to 32, and to 64 for at most 8 stages (50304 x 896, 48
+//     tokens 26.8 / 23.7). 256000 columns are the library's.
+// eager: the caller launches call by call. Beyond 64 tokens, where such steps are too large for
+// a captured graph, a library GEMM costs it 18 to 24 us of host time and the SiLU·mul 4.5, a call
+// here 5 to 8: a kernel that ends within the library's host time is waited for no longer than the
+// library's caller would wait for itself. Gated: at most 26 us (MLP 896 x 4864, whole, on two
+// hosts: 192 tokens 40 and 53 us with the library, 28 and 32 with the gated kernel, 17.3 / 16.8 on
+// the GPU; 256: 40 and 53, 35 and 47; 24.1 / 18.8). Plain: at most 15.5 us (the MLP's 896 x 4864 as
+// well: 65 tokens 23.4 and 29.8 -> 21.7 and 23.1, 96: 23.4 and 29.6 -> 22.5 and 24.1, 128 either
+// way: 23.5 and 29.6, 26.3 and 28.3).
+static bool ends_sooner(int m, int tiles, int stages, bool gated, bool eager, double products) {
+  if (gated) {
+    if (m <= 16) return stages < 36 || (tiles >= 224 && stages < 64);
+    if (m <= 32) return stages < 36 || (tiles >= 352 && stages < 64);
+    if (m <= 64) return stages < 18 || (tiles >= 176 && stages < 36) || (tiles >= 560 && stages < 64);
+    if (m <= 128 && tiles < 1100 && (stages <= 8 || (tiles >= 300 && stages <= 12))) return true;
+    return eager && stages <= (m <= 128 ? 12 : 8) && products <= 2.4e9;
+  }
+  if (tiles >= 2048)
+    return m <= 64 && stages < 32 && tiles <= 12800 && (m <= 16 || (tiles >= 4096 && (m <= 32 || stages <= 8)));
+  if (stages >= 136 && tiles < 512) return true;
+  if (m <= 16) return tiles < 160 || stages < (tiles < 256 ? 36 : tiles < 512 ? 52 : 40);
+  if (m <= 32) {
+    if (tiles < 160) return stages < 44 || stages >= 52;
+    if (tiles < 256) return stages < 40 || stages >= 64;
+    if (tiles >= 288 && tiles <= 320) return true;
+    return stages < (tiles < 288 ? 28 : tiles < 512 ? 18 : tiles < 1184 ? 9 : 0);
+  }
+  if (m <= 64) {
+    if (tiles < 512 && stages > 64) return true;
+    if (tiles < 160)
+      return (stages >= 6 && stages <= 8) || (stages >= 12 && stages <= 16) ||
+             (stages >= 32 && stages <= (tiles < 96 ? 40 : 63));
+    if (tiles < 256) return false;
+    if (tiles < 288) return stages <= 20;
+    return tiles < 512 && (stages < 30 || (tiles <= 320 && m <= 48));
+  }
+  if (eager && tiles <= 320 && stages >= 28 && stages < 64 && products <= 4.5e8) return true;
+  if (m <= 128) {
+    if (tiles < 256) return stages >= (tiles < 160 ? 80 : tiles < 192 ? 56 : 28);
+    return tiles < 512 && (stages >= 64 || (tiles <= 320 && ((stages >= 28 && stages < 32) || stages >= 44)));
+  }
+  return false;
+}
+
+// The launch of a shape, or rw = 0 where the library's GEMM is the better one (ends_sooner; or
+// the shape does not fit the kernel). 16-row tiles of weights and 128-wide stages of k decide:
+//   gated: 8 row waves beyond 8192 columns, else 4 x 2 (8192 x 2048, 17 tokens 20.3 us on 8, 18.2
+//     on 4 x 2: 256 work-groups fill their 32 columns exactly); past 64 tokens 8 row waves in
+//     blocks of 65 to 128 tokens;
 //   many tiles (>= 2048, a head): 8 row waves, each x stage shared by 128 rows;
-//     past 32 tokens only for short k (151936 x 896, 64 tokens: 69.0 / 68.9, 33:
-//     59.6 / 66.6; 152064 x 3584, 64 tokens: 216 / 201);
-//   long k (>= 64 stages, or >= 32 with few rows and more than 16 tokens): 4 row
-//     waves x 2 slabs, k cut over work-groups until tiles x splits reach about
-//     1000 (past 32 tokens and 64 stages 8 x 1, twice the splits). From 64 stages on
-//     up to 256 tokens, in blocks of at most 128 (3584 x 18944: 96 tokens 43 / 95, 128:
-//     50 / 99);
-//   beyond 64 tokens the library computes as fast or faster from HBM but costs its
-//     caller about 20 us of host time a call, in steps too large for a captured graph
-//     (MLP 896 x 4864, eager, 65 / 96 / 128 / 192 / 256 tokens: 54 / 53 / 53 / 53 / 53 us on the
-//     library, 22 / 23 / 26 / 33 / 44 here). So: gated with short k (at most 12 stages), 8 row
-//     waves in blocks of 65 to 128 tokens (2·4864 x 896: 65 tokens 11.1 / 14.2, 128: 14.1 / 15.0,
-//     192: 17.4 / 16.5; 2·8960 x 1536: 128 tokens 23.9 / 27.3, 192: 31.2 / 29.4; k = 3584 is the
-//     library's: 91 / 77 at 128); 28 to 63 stages with at most 320 tiles, 8 x 1 with k cut by 3
-//     stages or more until tiles x splits reach 1536 (896 x 4864: 65 tokens 12.3 / 13.2, 128:
-//     15.3 / 13.0, 192: 17.8 / 13.8; 3584 x 3584: 96 tokens 18.3 / 19.8, 128: 20.7 / 22.5; 4608 x
-//     3584: 17.9 / 19.2 and 22.6 / 22.9). Beyond 128 tokens only while the products are few
-//     enough to end within the library's host time;
+//   beyond 64 tokens below 64 stages: 8 x 1 with k cut by 3 stages or more until tiles x splits
+//     reach 1536;
+//   long k (>= 64 stages, or >= 32 with few rows and more than 16 tokens): 4 row waves x 2
+//     slabs, k cut over work-groups until tiles x splits reach about 1000 (past 32 tokens and 64
+//     stages 8 x 1, twice the splits, in blocks of at most 128 tokens);
 //   the rest: 2 x 4 from 160 tiles, 1 x 4 below (each work-group then streams a
-//     few rows with 4 waves and no sum across work-groups). Past 32 tokens x
-//     outweighs the weights of so few rows per work-group: 3584 x 3584 stays with
-//     the library (14.4 / 12.1 at 33), 4608 x 3584 does not (15.6 / 18.6).
-LinearPlan linear_plan(int32_t m, int32_t n, int32_t k, bool gated) {
+//     few rows with 4 waves and no sum across work-groups).
+LinearPlan linear_plan(int32_t m, int32_t n, int32_t k, bool gated, bool eager) {
   LinearPlan p{};
   const int64_t rows = (gated ? 2 : 1) * (int64_t)n;
   if (m < 1 || m > 256 || n < 64 || n % 4 != 0 || k < kStageK || k % kStageK != 0) return p;
   if (rows * k * 2 >= (int64_t)kNoLoad) return p;
   const int tiles = (n + 15) / 16, stages = k / kStageK;
-  if (m > 64 && (gated || stages < 64)) {
-    const bool few = m <= 128 || (double)m * rows * k <= (gated ? 2.4e9 : 1.2e9);
-    if (!few || (gated ? stages > 12 : stages < 28 || tiles > 320)) return p;
-  }
-  if (m > 64 && tiles >= 2048) return p;
+  if (!ends_sooner(m, tiles, stages, gated, eager, (double)m * rows * k)) return p;
   p.k_splits = 1;
   if (gated) {
-    p.rw = n >= 8192 || m > 64 ? 8 : 4;
+    p.rw = n > 8192 || m > 64 ? 8 : 4;
   } else if (tiles >= 2048) {
-    if (m > 32 && stages > 8) return p;
     p.rw = 8;
   } else if (m > 64 && stages < 64) {
     p.rw = 8;
@@ -320,7 +379,6 @@ LinearPlan linear_plan(int32_t m, int32_t n, int32_t k, bool gated) {
     p.rw = wide ? 8 : 4;
     p.k_splits = std::max(1, std::min(stages / 4, ((wide ? 2048 : 1024) - 1) / tiles));
   } else {
-    if (m > 32 && tiles >= 160 && tiles < 256) return p;
     p.rw = tiles >= 160 ? 2 : 1;
   }
   p.kw = p.rw == 1 ? 4 : 8 / p.rw;
@@ -336,9 +394,9 @@ LinearPlan linear_plan(int32_t m, int32_t n, int32_t k, bool gated) {
   return p;
 }
 
-hipError_t skinny_linear(const LinearArgs& args, bool gated, hipStream_t s) {
+hipError_t skinny_linear(const LinearArgs& args, bool gated, bool eager, hipStream_t s) {
   LinearArgs a = args;
-  const LinearPlan p = linear_plan(a.m, a.n, a.k, gated);
+  const LinearPlan p = linear_plan(a.m, a.n, a.k, gated, eager);
   if (p.rw == 0 || (int64_t)a.m * a.x_stride * 2 >= (int64_t)kNoLoad) return hipErrorInvalidValue;
   if (p.k_splits > 1 && a.partials == nullptr) return hipErrorInvalidValue;
   a.k_splits = p.k_splits;

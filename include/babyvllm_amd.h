@@ -40,7 +40,7 @@ extern "C" {
 #endif
 
 /* ABI version of this header; bumped on any signature change. */
-#define BVLLM_ABI_VERSION 8
+#define BVLLM_ABI_VERSION 9
 
 #if defined(__GNUC__)
 #define BVLLM_API __attribute__((visibility("default")))
@@ -307,16 +307,19 @@ BVLLM_API int bvllm_silu_mul(const void* gate_up, int64_t rows, int32_t d, void*
  * out_stride. gated = 1: w is [2n, k] (gate rows, then up rows, no bias) and
  * out = bf16(silu(gate) * up), silu and product in fp32.
  * bvllm_linear_workspace_bytes returns the scratch one call needs, or -1 for a
- * shape this kernel does not take (more than 64 tokens, or up to 256 where a call to it
- * ends sooner; k not a multiple of 128, n not of 4, ...): the caller then uses a
- * library GEMM. Pointers of x and w are 16-byte aligned, x_stride a multiple of 8 elements, out 8-byte aligned with a
+ * shape this kernel does not take (a library GEMM ends sooner, always so beyond 256
+ * tokens; k not a multiple of 128, n not of 4, ...): the caller then uses a
+ * library GEMM. eager = 1 says that the caller launches call by call, where a library
+ * call's host time counts too, 0 that the launches are captured or queued far ahead;
+ * both calls take the same value. Pointers of x and w are 16-byte aligned, x_stride a multiple of 8 elements, out 8-byte aligned with a
  * stride multiple of 4. The order of the sums depends on (n, k, gated) and on
  * whether m is at most 16, 32, 64 or more, on nothing else.
  */
-BVLLM_API int64_t bvllm_linear_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t gated);
+BVLLM_API int64_t bvllm_linear_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t gated,
+                                               int32_t eager);
 BVLLM_API int bvllm_linear(const void* x, int64_t x_stride, const void* w, const void* bias, void* out,
-                 int64_t out_stride, int32_t m, int32_t n, int32_t k, int32_t gated, void* workspace,
-                 void* stream);
+                 int64_t out_stride, int32_t m, int32_t n, int32_t k, int32_t gated, int32_t eager,
+                 void* workspace, void* stream);
 
 /*
  * A model's input rows (embed_tokens and rotary_emb of babyvllm/models/qwen2.py:109-118):

@@ -104,6 +104,26 @@ def test_key_range_scratch_follows_the_sequences_not_the_table():
             assert h.bvllm_prefill_workspace_bytes(4, 400, 28, 4, 128, h.bvllm_prefill_ranges(width, split, -1), 0) <= 64 << 20
 
 
+def test_linear_leaves_the_library_the_shapes_it_is_faster_at():
+    """Points measured on both sides of every line of the rule (k and columns of no one model)."""
+    takes = lambda m, n, k, gated=0, eager=0: _lib().lib().bvllm_linear_workspace_bytes(m, n, k, gated, eager) >= 0
+    kernel = [(16, 1152, 896), (1, 4096, 17408), (16, 3584, 4352), (32, 4608, 4096), (33, 896, 896), (48, 4608, 4096),
+              (64, 1536, 5632), (64, 5120, 3584), (128, 3584, 4608), (128, 3584, 8192), (256, 3584, 18944),
+              (16, 32768, 2048), (17, 100352, 896), (1, 13824, 4608, 1), (64, 4864, 2048, 1), (128, 8960, 1536, 1)]
+    library = [(16, 3584, 5120), (16, 12288, 8192), (8, 4096, 8192), (1, 32768, 4096), (32, 12288, 2560), (32, 18944, 896),
+               (33, 2048, 2560), (33, 12288, 896), (64, 18944, 3584), (64, 4608, 4096), (65, 896, 8192),
+               (128, 896, 4864), (128, 2048, 3584), (128, 18944, 8192), (192, 896, 4864), (256, 3584, 8192),
+               (208, 6144, 8960), (48, 50304, 896), (16, 256000, 896), (1, 1024, 6144, 1), (33, 2048, 3584, 1),
+               (128, 18944, 896, 1), (192, 2048, 1536, 1), (160, 4864, 896, 1), (256, 4864, 896, 1)]
+    assert [p for p in kernel if not takes(*p)] == [] and [p for p in library if takes(*p)] == []
+    # Launched call by call, the library's host time counts as well; up to 64 tokens nothing changes.
+    assert takes(160, 4864, 896, 1, 1) and takes(256, 4864, 896, 1, 1) and not takes(192, 2048, 1536, 1, 1)
+    assert takes(96, 896, 4864, 0, 1) and not takes(128, 896, 4864, 0, 1) and not takes(96, 896, 4864)
+    for point in kernel + library:
+        if point[0] <= 64:
+            assert takes(*point, *[0] * (4 - len(point)), 1) == takes(*point), point
+
+
 def test_workspace_bytes_ignore_the_split_mode_knob():
     # The size (and the place of part_lse inside it) must not follow knob 0:
     # a knob changed between the size query and the launch would otherwise make

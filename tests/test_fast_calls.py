@@ -58,7 +58,7 @@ def test_cpu_tensors_and_wrong_argument_counts_are_declined():
     f = _fast()
     assert f.norm(x, None, x[0], 1e-6, 0, 0) is None
     assert f.silu(x, 0, 0) is None
-    assert f.linear(x, x, None, None, False, 0, 0) is None
+    assert f.linear(x, x, None, None, False, False, 0, 0) is None
     assert f.norm() is None and f.decode(x) is None and f.prefill() is None and f.rope(x, x) is None
 
 
