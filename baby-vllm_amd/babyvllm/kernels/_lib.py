@@ -130,6 +130,9 @@ SIGNATURES = {
 ABI_VERSION = 9
 
 
+# Pages (rows · table width) that the balanced launches take.
+BALANCED_MAX_PAGES = 1 << 30
+
 # Knobs of bvllm_set_tuning (include/babyvllm_amd.h).
 TUNE_DECODE_SPLIT_MODE = 0
 TUNE_PREFILL_BLOCKS_PER_WG = 1

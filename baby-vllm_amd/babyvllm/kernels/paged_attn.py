@@ -93,7 +93,7 @@ def paged_decode_attention(q, kv_cache, block_tables, seq_lens, scale,
         out.data_ptr(), out.stride(0), out.stride(1),
     )
     balanced = num_splits == 1 and blocks_per_split > BALANCE_MIN_PAGES and partition_blocks is None \
-        and os.environ.get(DECODE_PARTITION_ENV, "auto") == "auto"
+        and B * width <= _lib.BALANCED_MAX_PAGES and os.environ.get(DECODE_PARTITION_ENV, "auto") == "auto"
     if balanced:
         nbytes = h.bvllm_decode_balanced_workspace_bytes(B, n_heads, n_kv_heads, head_dim)
     else:

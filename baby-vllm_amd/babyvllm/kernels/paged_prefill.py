@@ -125,7 +125,9 @@ def paged_prefill_attention(q, kv_cache, md, scale):
         num_heads, num_kv_heads, head_dim, page,
     )
     h = _lib.lib()
-    balance = _balance_rows(md, num_seqs, num_heads, num_kv_heads) if single > 0 else 0
+    balance = 0
+    if single > 0 and num_seqs * bt.shape[1] <= _lib.BALANCED_MAX_PAGES:
+        balance = _balance_rows(md, num_seqs, num_heads, num_kv_heads)
     if split_tiles > 0 or balance:
         ranges = 0
         if split_tiles > 0:

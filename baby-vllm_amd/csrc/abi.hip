@@ -153,6 +153,7 @@ extern "C" int bvllm_paged_decode_balanced(const void* q, int64_t q_stride_b, in
   if (head_dim != 64 && head_dim != 128) return kBad;
   if (block_size != 16) return kBad;
   if (batch == 0) return 0;
+  if ((int64_t)batch * max_blocks > BVLLM_BALANCED_MAX_PAGES) return kBad;
   if (!q || !out || !block_tables || !seq_lens || !workspace || !aligned16(workspace)) return kBad;
   if (!cache_ok(k_cache, v_cache, cache_stride_block, cache_stride_tok, cache_stride_head, num_blocks))
     return kBad;
@@ -303,6 +304,7 @@ extern "C" int bvllm_paged_prefill_split(const void* q, int64_t q_stride_t, int6
   if (rc != 0 || nothing) return rc;
   if (split_tiles < 0 || split_tiles > (1 << 20) || !workspace || !aligned16(workspace)) return kBad;
   // Every range starts inside the table.
+  if (balance_rows && (int64_t)num_seqs * max_blocks > BVLLM_BALANCED_MAX_PAGES) return kBad;
   if (split_tiles > 0 && (num_ranges < 1 || num_ranges > prefill_ranges(max_blocks, split_tiles, -1))) return kBad;
   float* ws = reinterpret_cast<float*>(workspace);
   if (split_tiles > 0) {

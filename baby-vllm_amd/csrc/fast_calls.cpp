@@ -266,7 +266,7 @@ PyObject* fast_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (env != nullptr && std::strcmp(env, "auto") != 0) return none();
   const Plan p = auto_plan(batch, hkv, c->size(2), width, max_seq_len, cus, min_pages);
   if (!small(p.splits) || !small(p.pages)) return none();
-  const bool balanced = p.splits == 1 && p.pages > balance;
+  const bool balanced = p.splits == 1 && p.pages > balance && batch * width <= BVLLM_BALANCED_MAX_PAGES;
   const int64_t bytes =
       balanced ? g.balanced_bytes((int32_t)batch, (int32_t)heads, (int32_t)hkv, (int32_t)d)
                : g.decode_bytes((int32_t)batch, (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)p.splits, (int32_t)p.pages);
@@ -351,7 +351,7 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                    : g.split_tiles((int32_t)seqs, (int32_t)tokens, (int32_t)max_q, (int32_t)single,
                                                    (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)width, tiles,
                                                    longest_tiles);
-  const int32_t balance = pages > 0 ? g.balance_rows((int32_t)heads, (int32_t)hkv, longest, pages) : 0;
+  const int32_t balance = pages > 0 && seqs * width <= BVLLM_BALANCED_MAX_PAGES ? g.balance_rows((int32_t)heads, (int32_t)hkv, longest, pages) : 0;
   const int32_t ranges = split > 0 ? g.ranges((int32_t)width, split, longest_tiles) : 0;
   at::Tensor out = new_empty({tokens, heads, d}, *q, at::kBFloat16), ws;
   if (split > 0 || balance)

@@ -392,7 +392,8 @@ struct RowChunk {
 
 // Chunk number `item` (item >= 0), or the chunks of row `item_row` (item < 0: `row`
 // then is item_row and `index` the number of its first chunk). Every wave computes the
-// same answer from the batch's lengths, 64 rows per step.
+// same answer from the batch's lengths, 64 rows per step. (Their pages add up in 32 bits:
+// at most BVLLM_BALANCED_MAX_PAGES, checked on the host, so the chunks fit their slots.)
 __device__ __forceinline__ RowChunk find_row_chunk(const DecodeArgs& a, int item, int item_row) {
   const int lane = lane_id();
   // Pages of row b; -1 for a row of a prefill batch that is not a single query.

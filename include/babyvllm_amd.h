@@ -126,8 +126,10 @@ BVLLM_API int bvllm_paged_decode(const void* q, int64_t q_stride_b, int64_t q_st
  * chunks' fp32 (o, lse). A row that stays whole has the single pass's bits; the cut
  * depends on seq_lens and the head counts only, never on max_blocks, so a launch
  * sized for a longer context gives the same bits. workspace holds
- * bvllm_decode_balanced_workspace_bytes() bytes.
+ * bvllm_decode_balanced_workspace_bytes() bytes. batch * max_blocks is at most
+ * BVLLM_BALANCED_MAX_PAGES (the device adds the batch's pages in 32 bits).
  */
+#define BVLLM_BALANCED_MAX_PAGES (1ll << 30)
 BVLLM_API int64_t bvllm_decode_balanced_workspace_bytes(int32_t batch, int32_t num_heads, int32_t num_kv_heads,
                                                         int32_t head_dim);
 BVLLM_API int bvllm_paged_decode_balanced(const void* q, int64_t q_stride_b, int64_t q_stride_h,
@@ -208,8 +210,8 @@ BVLLM_API int bvllm_paged_prefill(const void* q, int64_t q_stride_t, int64_t q_s
  *     tiles, every (block, range) on a work-group of its own, for few new tokens
  *     behind long prefixes;
  *   balance_rows = 1: the single-query sequences' rows are cut into chunks chosen on
- *     the device from their lengths (as bvllm_paged_decode_balanced does), for decode
- *     rows far from equal or few.
+ *     the device from their lengths (as bvllm_paged_decode_balanced does, with
+ *     num_seqs * max_blocks in its bound), for decode rows far from equal or few.
  * bvllm_prefill_split_tiles returns the split_tiles to use for a batch's shape, or 0
  * where the plain launch is the better one; key_tiles is the number of 64-key tiles the
  * batch's blocks of 128 (query, head) pairs cover, per KV head, summed over its

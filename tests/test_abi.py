@@ -169,6 +169,19 @@ def test_host_side_argument_rejection():
                                 None, 0, 0, None, 1, 1, 0, 28, 4, 128, 16, 0, None) == 0
 
 
+def test_balanced_launches_refuse_more_pages_than_they_can_add_up():
+    # Refused before anything is launched: the pointers below are never read.
+    mod = _lib()
+    h, p = mod.lib(), 4096
+    limit = int(re.search(r"#define BVLLM_BALANCED_MAX_PAGES \(1ll << (\d+)\)", HEADER.read_text()).group(1))
+    assert mod.BALANCED_MAX_PAGES == 1 << limit
+    for batch, width in ((64, (1 << 24) + 1), (1, (1 << 30) + 1), (300, 1 << 23)):
+        assert h.bvllm_paged_decode_balanced(p, 3584, 128, p, p, 8192, 512, 128, 100, p, width, width, p, 1.0, p, 3584,
+                                             128, p, batch, 28, 4, 128, 16, None) == 1
+        assert h.bvllm_paged_prefill_split(p, 3584, 128, p, p, 8192, 512, 128, 100, p, width, width, p, p, p, 1.0, p,
+                                           3584, 128, batch, batch, 1, batch, 28, 4, 128, 16, p, 0, 0, 1, None) == 1
+
+
 def test_python_ops_refuse_cpu_tensors():
     from babyvllm.kernels.paged_attn import paged_decode_attention
     from babyvllm.kernels.rope import fused_rope_and_cache
