@@ -215,6 +215,16 @@ def stream_handle(device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def optional_scratch(nbytes: int, device):
+    """Scratch of a launch that a form without any can stand in for, or None without the memory for it."""
+    import torch
+
+    try:
+        return torch.empty(nbytes // 4, device=device, dtype=torch.float32)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def require_rocm_tensor(name: str, t) -> None:
     if not t.is_cuda:
         raise RuntimeError(

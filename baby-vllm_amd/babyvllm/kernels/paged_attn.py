@@ -94,11 +94,14 @@ def paged_decode_attention(q, kv_cache, block_tables, seq_lens, scale,
     )
     balanced = num_splits == 1 and blocks_per_split > BALANCE_MIN_PAGES and partition_blocks is None \
         and B * width <= _lib.BALANCED_MAX_PAGES and os.environ.get(DECODE_PARTITION_ENV, "auto") == "auto"
+    workspace = None
     if balanced:
         nbytes = h.bvllm_decode_balanced_workspace_bytes(B, n_heads, n_kv_heads, head_dim)
-    else:
+        workspace = _lib.optional_scratch(nbytes, q.device) if nbytes > 0 else None
+        balanced = workspace is not None
+    if not balanced:
         nbytes = h.bvllm_decode_workspace_bytes(B, n_heads, n_kv_heads, head_dim, num_splits, blocks_per_split)
-    workspace = torch.empty(nbytes // 4, device=q.device, dtype=torch.float32) if nbytes > 0 else None
+        workspace = torch.empty(nbytes // 4, device=q.device, dtype=torch.float32) if nbytes > 0 else None
     ws = None if workspace is None else workspace.data_ptr()
     stream = _lib.stream_handle(q.device)
     if balanced:

@@ -128,6 +128,7 @@ def paged_prefill_attention(q, kv_cache, md, scale):
     balance = 0
     if single > 0 and num_seqs * bt.shape[1] <= _lib.BALANCED_MAX_PAGES:
         balance = _balance_rows(md, num_seqs, num_heads, num_kv_heads)
+    workspace = None
     if split_tiles > 0 or balance:
         ranges = 0
         if split_tiles > 0:
@@ -135,7 +136,8 @@ def paged_prefill_attention(q, kv_cache, md, scale):
             ranges = h.bvllm_prefill_ranges(bt.shape[1], split_tiles, longest)
         nbytes = h.bvllm_prefill_workspace_bytes(num_seqs, num_tokens, num_heads, num_kv_heads, head_dim, ranges,
                                                  balance)
-        workspace = torch.empty(nbytes // 4, device=q.device, dtype=torch.float32)
+        workspace = _lib.optional_scratch(nbytes, q.device)
+    if workspace is not None:
         rc = h.bvllm_paged_prefill_split(*args, workspace.data_ptr(), split_tiles, ranges, balance,
                                          _lib.stream_handle(q.device))
     else:

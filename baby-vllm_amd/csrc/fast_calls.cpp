@@ -104,6 +104,16 @@ at::Tensor new_empty(at::IntArrayRef sizes, const at::Tensor& like, at::ScalarTy
   return at::empty(sizes, like.options().dtype(t).requires_grad(false));
 }
 
+// Scratch of a launch that a form without any can stand in for: undefined where there is no
+// memory for it, and the caller takes that form.
+at::Tensor optional_scratch(int64_t bytes, const at::Tensor& like) {
+  try {
+    return new_empty({bytes / 4}, like, at::kFloat);
+  } catch (const c10::OutOfMemoryError&) {
+    return {};
+  }
+}
+
 void* ptr(const at::Tensor& t) { return const_cast<void*>(t.const_data_ptr()); }
 // What a kernel writes: a lazily cloned tensor gets its own storage here, as with data_ptr() in Python.
 void* out_ptr(const at::Tensor& t) { return t.mutable_data_ptr(); }
@@ -266,13 +276,19 @@ PyObject* fast_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (env != nullptr && std::strcmp(env, "auto") != 0) return none();
   const Plan p = auto_plan(batch, hkv, c->size(2), width, max_seq_len, cus, min_pages);
   if (!small(p.splits) || !small(p.pages)) return none();
-  const bool balanced = p.splits == 1 && p.pages > balance && batch * width <= BVLLM_BALANCED_MAX_PAGES;
-  const int64_t bytes =
-      balanced ? g.balanced_bytes((int32_t)batch, (int32_t)heads, (int32_t)hkv, (int32_t)d)
-               : g.decode_bytes((int32_t)batch, (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)p.splits, (int32_t)p.pages);
+  bool balanced = p.splits == 1 && p.pages > balance && batch * width <= BVLLM_BALANCED_MAX_PAGES;
   at::Tensor out = new_empty({batch, heads, d}, *q, at::kBFloat16), ws;
-  if (bytes > 0) ws = new_empty({bytes / 4}, *q, at::kFloat);
-  void* wp = bytes > 0 ? ptr(ws) : nullptr;
+  if (balanced) {
+    const int64_t bytes = g.balanced_bytes((int32_t)batch, (int32_t)heads, (int32_t)hkv, (int32_t)d);
+    if (bytes > 0) ws = optional_scratch(bytes, *q);
+    balanced = ws.defined();
+  }
+  if (!balanced) {
+    const int64_t bytes =
+        g.decode_bytes((int32_t)batch, (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)p.splits, (int32_t)p.pages);
+    if (bytes > 0) ws = new_empty({bytes / 4}, *q, at::kFloat);
+  }
+  void* wp = ws.defined() ? ptr(ws) : nullptr;
   return launch(out, "bvllm_paged_decode", [&] {
     const int32_t* tables = bt->const_data_ptr<int32_t>();
     const int32_t* l = lens->const_data_ptr<int32_t>();
@@ -347,18 +363,19 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* stream = PyLong_AsVoidPtr(a[12]);
   if (PyErr_Occurred()) return nullptr;
   if (!small(max_q)) return none();
-  const int32_t split = !may_split ? 0
+  int32_t split = !may_split ? 0
                                    : g.split_tiles((int32_t)seqs, (int32_t)tokens, (int32_t)max_q, (int32_t)single,
                                                    (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)width, tiles,
                                                    longest_tiles);
-  const int32_t balance = pages > 0 && seqs * width <= BVLLM_BALANCED_MAX_PAGES ? g.balance_rows((int32_t)heads, (int32_t)hkv, longest, pages) : 0;
+  int32_t balance = pages > 0 && seqs * width <= BVLLM_BALANCED_MAX_PAGES ? g.balance_rows((int32_t)heads, (int32_t)hkv, longest, pages) : 0;
   const int32_t ranges = split > 0 ? g.ranges((int32_t)width, split, longest_tiles) : 0;
   at::Tensor out = new_empty({tokens, heads, d}, *q, at::kBFloat16), ws;
-  if (split > 0 || balance)
-    ws = new_empty({g.prefill_bytes((int32_t)seqs, (int32_t)tokens, (int32_t)heads, (int32_t)hkv, (int32_t)d, ranges,
-                                    balance) /
-                    4},
-                   *q, at::kFloat);
+  if (split > 0 || balance) {
+    ws = optional_scratch(g.prefill_bytes((int32_t)seqs, (int32_t)tokens, (int32_t)heads, (int32_t)hkv, (int32_t)d,
+                                          ranges, balance),
+                          *q);
+    if (!ws.defined()) split = balance = 0;
+  }
   return launch(out, "bvllm_paged_prefill", [&] {
     const int32_t *tables = bt->const_data_ptr<int32_t>(), *ql = qsl->const_data_ptr<int32_t>();
     const int32_t *sl = seq->const_data_ptr<int32_t>(), *cl = ctx->const_data_ptr<int32_t>();
@@ -414,7 +431,10 @@ PyObject* fast_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   } else {
     out = new_empty({m, cols}, *x, at::kBFloat16);
   }
-  if (bytes > 0) ws = new_empty({bytes / 4}, *x, at::kFloat);
+  if (bytes > 0) {
+    ws = optional_scratch(bytes, *x);
+    if (!ws.defined()) return none();  // the library's
+  }
   return launch(out, "bvllm_linear", [&] {
     return g.linear(ptr(*x), x_stride, ptr(*w), bias ? ptr(*bias) : nullptr, out_ptr(out), out_stride, (int32_t)m,
                     (int32_t)cols, (int32_t)k, gated, eager, bytes > 0 ? ptr(ws) : nullptr, stream);

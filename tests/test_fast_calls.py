@@ -156,6 +156,61 @@ def test_decode_takes_a_bucket_of_any_size_as_the_python_path_does(max_len, monk
 
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a ROCm GPU")
+@pytest.mark.parametrize("path", ["native", "python"])
+@pytest.mark.parametrize("op", ["decode", "prefill", "linear"])
+def test_calls_without_the_memory_for_scratch_take_the_form_that_needs_none(op, path, monkeypatch):
+    """A serving process may have given the card to its KV pool: calls that ran without scratch
+    before they had a faster form with some still run."""
+    import babyvllm.kernels.paged_prefill as pp
+    from babyvllm.kernels.paged_attn import paged_decode_attention
+    from babyvllm.layers.linear import Linear
+
+    if path == "python":
+        python_path(monkeypatch)
+    if op == "decode":
+        args = make_decode_inputs([9000] + [40] * 39)
+        call = lambda: paged_decode_attention(*args, 0.1)
+        plain = lambda: paged_decode_attention(*args, 0.1, partition_blocks=0)
+    elif op == "prefill":
+        args = build_prefill_case([(6000, 150)], 4, 7, 128)
+        call = lambda: pp.paged_prefill_attention(*args, 0.1)
+
+        def plain():
+            with monkeypatch.context() as m:
+                python_path(m)
+                m.setattr(pp, "_split_tiles", lambda *a: 0)
+                return pp.paged_prefill_attention(*args, 0.1)
+    else:
+        lin = Linear(18944, 3584, bias=False).to("cuda", torch.bfloat16)
+        x = torch.randn(64, 18944, device="cuda", dtype=torch.bfloat16)
+        call = lambda: lin(x)
+        plain = lambda: torch.nn.functional.linear(x, lin.weight)
+    with torch.no_grad():
+        want, usual = plain(), call()
+        assert path == "python" and op == "linear" or not torch.equal(want, usual)  # (sums in another order)
+        del usual
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        out = torch.empty_like(want)
+        total = torch.cuda.get_device_properties(0).total_memory
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+        try:
+            rest = []  # all that is left of the reserved memory, but for the output's block
+            for size in (1 << 30, 1 << 26, 1 << 23, 1 << 21, 1100000):
+                while True:
+                    try:
+                        rest.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+                    except torch.OutOfMemoryError:
+                        break
+            del out
+            got = call()
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a ROCm GPU")
 def test_refused_calls_raise_as_before():
     from babyvllm.kernels._lib import KernelLibraryError
     from babyvllm.kernels.activation import fused_silu_mul
