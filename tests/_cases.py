@@ -128,6 +128,31 @@ def tuned(knob: int, value: int):
         _lib.set_tuning(knob, prev)
 
 
+def assert_linear_close(got, x, w, bias, gated):
+    """got against x @ w.T (+ bias), or silu(gate) * up, in float64, element by element and as a whole.
+
+    An fp32 sum of k bf16 products is off by at most k/2^24 of the sum of their magnitudes (eg, eu
+    for gate and up). It passes through silu(g)·u by |silu'| <= 1.1 and by the other factor; exp and
+    rcp add (|g| + 8)/2^23 of the value, the bf16 rounding 2^-8 of it. Roundings alone leave 1.7e-3
+    of the whole (rms), which a wrong or missing part of the sums exceeds long before single
+    elements leave their bounds.
+    """
+    import torch.nn.functional as F
+
+    k, n = x.shape[1], got.shape[1]
+    y = x.double() @ w.double().T
+    off = (x.double().abs() @ w.double().abs().T) * k * 2 ** -24
+    if gated:
+        g, u, eg, eu = y[:, :n], y[:, n:], off[:, :n], off[:, n:]
+        want = F.silu(g) * u
+        off = 1.1 * eg * (u.abs() + eu) + F.silu(g).abs() * eu + want.abs() * (g.abs() + 8) * 2 ** -23
+    else:
+        want = y if bias is None else y + bias.double()
+    diff = (got.double() - want).abs()
+    assert (diff <= want.abs() * 2 ** -8 + off + 1e-30).all()
+    assert diff.norm() <= 4e-3 * want.norm()
+
+
 class _Declining:
     """Stands in for the wrappers' native host side: every call takes the Python path."""
 

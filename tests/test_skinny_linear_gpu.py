@@ -2,7 +2,8 @@
 
 import pytest
 import torch
-import torch.nn.functional as F
+
+from tests._cases import assert_linear_close
 
 pytestmark = pytest.mark.gpu
 
@@ -25,14 +26,6 @@ SHAPES = [
 ]
 
 
-def _reference(x, w, bias, gated):
-    y = x.double() @ w.double().T
-    if gated:
-        n = w.shape[0] // 2
-        return F.silu(y[:, :n]) * y[:, n:]
-    return y if bias is None else y + bias.double()
-
-
 @pytest.mark.parametrize("m,n,k,gated", SHAPES)
 def test_values_against_float64(m, n, k, gated):
     from babyvllm.kernels.linear import gated_linear, skinny_linear
@@ -44,14 +37,7 @@ def test_values_against_float64(m, n, k, gated):
     with torch.no_grad():
         got = gated_linear(x, w) if gated else skinny_linear(x, w, bias)
     assert got is not None and got.shape == (m, n)
-    want = _reference(x, w, bias, gated)
-    # fp32 sums of k bf16 products: at most k/2^24 of the sum of magnitudes off, then one
-    # bf16 rounding (2^-8 of the value). silu·up doubles the relative part.
-    mag = x.double().abs() @ w.double().abs().T
-    if gated:
-        mag = mag[:, :n] * mag[:, n:]
-    bound = (2 if gated else 1) * (want.abs() * 2 ** -8 + mag * k * 2 ** -24) + 1e-30
-    assert ((got.double() - want).abs() <= bound).all()
+    assert_linear_close(got, x, w, bias, gated)
 
 
 def test_a_captured_call_takes_the_faster_kernel_on_the_gpu():
