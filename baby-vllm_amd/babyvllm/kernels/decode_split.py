@@ -19,6 +19,15 @@ The page count per split depends only on the batch rounded up to a power of
 two, and the split count only on the context bucket. An eager step (live
 lengths) and a graph step (bucket) therefore cut every row at the same pages,
 which is what lets the decode kernel return identical bits for both.
+
+That is also all a row's bits depend on for plans of several splits, for an
+explicit partition (0 among them: one work-group per row and KV head), and for
+"auto" plans of one split whose longest live row has at most 128 pages. An
+"auto" plan of one split with a longer row (and the decode rows of a prefill
+step, likewise) is balanced: the device cuts long rows into chunks by all of
+the batch's live lengths, so a row that is cut changes with the other rows'
+lengths, within the rounding of fp32 sums in another order. Eager and graph
+steps of the same batch still agree bit for bit.
 """
 
 from __future__ import annotations

@@ -6,6 +6,11 @@ one query token per sequence, GQA, pages read through the block table, and
 the flash-decoding split chosen by ``decode_split_plan`` from the context
 *bucket* (``max_seq_len``) and the batch's power-of-two bucket, never from the
 live lengths, so the launch is identical on every replay of a captured graph.
+Within it, a plan of one split with a bucket above ``BALANCE_MIN_PAGES`` lets the
+device cut rows of more than 128 pages into chunks by the live lengths of the whole
+batch: such a row's bits depend on the other rows' lengths too. ``partition_blocks=0``
+(or the environment's "0") keeps one work-group per row and KV head, whose bits
+depend on the row alone.
 
 The wrapper allocates the output and, for a split launch, the fp32 partial
 scratch through torch (so both land in a graph's private pool under capture),

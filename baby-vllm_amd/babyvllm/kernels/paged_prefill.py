@@ -5,6 +5,12 @@ signature and semantics: a flattened batch of sequences, each with
 ``context_lens[s]`` cached tokens plus ``q_len`` new query rows, causal, GQA,
 with K/V (prefix and new tokens alike) read from the paged cache through
 ``md.block_tables``. Decode rows (query length 1) may be mixed into the step.
+
+Few new tokens behind long prefixes run in key ranges, and long uneven decode rows
+in chunks, chosen from the step's host lists and the live lengths: the bits of such
+a sequence depend on the other sequences of the step, within the rounding of fp32
+sums in another order. Both take fp32 scratch (key ranges at most 64 MiB); without
+the memory for it the launch that needs none runs.
 """
 
 from __future__ import annotations

@@ -471,6 +471,17 @@ def test_balanced_bits_do_not_depend_on_the_bucket_or_other_columns(longest, mon
     assert torch.equal(live, _kernel()(q, kv_cache, bt, seq_lens, scale))
 
 
+def test_balanced_bits_do_not_depend_on_padded_rows(monkeypatch):
+    from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV
+
+    monkeypatch.delenv(DECODE_PARTITION_ENV, raising=False)
+    lens = [9000, 3000] + [60] * 35  # 37 live rows in a bucket of 64
+    q, kv_cache, bt, seq_lens = make_decode_inputs(lens + [0] * 27, seed=34)
+    padded = _kernel()(q, kv_cache, bt, seq_lens, HEAD_DIM ** -0.5)
+    live = _kernel()(q[:37], kv_cache, bt[:37], seq_lens[:37], HEAD_DIM ** -0.5)
+    assert torch.equal(padded[:37], live) and padded[37:].abs().max() == 0
+
+
 def test_balanced_launch_in_a_graph_follows_the_lengths(monkeypatch):
     from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV
 
