@@ -270,8 +270,9 @@ hipError_t launch_waves(const LinearArgs& a, hipStream_t s) {
 
 // Whether the kernel's call ends sooner than the library's, for n = 16 * tiles columns and
 // k = 128 * stages. Measured in graphs of back-to-back calls, weights from HBM, at 7,900 points:
-// 640 to 256000 columns, k 384 to 28672, 1 to 256 tokens. Of the 4,800 taken 19 in 20 are faster,
-// 22 more than a twentieth slower and none more than a tenth. The library's time jumps with its own choice of tiles, so
+// 640 to 256000 columns, k 384 to 28672, 1 to 256 tokens, and checked at 10,700 random ones (64
+// columns and k 128 up), 97% of which are faster and 0.6% more than a twentieth slower (3 of
+// them more than a tenth). The library's time jumps with its own choice of tiles, so
 // its good shapes lie between bad ones; where they do, the line leaves both to it. Lines and
 // figures (us, kernel / library):
 //   gated (the library's side includes its SiLU·mul launch): the kernel reads gate and up once
@@ -282,23 +283,26 @@ hipError_t launch_waves(const LinearArgs& a, hipStream_t s) {
 //     stages, 128 tokens 31.1 / 27.2);
 //   beyond 17 thousand k the library reads the weights at 1.1 to 1.4 TB/s (3584 x 18944: 16
 //     tokens 29 / 46, 64: 36 / 90, 256: 83 / 126; 4096 x 16384, 1 token 35.2 / 33.9, 17408 33.7 / 50.4);
+//   a k of 128 beyond 256 columns is two launches' latency either way (2680 columns, 6 tokens 4.0 /
+//     3.5);
 //   1 to 16 tokens: few rows are the kernel's at any k (16 tokens, 1152 x 896 4.7 / 6.8, 896 x
 //     8192 10.1 / 12.2); 160 to 255 tiles up to 35 stages (3584 x 4608 13.1 / 11.4, 4352 12.8 /
 //     17.1), 256 to 511 up to 51 (4096 x 6656 17.9 / 15.5), more columns up to 39 (12288 x 5120
 //     35.2 / 29.9);
 //   17 to 32: 160 to 255 tiles lose from 40 stages (32 tokens, 3584 x 5120 17.0 / 15.8), 288 to
 //     320 nowhere (4608 x 3584 0.95 times), the rest of 256 to 511 from 28 or 18 (4096 x 3840
-//     14.4 / 13.0, 7168 x 2304 11.7 / 11.2), more columns from 9 (10240 x 1280 12.4 / 10.9), 1184
-//     tiles and more at once (18944 x 1536 21.8 / 18.9);
+//     14.4 / 13.0, 7168 x 2304 11.7 / 11.2), more columns from 9 (10240 x 1280 12.4 / 10.9), 1024
+//     tiles and more at once (17032 x 640, 23 tokens 13.6 / 11.5, 28672 x 896 21.3 / 15.8);
 //   33 to 64: x outweighs the weights of few rows per work-group. Below 160 tiles the lines
 //     follow the library's jumps (2048 x 2560, 33 tokens 11.1 / 9.3, 1280 x 5632, 48: 12.8 / 10.6,
-//     896 x 896 0.77 times, 896 x 4864 0.70); 256 to 287 tiles up to 20 stages (4096 x 3072, 48
-//     tokens 14.7 / 11.4), 288 to 511 up to 29 (4608 x 3584 0.89 times; 4608 x 4096, 48 tokens
-//     18.3 / 22.7, 64: 19.4 / 17.8), none beyond (12288 x 3584, 33 tokens 32.6 / 23.1);
-//   65 to 128: from 80, 56 or 28 stages with the row tiles (896 x 8192, 65 tokens 14.8 / 13.3;
-//     2560 x 6656 18.8 / 19.1; 3584 x 3584 0.95 times), 256 to 320 tiles but for 32 to 43 stages
-//     (5120 x 4096, 65 tokens 19.7 / 17.2, 5632 23.7 / 23.0; 4608 x 3584 1.01 times), up to 511
-//     from 64;
+//     92 x 1792, 33: 8.6 / 7.3, 896 x 896 0.77 times, 896 x 4864 0.70); 256 to 287 tiles up to 20
+//     stages (4096 x 3072, 48 tokens 14.7 / 11.4), 288 to 511 up to 29 (4608 x 3584 0.89 times;
+//     4608 x 4096, 48 tokens 18.3 / 22.7, 64: 19.4 / 17.8), none beyond (12288 x 3584, 33 tokens
+//     32.6 / 23.1);
+//   65 to 128: below 192 tiles from 80 or 56 stages (896 x 8192, 65 tokens 14.8 / 13.3; 2560 x
+//     6656 18.8 / 19.1), 192 to 320 tiles but for 32 to 43 or 47 (5120 x 4096, 65 tokens 19.7 /
+//     17.2, 5632 23.7 / 23.0, 3148 x 4864, 119: 22.6 / 19.8; 3584 x 3584 0.95 times, 4608 x 3584
+//     1.01), up to 511 from 64;
 //   heads (2048 tiles and more) are within a tenth of each other but for the library's bad
 //     sizes (100352 x 896, 17 tokens 42 / 126; 152064 x 3584, 16 tokens 188 / 231): below 32
 //     stages, up to 16 tokens; from 4096 tiles up to 32, and to 64 for at most 8 stages (50304 x 896, 48
@@ -316,9 +320,11 @@ static bool ends_sooner(int m, int tiles, int stages, bool gated, bool eager, do
     if (m <= 16) return stages < 36 || (tiles >= 224 && stages < 64);
     if (m <= 32) return stages < 36 || (tiles >= 352 && stages < 64);
     if (m <= 64) return stages < 18 || (tiles >= 176 && stages < 36) || (tiles >= 560 && stages < 64);
-    if (m <= 128 && tiles < 1100 && (stages <= 8 || (tiles >= 300 && stages <= 12))) return true;
+    if (m <= 128 && tiles < 1100 && (stages <= 4 || (tiles >= 64 && stages <= 8) || (tiles >= 300 && stages <= 12)))
+      return true;
     return eager && stages <= (m <= 128 ? 12 : 8) && products <= 2.4e9;
   }
+  if (stages < 2 && tiles > 16 && tiles < 2048) return false;
   if (tiles >= 2048)
     return m <= 64 && stages < 32 && tiles <= 12800 && (m <= 16 || (tiles >= 4096 && (m <= 32 || stages <= 8)));
   if (stages >= 136 && tiles < 512) return true;
@@ -327,12 +333,13 @@ static bool ends_sooner(int m, int tiles, int stages, bool gated, bool eager, do
     if (tiles < 160) return stages < 44 || stages >= 52;
     if (tiles < 256) return stages < 40 || stages >= 64;
     if (tiles >= 288 && tiles <= 320) return true;
-    return stages < (tiles < 288 ? 28 : tiles < 512 ? 18 : tiles < 1184 ? 9 : 0);
+    if (tiles >= 512) return tiles < 1024 && stages >= 3 && stages < 9;
+    return stages < (tiles < 288 ? 28 : 18);
   }
   if (m <= 64) {
     if (tiles < 512 && stages > 64) return true;
     if (tiles < 160)
-      return (stages >= 6 && stages <= 8) || (stages >= 12 && stages <= 16) ||
+      return (stages >= 6 && stages <= 8) || (tiles >= 40 && stages >= 12 && stages <= 16) ||
              (stages >= 32 && stages <= (tiles < 96 ? 40 : 63));
     if (tiles < 256) return false;
     if (tiles < 288) return stages <= 20;
@@ -340,8 +347,9 @@ static bool ends_sooner(int m, int tiles, int stages, bool gated, bool eager, do
   }
   if (eager && tiles <= 320 && stages >= 28 && stages < 64 && products <= 4.5e8) return true;
   if (m <= 128) {
-    if (tiles < 256) return stages >= (tiles < 160 ? 80 : tiles < 192 ? 56 : 28);
-    return tiles < 512 && (stages >= 64 || (tiles <= 320 && ((stages >= 28 && stages < 32) || stages >= 44)));
+    if (tiles < 192) return stages >= (tiles < 160 ? 80 : 56);
+    return tiles < 512 &&
+           (stages >= 64 || (tiles <= 320 && ((stages >= 28 && stages < 32) || stages >= (tiles < 256 ? 48 : 44))));
   }
   return false;
 }

@@ -108,11 +108,11 @@ def test_linear_leaves_the_library_the_shapes_it_is_faster_at():
     """Points measured on both sides of every line of the rule (k and columns of no one model)."""
     takes = lambda m, n, k, gated=0, eager=0: _lib().lib().bvllm_linear_workspace_bytes(m, n, k, gated, eager) >= 0
     kernel = [(16, 1152, 896), (1, 4096, 17408), (16, 3584, 4352), (32, 4608, 4096), (33, 896, 896), (48, 4608, 4096),
-              (64, 1536, 5632), (64, 5120, 3584), (128, 3584, 4608), (128, 3584, 8192), (256, 3584, 18944),
+              (64, 1536, 5632), (64, 5120, 3584), (128, 3584, 6656), (128, 3584, 8192), (256, 3584, 18944),
               (16, 32768, 2048), (17, 100352, 896), (1, 13824, 4608, 1), (64, 4864, 2048, 1), (128, 8960, 1536, 1)]
     library = [(16, 3584, 5120), (16, 12288, 8192), (8, 4096, 8192), (1, 32768, 4096), (32, 12288, 2560), (32, 18944, 896),
                (33, 2048, 2560), (33, 12288, 896), (64, 18944, 3584), (64, 4608, 4096), (65, 896, 8192),
-               (128, 896, 4864), (128, 2048, 3584), (128, 18944, 8192), (192, 896, 4864), (256, 3584, 8192),
+               (128, 896, 4864), (128, 3148, 4864), (128, 2048, 3584), (6, 2680, 128), (33, 92, 1792), (128, 256, 1024, 1), (128, 18944, 8192), (192, 896, 4864), (256, 3584, 8192),
                (208, 6144, 8960), (48, 50304, 896), (16, 256000, 896), (1, 1024, 6144, 1), (33, 2048, 3584, 1),
                (128, 18944, 896, 1), (192, 2048, 1536, 1), (160, 4864, 896, 1), (256, 4864, 896, 1)]
     assert [p for p in kernel if not takes(*p)] == [] and [p for p in library if takes(*p)] == []

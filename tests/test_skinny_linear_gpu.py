@@ -22,7 +22,7 @@ SHAPES = [
     (1, 64, 128, True), (16, 4864, 896, True), (33, 4868, 896, True), (64, 8192, 384, True), (64, 8196, 384, True),
     (16, 18944, 3584, True), (17, 9000, 640, True),
     (65, 4864, 896, True), (97, 8964, 1536, True), (128, 64, 128, True), (129, 4868, 896, True), (192, 4864, 896, True),
-    (256, 4864, 896, True), (65, 896, 4864, False), (65, 3588, 4864, False), (96, 3588, 3584, False), (128, 5120, 3584, False),
+    (256, 4864, 896, True), (65, 896, 4864, False), (65, 3588, 6272, False), (96, 3588, 3584, False), (128, 5120, 3584, False),
 ]
 
 
