@@ -42,12 +42,12 @@ struct DecodeArgs {
   int32_t splits_per_item;                 // consecutive splits one streaming wave computes
   int32_t num_partials;                    // partial states per (row, head) the launch writes
   int32_t ws_partials;                     // partial states per (row, head) the workspace holds
-  int32_t item_order;                      // numbering: 0 KV head, row, unit (fastest first); 1 unit, KV head, row;
-                                           // 2 as 0 with each row's units together and the empty ones last
+  int32_t item_order;                      // numbering: 0 KV head, unit, row (fastest first); 1 unit, KV head, row;
+                                           // 2 as 0 with the empty units last
   // Balanced single pass (RowChunk): chunks aimed at per column group, rows an even
   // share of which keeps every CU busy.
   int32_t chunk_target, row_slots;
-  FastDiv by_col_groups, by_batch;         // of item orders 0 and 2
+  FastDiv by_col_groups, by_units;         // of item orders 0 and 2
   // Prefill view (both null for a decode batch): row b is sequence b of a
   // varlen prefill batch. Only sequences with exactly one query token are
   // computed; their q / out row is query_start_loc[b] and they attend keys

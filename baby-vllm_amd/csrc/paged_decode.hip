@@ -342,7 +342,7 @@ DecodePlan decode_plan(int32_t batch, int32_t num_kv_heads, int32_t head_dim, in
   p.quad = group_mode ? forced == 5 || (forced != 2 && forced != 3 && long_groups &&
                                         (head_dim == 64 || blocks_per_split >= 64))
                       : p.pair && blocks_per_split <= 64 && forced != 4;
-  p.live_first = p.pair && group_mode && long_groups && batch > 1;
+  p.live_first = p.pair && batch > 1 && (group_mode ? long_groups : blocks_per_split > 32);
   return p;
 }
 
@@ -463,7 +463,7 @@ static hipError_t launch_decode(const DecodeArgs& args, hipStream_t stream) {
   const int64_t items = (int64_t)a.batch * decode_col_groups(a) * units;
   if (items > 0x7ffffff0) return hipErrorInvalidValue;
   a.by_col_groups = fast_div((int32_t)ncg);
-  a.by_batch = fast_div(a.batch);
+  a.by_units = fast_div((int32_t)units);
   hipError_t err;
   if (p.quad && a.splits_per_item > 1) {
     err = launch_quad_group_vgpr(a, items, tuning(kTuneDecodeCached) == 0, stream);

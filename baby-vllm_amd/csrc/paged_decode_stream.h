@@ -95,10 +95,12 @@ constexpr int kPairLdsFloats = 4 * kPairRecFloats<D>;
 // Item order 2: the units with a live page first, row by row, then the empty ones (which
 // only write empty partials). Work-groups that end at once shift the dispatcher's
 // round, and it then puts two or three live ones on some CUs while others idle; with
-// the empty ones last the live ones are dealt evenly. For groups of long splits, where
-// a second group on a CU costs far more than the round trip of finding the unit (12
-// rows of 100 to 32768, two waves per group of 64 pages: 55 -> 40 us; two rows of 16000
-// among 18 of 16, four waves: 49 -> 32; equal rows lose about 1 us: 32 x 16000 169 -> 170).
+// the empty ones last the live ones are dealt evenly. For groups of long splits and splits
+// of more than 32 pages, where a second unit on a CU costs far more than the round trip of
+// finding the unit (12 rows of 100 to 32768, two waves per group of 64 pages: 55 -> 40 us;
+// 61 rows of 393 to 8625, one KV head, splits of 64 pages: 38.7 -> 24.0; equal rows lose
+// about 1 us: 32 x 16000 169 -> 170). Below that the round trip is what it costs (splits
+// of at most 16 pages: 4% on average, ragged or equal).
 __device__ __forceinline__ void find_live_unit(const DecodeArgs& a, int t, int units, int unit_pages, int& b_out,
                                                int& unit_out) {
   const int lane = lane_id();
@@ -154,25 +156,21 @@ __device__ __forceinline__ void decode_stream_wave(const DecodeArgs& a, const in
   // Column groups: the KV heads, or their 16-head parts when G > 16 (ColGroup).
   const int ncg = a.num_kv_heads * col_groups_per_kv(a.num_heads / a.num_kv_heads);
   int cg, unit, b;
-  if (GROUP && a.item_order == 2) {
+  if (a.item_order == 2) {
     const int rest = a.by_col_groups(item);
     cg = item - rest * ncg;
     find_live_unit(a, rest, units, spi * a.blocks_per_split, b, unit);
   } else if (a.item_order == 0) {
-    // KV head fastest, then the row, then the unit: the first units of every row come
-    // first and units past the end of short rows last, so that the live work-groups
-    // are dealt evenly to the CUs (empty ones between them leave some CUs with two or
-    // three and others with none). The row is shifted by the unit, since work-groups
-    // go round-robin to the 8 XCDs and a row's units must not all meet on one (rows'
-    // units next to each other put the first unit of every row on the same XCDs: 64
-    // rows of 200 to 8192, 2 KV heads of 64: 34.4 -> 29.4 us). The divisions stand before the
-    // first load: by multiplication they cost a short launch nothing (8 x 1920: 14.8 us with
-    // divide instructions, 14.1 so, 14.4 row by row with divides, 14.2 row by row so).
+    // KV head fastest, then the unit, then the row: a row's units are dealt to all XCDs.
+    // (Units before rows, the row shifted by the unit, puts the first units of all rows
+    // first and the empty ones last: over 6,000 random ragged batches of splits of at most 32
+    // pages and short groups no faster on average, 7% slower and more in one of 20 and up to
+    // 32%.) The divisions stand before the first load: by multiplication they cost a short
+    // launch nothing (8 x 1920: 14.4 us with divide instructions, 14.2 so).
     const int rest = a.by_col_groups(item);
     cg = item - rest * ncg;
-    unit = a.by_batch(rest);
-    b = rest - unit * a.batch - (unit - a.by_batch(unit) * a.batch);
-    if (b < 0) b += a.batch;
+    b = a.by_units(rest);
+    unit = rest - b * units;
   } else {  // unit fastest
     unit = item % units;
     const int rest = item / units;
