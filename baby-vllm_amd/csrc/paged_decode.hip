@@ -340,7 +340,8 @@ DecodePlan decode_plan(int32_t batch, int32_t num_kv_heads, int32_t head_dim, in
                ? (forced == 3 || forced == 5 || (forced != 2 && (long_groups || group_items <= 2 * (int64_t)device_cus())))
                : forced != 1;
   p.quad = group_mode ? forced == 5 || (forced != 2 && forced != 3 && long_groups &&
-                                        (head_dim == 64 || blocks_per_split >= 64))
+                                        (head_dim == 64 || blocks_per_split >= 64 ||
+                                         group_items > 2 * (int64_t)device_cus()))
                       : p.pair && blocks_per_split <= 64 && forced != 4;
   p.live_first = p.pair && batch > 1 && (group_mode ? long_groups : blocks_per_split > 32);
   return p;

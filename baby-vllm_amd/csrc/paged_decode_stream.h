@@ -641,9 +641,11 @@ __global__ __launch_bounds__(256) void paged_decode_quad_kernel(DecodeArgs a, in
 // Four waves per group of splits (one state each, two pages in flight): the groups
 // of long splits at D = 64, where one or two waves read too little at a time to keep
 // a CU's share of HBM busy (36 rows of 100 to 32000, groups of 256 pages: one wave 128
-// us, two 68, four 43; 16 x 16000: two 29.7, four 28.1), and of 64 pages and more.
-// At D = 128 two waves do as well (24 rows of 100 to 32768: one wave 94, two 67, four
-// 74; 20 of 200 to 16000: 89, 47, 40; 32 x 16000: 177, 170.6, 171.4).
+// us, two 68, four 43; 16 x 16000: two 29.7, four 28.1), of 64 pages and more, and at
+// D = 128 launches of more than two groups per CU, where two waves leave the groups beyond
+// the first round nearly alone on the card (20 x 10313, 4 KV heads, splits of 16 pages, 880
+// groups: one wave 107, two 126, four 108 us; 20 rows of 200 to 16000: 89, 47, 40). Up to
+// two groups per CU two waves are 5 to 18% faster there on equal rows.
 template <int D, bool NT>
 __global__ __launch_bounds__(256) void paged_decode_quad_group_kernel(DecodeArgs a, int items) {
   __shared__ __attribute__((aligned(16))) unsigned char tile[4 * kTileBytes<D>];
