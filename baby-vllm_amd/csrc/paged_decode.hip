@@ -335,6 +335,7 @@ DecodePlan decode_plan(int32_t batch, int32_t num_kv_heads, int32_t head_dim, in
   // -> 18.2 us), one beyond (8 x 16384, 1024 groups: 52.8 against 56.4 us on two waves;
   // 4 x 32768, 2048 groups: 60.0 against 64.3 us).
   const int64_t group_items = (int64_t)batch * num_kv_heads * groups;
+  const int64_t split_items = (int64_t)batch * num_kv_heads * num_splits;
   const bool long_groups = blocks_per_split >= 16;
   p.pair = group_mode
                ? (forced == 3 || forced == 5 || (forced != 2 && (long_groups || group_items <= 2 * (int64_t)device_cus())))
@@ -343,7 +344,10 @@ DecodePlan decode_plan(int32_t batch, int32_t num_kv_heads, int32_t head_dim, in
                                         (head_dim == 64 || blocks_per_split >= 64 ||
                                          group_items > 2 * (int64_t)device_cus()))
                       : p.pair && blocks_per_split <= 64 && forced != 4;
-  p.live_first = p.pair && batch > 1 && (group_mode ? long_groups : blocks_per_split > 32);
+  // Live units first (see find_live_unit); single splits only where a CU can get a second one
+  // (with one per CU at most the round trip costs 3 to 4% and there is nothing to even out).
+  p.live_first = p.pair && batch > 1 &&
+                 (group_mode ? long_groups : blocks_per_split > 32 && split_items > device_cus());
   return p;
 }
 
