@@ -22,9 +22,9 @@ which is what lets the decode kernel return identical bits for both.
 
 That is also all a row's bits depend on for plans of several splits, for an
 explicit partition (0 among them: one work-group per row and KV head), and for
-"auto" plans of one split whose longest live row has at most 128 pages. An
-"auto" plan of one split with a longer row (and the decode rows of a prefill
-step, likewise) is balanced: the device cuts long rows into chunks by all of
+"auto" plans of one split whose longest live row has at most 128 pages or whose
+rows and KV heads are more than two per CU. Any other "auto" plan of one split
+(and the decode rows of a prefill step, likewise) is balanced: the device cuts long rows into chunks by all of
 the batch's live lengths, so a row that is cut changes with the other rows'
 lengths, within the rounding of fp32 sums in another order. Eager and graph
 steps of the same batch still agree bit for bit.
@@ -44,7 +44,7 @@ def _ceil_div(a: int, b: int) -> int:
     return -(-a // b)
 
 
-def _pow2_at_least(n: int) -> int:
+def pow2_at_least(n: int) -> int:
     p = 1
     while p < n:
         p <<= 1
@@ -57,12 +57,12 @@ def auto_partition_blocks(batch: int) -> int:
     A function of the batch's power-of-two bucket only, so every live batch
     size inside one graph bucket gets the same partition.
     """
-    return max(MIN_PARTITION_BLOCKS, _pow2_at_least(batch))
+    return max(MIN_PARTITION_BLOCKS, pow2_at_least(batch))
 
 
 def grid_fills_gpu(batch: int, n_kv_heads: int, num_sms: int) -> bool:
     """True when one work-group per (bucketed row, KV head) already covers ``num_sms`` units."""
-    return _pow2_at_least(batch) * n_kv_heads >= num_sms
+    return pow2_at_least(batch) * n_kv_heads >= num_sms
 
 
 def decode_split_plan(

@@ -6,8 +6,8 @@ one query token per sequence, GQA, pages read through the block table, and
 the flash-decoding split chosen by ``decode_split_plan`` from the context
 *bucket* (``max_seq_len``) and the batch's power-of-two bucket, never from the
 live lengths, so the launch is identical on every replay of a captured graph.
-Within it, a plan of one split with a bucket above ``BALANCE_MIN_PAGES`` lets the
-device cut rows of more than 128 pages into chunks by the live lengths of the whole
+Within it, a plan of one split with a bucket above ``BALANCE_MIN_PAGES`` and at most two
+walks per CU (``balance_pays``) lets the device cut rows of more than 128 pages into chunks by the live lengths of the whole
 batch: such a row's bits depend on the other rows' lengths too. ``partition_blocks=0``
 (or the environment's "0") keeps one work-group per row and KV head, whose bits
 depend on the row alone.
@@ -26,13 +26,25 @@ import os
 import torch
 
 from babyvllm.kernels import _lib
-from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV, MIN_PARTITION_BLOCKS, decode_split_plan
+from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV, MIN_PARTITION_BLOCKS, decode_split_plan, pow2_at_least
 
 # A single-pass plan ("auto") sized for more pages than this runs the balanced launch
 # (bvllm_paged_decode_balanced). Shorter rows can lose less to each other than its second
 # launch costs equal ones (64 x 2048: 45.1 against 46.4 us; 64 rows of 200 to 2048: 30.2
 # against 27.1; 64 of 100 to 4096: 52 against 34; 64 x 4096: 86.7 against 87.7).
 BALANCE_MIN_PAGES = 128
+
+
+def balance_pays(batch: int, n_heads: int, n_kv_heads: int, num_sms: int) -> bool:
+    """At most two walks of a (row, 16 query heads of a KV head) per CU, so that one can be
+    left alone on the card. With more, the plain launch evens the rows out by itself: over
+    random batches of up to two per CU the balanced one takes 0.54 to 0.91 of its time on
+    ragged rows, beyond 2.5 it is 2% slower on average and never pays (160 rows, 4 KV heads).
+    The batch counts as the next power of two, as in the plan, so that an eager step and its
+    graph agree."""
+    if n_kv_heads < 1 or n_heads % n_kv_heads:
+        return False
+    return pow2_at_least(batch) * n_kv_heads * -(-n_heads // n_kv_heads // 16) <= 2 * num_sms
 
 
 @functools.lru_cache(maxsize=None)
@@ -98,6 +110,7 @@ def paged_decode_attention(q, kv_cache, block_tables, seq_lens, scale,
         out.data_ptr(), out.stride(0), out.stride(1),
     )
     balanced = num_splits == 1 and blocks_per_split > BALANCE_MIN_PAGES and partition_blocks is None \
+        and balance_pays(B, n_heads, n_kv_heads, _num_sms(_device_index(q))) \
         and B * width <= _lib.BALANCED_MAX_PAGES and os.environ.get(DECODE_PARTITION_ENV, "auto") == "auto"
     workspace = None
     if balanced:

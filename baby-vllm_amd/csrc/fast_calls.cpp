@@ -245,6 +245,12 @@ PyObject* fast_auto_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return Py_BuildValue("LL", (long long)p.splits, (long long)p.pages);
 }
 
+// balance_pays (babyvllm/kernels/paged_attn.py).
+bool balance_pays(int64_t batch, int64_t heads, int64_t hkv, int64_t cus) {
+  if (hkv < 1 || heads % hkv != 0) return false;
+  return pow2_at_least(batch) * hkv * cdiv(heads / hkv, 16) <= 2 * cus;
+}
+
 // (q, kv_cache, block_tables, seq_lens, scale, max_seq_len | None, cus, min_pages, balance_min_pages,
 //  partition env name, device, stream): the "auto" plan
 PyObject* fast_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -276,7 +282,8 @@ PyObject* fast_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (env != nullptr && std::strcmp(env, "auto") != 0) return none();
   const Plan p = auto_plan(batch, hkv, c->size(2), width, max_seq_len, cus, min_pages);
   if (!small(p.splits) || !small(p.pages)) return none();
-  bool balanced = p.splits == 1 && p.pages > balance && batch * width <= BVLLM_BALANCED_MAX_PAGES;
+  bool balanced = p.splits == 1 && p.pages > balance && batch * width <= BVLLM_BALANCED_MAX_PAGES &&
+                  balance_pays(batch, heads, hkv, cus);
   at::Tensor out = new_empty({batch, heads, d}, *q, at::kBFloat16), ws;
   if (balanced) {
     const int64_t bytes = g.balanced_bytes((int32_t)batch, (int32_t)heads, (int32_t)hkv, (int32_t)d);

@@ -482,6 +482,31 @@ def test_balanced_bits_do_not_depend_on_padded_rows(monkeypatch):
     assert torch.equal(padded[:37], live) and padded[37:].abs().max() == 0
 
 
+@pytest.mark.parametrize("rows,hkv,group,cut", [(65, 4, 7, True), (128, 4, 7, True), (129, 4, 7, False),
+                                                (64, 4, 20, True), (65, 4, 20, False)])
+def test_balanced_up_to_two_walks_per_cu(rows, hkv, group, cut, monkeypatch):
+    """Beyond two walks of 16 query heads per CU (on 256 CUs) the plain single pass runs: its bits,
+    from the native wrapper and from the Python one (which an int subclass takes)."""
+    from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV
+
+    monkeypatch.delenv(DECODE_PARTITION_ENV, raising=False)
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes of a card with 256 CUs")
+
+    class Int(int):
+        pass
+
+    lens = [5000] + [1 + 3 * i for i in range(rows - 1)]
+    q, kv_cache, bt, seq_lens = make_decode_inputs(lens, hkv=hkv, group=group, seed=35)
+    scale = HEAD_DIM ** -0.5
+    single = _kernel()(q, kv_cache, bt, seq_lens, scale, max_seq_len=5000, partition_blocks=0)
+    outs = [_kernel()(q, kv_cache, bt, seq_lens, scale, max_seq_len=n) for n in (5000, Int(5000))]
+    assert torch.equal(outs[0], outs[1])
+    assert torch.equal(outs[0][1:], single[1:])  # at most 24 pages: whole
+    assert torch.equal(outs[0][0], single[0]) != cut
+    assert_attn_close(outs[0], _oracle(q, kv_cache, bt, lens, scale))
+
+
 def test_balanced_launch_in_a_graph_follows_the_lengths(monkeypatch):
     from babyvllm.kernels.decode_split import DECODE_PARTITION_ENV
 
