@@ -96,7 +96,7 @@ SIGNATURES = {
         _p, _i32, _i32, _i32, _p,   # workspace, split_tiles, num_ranges, balance_rows, stream
     ]),
     "bvllm_prefill_split_tiles": (ctypes.c_int32, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i64, _i64]),
-    "bvllm_prefill_balance_rows": (ctypes.c_int32, [_i32, _i32, _i64, _i64]),
+    "bvllm_prefill_balance_rows": (ctypes.c_int32, [_i32, _i32, _i64, _i64, _i64]),
     "bvllm_prefill_ranges": (ctypes.c_int32, [_i32, _i32, _i64]),
     "bvllm_prefill_workspace_bytes": (ctypes.c_int64, [_i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "bvllm_set_tuning": (ctypes.c_int, [_i32, _i32]),
@@ -127,7 +127,7 @@ SIGNATURES = {
     ]),
 }
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 
 # Pages (rows · table width) that the balanced launches take.

@@ -65,13 +65,19 @@ def _split_tiles(md, num_seqs, num_tokens, single, num_heads, num_kv_heads, head
                                                 num_kv_heads, head_dim, width, tiles, longest)
 
 
-def _balance_rows(md, num_seqs, num_heads, num_kv_heads):
-    """Whether the single-query rows are cut into chunks (also a choice by the host lists)."""
+def _balance_rows(md, num_seqs, num_heads, num_kv_heads, split_tiles=0):
+    """Whether the single-query rows are cut into chunks (also a choice by the host lists);
+    ``split_tiles`` is the key range that the other sequences are cut into, 0 if they are whole."""
     qsl, seq = getattr(md, "query_start_loc_cpu", None), getattr(md, "seq_lens_cpu", None)
     if qsl is None or seq is None or len(seq) != num_seqs or len(qsl) != num_seqs + 1:
         return 0
     pages = [(int(seq[i]) + 15) // 16 for i in range(num_seqs) if qsl[i + 1] - qsl[i] == 1]
-    return _lib.lib().bvllm_prefill_balance_rows(num_heads, num_kv_heads, max(pages), sum(pages)) if pages else 0
+    if not pages:
+        return 0
+    tiles = _key_tiles(md, num_seqs, num_heads, num_kv_heads)[1]
+    if split_tiles > 0:
+        tiles = min(split_tiles, tiles)
+    return _lib.lib().bvllm_prefill_balance_rows(num_heads, num_kv_heads, max(pages), sum(pages), tiles)
 
 
 def paged_prefill_attention(q, kv_cache, md, scale):
@@ -133,7 +139,7 @@ def paged_prefill_attention(q, kv_cache, md, scale):
     h = _lib.lib()
     balance = 0
     if single > 0 and num_seqs * bt.shape[1] <= _lib.BALANCED_MAX_PAGES:
-        balance = _balance_rows(md, num_seqs, num_heads, num_kv_heads)
+        balance = _balance_rows(md, num_seqs, num_heads, num_kv_heads, split_tiles)
     workspace = None
     if split_tiles > 0 or balance:
         ranges = 0

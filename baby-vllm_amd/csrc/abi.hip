@@ -260,9 +260,9 @@ extern "C" int32_t bvllm_prefill_split_tiles(int32_t num_seqs, int32_t num_token
 }
 
 extern "C" int32_t bvllm_prefill_balance_rows(int32_t num_heads, int32_t num_kv_heads, int64_t longest_pages,
-                                              int64_t total_pages) {
+                                              int64_t total_pages, int64_t prefill_tiles) {
   if (!valid_heads(num_heads, num_kv_heads) || longest_pages < 1 || total_pages < 1) return 0;
-  return prefill_balance_rows(num_heads, num_kv_heads, longest_pages, total_pages) ? 1 : 0;
+  return prefill_balance_rows(num_heads, num_kv_heads, longest_pages, total_pages, prefill_tiles) ? 1 : 0;
 }
 
 extern "C" int32_t bvllm_prefill_ranges(int32_t max_blocks, int32_t split_tiles, int64_t longest_tiles) {

@@ -158,8 +158,10 @@ int64_t decode_chunk_slots(int32_t batch, int32_t num_heads, int32_t num_kv_head
 void decode_set_chunks(DecodeArgs& a);
 hipError_t decode_merge_chunks(const DecodeArgs& a, hipStream_t stream);
 // Whether a prefill batch's single-query rows (the longest and all of their pages) are
-// uneven enough that cutting them pays for the merge.
-bool prefill_balance_rows(int32_t num_heads, int32_t num_kv_heads, int64_t longest, int64_t total);
+// uneven enough, and long enough beside the other work-groups' key tiles, that cutting them
+// pays for the merge.
+bool prefill_balance_rows(int32_t num_heads, int32_t num_kv_heads, int64_t longest, int64_t total,
+                          int64_t prefill_tiles);
 
 // How a decode launch with the caller's split plan runs (paged_decode.hip).
 struct DecodePlan {

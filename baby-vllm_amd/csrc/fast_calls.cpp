@@ -337,8 +337,7 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!PyList_CheckExact(a[6]) || PyList_GET_SIZE(a[6]) != seqs + 1) return none();
   const bool lens_known = PyList_CheckExact(a[7]) && PyList_GET_SIZE(a[7]) == seqs;
   const int64_t split_min = PyLong_AsLongLong(a[10]);
-  const bool may_split = width >= split_min;
-  int64_t single = 0, tiles = may_split && lens_known ? 0 : -1, prev = 0, longest = 0, pages = 0;
+  int64_t single = 0, tiles = lens_known ? 0 : -1, prev = 0, longest = 0, pages = 0;
   int64_t longest_tiles = tiles;
   for (int64_t i = 0; i <= seqs; ++i) {
     PyObject* o = PyList_GET_ITEM(a[6], i);
@@ -356,7 +355,7 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (m == 1) {
           longest = std::max(longest, cdiv(len, 16));
           pages += cdiv(len, 16);
-        } else if (m > 1 && may_split) {
+        } else if (m > 1) {
           tiles += cdiv(m * (heads / hkv), 128) * cdiv(len, 64);
           longest_tiles = std::max(longest_tiles, cdiv(len, 64));
         }
@@ -370,11 +369,14 @@ PyObject* fast_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* stream = PyLong_AsVoidPtr(a[12]);
   if (PyErr_Occurred()) return nullptr;
   if (!small(max_q)) return none();
-  int32_t split = !may_split ? 0
-                                   : g.split_tiles((int32_t)seqs, (int32_t)tokens, (int32_t)max_q, (int32_t)single,
-                                                   (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)width, tiles,
-                                                   longest_tiles);
-  int32_t balance = pages > 0 && seqs * width <= BVLLM_BALANCED_MAX_PAGES ? g.balance_rows((int32_t)heads, (int32_t)hkv, longest, pages) : 0;
+  int32_t split = width < split_min ? 0
+                                    : g.split_tiles((int32_t)seqs, (int32_t)tokens, (int32_t)max_q, (int32_t)single,
+                                                    (int32_t)heads, (int32_t)hkv, (int32_t)d, (int32_t)width, tiles,
+                                                    longest_tiles);
+  int32_t balance = 0;
+  if (pages > 0 && seqs * width <= BVLLM_BALANCED_MAX_PAGES)
+    balance = g.balance_rows((int32_t)heads, (int32_t)hkv, longest, pages,
+                             split > 0 ? std::min<int64_t>(split, longest_tiles) : longest_tiles);
   const int32_t ranges = split > 0 ? g.ranges((int32_t)width, split, longest_tiles) : 0;
   at::Tensor out = new_empty({tokens, heads, d}, *q, at::kBFloat16), ws;
   if (split > 0 || balance) {

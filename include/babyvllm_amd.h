@@ -40,7 +40,7 @@ extern "C" {
 #endif
 
 /* ABI version of this header; bumped on any signature change. */
-#define BVLLM_ABI_VERSION 9
+#define BVLLM_ABI_VERSION 10
 
 #if defined(__GNUC__)
 #define BVLLM_API __attribute__((visibility("default")))
@@ -221,7 +221,9 @@ BVLLM_API int bvllm_paged_prefill(const void* q, int64_t q_stride_t, int64_t q_s
  * (of the table's width if longest_tiles is -1); the last range of a launch runs to the
  * row's end, so any num_ranges from 1 to that of the width computes every key.
  * bvllm_prefill_balance_rows returns whether cutting pays, from the pages of the longest
- * single-query row and of all of them. All three steer the choice only, never what is
+ * single-query row and of all of them and from the 64-key tiles that the longest other
+ * work-group walks (prefill_tiles: longest_tiles, or split_tiles where that is smaller and
+ * not 0; 0 without other sequences). All three steer the choice only, never what is
  * computed. workspace holds bvllm_prefill_workspace_bytes() bytes (num_ranges 0 without
  * key ranges; partials of the ranges that bvllm_prefill_split_tiles chooses are at most
  * 64 MiB). Results agree with bvllm_paged_prefill within the rounding of fp32 sums in
@@ -231,7 +233,7 @@ BVLLM_API int32_t bvllm_prefill_split_tiles(int32_t num_seqs, int32_t num_tokens
                         int32_t single_query_seqs, int32_t num_heads, int32_t num_kv_heads,
                         int32_t head_dim, int32_t max_blocks, int64_t key_tiles, int64_t longest_tiles);
 BVLLM_API int32_t bvllm_prefill_balance_rows(int32_t num_heads, int32_t num_kv_heads, int64_t longest_pages,
-                        int64_t total_pages);
+                        int64_t total_pages, int64_t prefill_tiles);
 BVLLM_API int32_t bvllm_prefill_ranges(int32_t max_blocks, int32_t split_tiles, int64_t longest_tiles);
 BVLLM_API int64_t bvllm_prefill_workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t num_heads,
                         int32_t num_kv_heads, int32_t head_dim, int32_t num_ranges,

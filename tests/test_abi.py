@@ -182,6 +182,15 @@ def test_balanced_launches_refuse_more_pages_than_they_can_add_up():
                                            3584, 128, batch, batch, 1, batch, 28, 4, 128, 16, p, 0, 0, 1, None) == 1
 
 
+def test_decode_rows_are_cut_only_where_they_outlast_the_prefill():
+    h = _lib().lib()
+    huge = 1 << 62
+    for longest, tiles, want in ((400, 0, 1), (400, 66, 1), (400, 67, 0), (396, 66, 0), (397, 66, 1), (400, huge, 0)):
+        assert h.bvllm_prefill_balance_rows(28, 4, longest, 4 * longest, tiles) == want, (longest, tiles)
+    assert h.bvllm_prefill_balance_rows(28, 4, 400, 1000 * 400, 1) == 0  # even rows
+    assert h.bvllm_prefill_balance_rows(28, 3, 400, 400, 1) == h.bvllm_prefill_balance_rows(28, 4, 0, 0, 0) == 0
+
+
 def test_python_ops_refuse_cpu_tensors():
     from babyvllm.kernels.paged_attn import paged_decode_attention
     from babyvllm.kernels.rope import fused_rope_and_cache

@@ -533,6 +533,23 @@ def test_even_decode_rows_keep_the_plain_launch():
     assert pp._balance_rows(few, 10, 28, 4) == 0
 
 
+def test_decode_rows_that_end_with_the_prefill_keep_the_plain_launch(monkeypatch):
+    """3,000 keys (188 pages) beside a walk of 32 key tiles: whole, with the plain launch's bits, from
+    the native wrapper and the Python one; beside the same walk cut into ranges of 4 tiles: cut."""
+    import babyvllm.kernels.paged_prefill as pp
+
+    q, kv_cache, md = build_prefill_case([(0, 2048)] + [(3000, 1)] * 9, 4, 7, 128)
+    assert pp._balance_rows(md, 10, 28, 4) == 0 and pp._balance_rows(md, 10, 28, 4, 4) == 1
+    native = _kernel()(q, kv_cache, md, 128 ** -0.5)
+    python_path(monkeypatch)
+    monkeypatch.setattr(pp, "_split_tiles", lambda *a: 0)
+    assert torch.equal(_kernel()(q, kv_cache, md, 128 ** -0.5), native)
+    monkeypatch.setattr(pp, "_balance_rows", lambda *a: 0)
+    assert torch.equal(_kernel()(q, kv_cache, md, 128 ** -0.5), native)
+    monkeypatch.setattr(pp, "_balance_rows", lambda *a: 1)
+    assert not torch.equal(_kernel()(q, kv_cache, md, 128 ** -0.5), native)
+
+
 @pytest.mark.parametrize("case", list(CASES) + list(SPLIT_CASES))
 @pytest.mark.parametrize("hkv,group,d", [(4, 7, 128), (2, 7, 64), (1, 33, 128), (8, 1, 128)])
 def test_narrow_blocks_of_short_grids(case, hkv, group, d):
