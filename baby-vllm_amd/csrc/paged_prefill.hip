@@ -1036,6 +1036,10 @@ static hipError_t launch_prefill_split(const PrefillArgs& a, hipStream_t stream)
 // 60 us at 13 tiles per range, 46 at 15, 51 at 20, 75 at 48; 92 unsplit). 0.86 of the
 // slots, since blocks fall unevenly on the XCDs; one work-group per CU beside decode
 // rows (100 new tokens behind 6000 + 20 rows: 44 us at 7 tiles, 34 at 15; 83 unsplit).
+// Predicted times are compared at 0.9 where the longest walk makes four ranges or more and at
+// 0.75 where it makes fewer: there the second half-empty range is what the prediction misses
+// (of 2,054 random steps that 0.9 alone splits, 2.1% were more than 3% slower than unsplit; so,
+// 1,822 are split and 0.3% are).
 // The partials hold every token of the step for every range: at most kMaxRangeBytes (the
 // choices above stay under 50 MB over steps of 2 to 4096 new tokens behind up to 16 thousand;
 // a few tokens on a long prefix beside fresh prompts would take ten times that).
@@ -1050,7 +1054,7 @@ int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles, int64_t lon
   const double blocks = hkv * p.bound;
   const bool narrow = 2.0 * blocks <= cus && p.dec_wgs == 0;
   const double unsplit = narrow ? 5.5 + 0.6 * longest : 7.0 + (2.0 * blocks <= cus ? 0.79 : 1.1) * longest;
-  double best = 0.9 * unsplit;
+  double best = unsplit;
   const int64_t max_ranges = kMaxRangeBytes / (prefill_range_floats(1, a.num_tokens, a.num_heads, a.head_dim) * 4);
   if (max_ranges < 2) return 0;
   int32_t tiles = 0;
@@ -1062,7 +1066,7 @@ int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles, int64_t lon
     const double ranges = steps / (blocks * c) + 0.5;
     const double bytes = (double)a.num_tokens * a.num_heads * (a.head_dim + 2) * 4 * ranges;
     const double t = 14.0 + 2 * bytes / 8e6 + (per_cu == 1 ? 1.3 : 1.75) * c;
-    if (t < best) {
+    if (t < best && t < (4 * c <= longest ? 0.9 : 0.75) * unsplit) {
       best = t;
       tiles = (int32_t)c;
     }
