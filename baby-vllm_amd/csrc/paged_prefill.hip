@@ -1087,7 +1087,11 @@ int32_t prefill_split_tiles(const PrefillArgs& a, int64_t key_tiles, int64_t lon
 // and twice the work-groups (1 x 64: 6.9 -> 5.5 us, 1 x 560: 14.1 -> 12.1, 40 behind 1500:
 // 25.1 -> 19.6, 0.5B 1 x 1000: 14.3 -> 11.8). Not with more (8 x 60-120 tokens, 316
 // work-groups of 64: 11.0 against 13.2; 800 tokens, 352: 19.1 either way), nor beside
-// decode rows, which the extra work-groups delay (1 x 512 + 63 x 1001: 28.3 against 41.4).
+// decode rows, which the extra work-groups delay (1 x 512 + 63 x 1001: 28.3 against 41.4),
+// nor with many sequences of few tokens behind long prefixes once half the CUs have a
+// 64-column block (32-column blocks hold a few columns of one sequence there and stream its
+// keys twice over: 26 x 9 tokens behind 6000, 8 KV heads: 144 against 165 us; 48 x 5-78
+// behind 10000: 181 against 210; on average over 24 sequences and 64 pages the two are even).
 template <int D>
 static hipError_t prefill_for_dim(const PrefillArgs& a, hipStream_t stream) {
   if (a.split_tiles > 0) return launch_prefill_split<D>(a, stream);
@@ -1099,7 +1103,8 @@ static hipError_t prefill_for_dim(const PrefillArgs& a, hipStream_t stream) {
   }
   if (tuning(kTunePrefillShortGrid) == 1) return launch_prefill<D, 4, 1>(a, plan_prefill(a, 4 * 1 * 16), 1, stream);
   const PrefillGrid p1 = plan_prefill(a, 4 / 2 * 2 * 16);
-  if (tuning(kTunePrefillShortGrid) != 2 && p1.dec_wgs == 0 && p1.prefill_wgs <= (int64_t)device_cus())
+  const bool long_thin = a.num_seqs >= 24 && a.max_blocks >= 64 && 2 * p1.prefill_wgs > (int64_t)device_cus();
+  if (tuning(kTunePrefillShortGrid) != 2 && p1.dec_wgs == 0 && p1.prefill_wgs <= (int64_t)device_cus() && !long_thin)
     return launch_prefill<D, 4, 1, 2>(a, plan_prefill(a, 4 / 2 * 1 * 16), 1, stream);
   return launch_prefill<D, 4, 2, 2>(a, p1, 1, stream);
 }

@@ -562,3 +562,14 @@ def test_narrow_blocks_of_short_grids(case, hkv, group, d):
     for knob in (0, 2):
         with tuned(_SHORT_GRID, knob):
             assert_attn_close(_kernel()(q, kv_cache, md, d ** -0.5), expected)
+
+
+@pytest.mark.parametrize("seqs,context", [(24, 1020), (23, 1020), (24, 900)])
+def test_many_thin_sequences_on_either_block_width(seqs, context):
+    """Around the line where 32-column blocks stop paying (24 sequences, 64 pages): the bits of
+    64-column blocks on both sides."""
+    q, kv_cache, md = build_prefill_case([(context + i % 3, 2 + i % 7) for i in range(seqs)], 8, 4, 128, seed=4)
+    out = _kernel()(q, kv_cache, md, 128 ** -0.5)
+    with tuned(_SHORT_GRID, 2):
+        assert torch.equal(_kernel()(q, kv_cache, md, 128 ** -0.5), out)
+    assert_attn_close(out, _oracle(q, kv_cache, md, 4))
