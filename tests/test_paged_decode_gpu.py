@@ -523,6 +523,24 @@ def test_balanced_launch_in_a_graph_follows_the_lengths(monkeypatch):
         assert_attn_close(out, _oracle(q, kv_cache, bt, lens, scale, 4000), rows=_live(lens))
 
 
+@pytest.mark.parametrize("partition", [32, 33, 64, 68])
+@pytest.mark.parametrize("hkv,group,d", [(1, 8, 128), (1, 7, 64), (1, 20, 128)])
+def test_long_splits_agree_on_every_wave_count_and_order(partition, hkv, group, d):
+    """Single splits of more than 32 pages that outnumber the CUs (live units first, two or four
+    waves) against one wave per split, which numbers them row by row, and against units
+    fastest: the same bits, with empty rows, empty splits and more rows than a wave's lanes."""
+    lens = [5000, 0, 1, 16 * partition, 16 * partition + 1, 300, 4999] + [40, 0] * 30
+    q, kv_cache, bt, seq_lens = make_decode_inputs(lens, hkv=hkv, group=group, d=d, seed=43)
+    outs = {}
+    for mode, order in ((0, 0), (1, 0), (4, 0), (0, 1)):
+        with tuned(0, mode), tuned(2, order):
+            outs[mode, order] = _kernel()(q, kv_cache, bt, seq_lens, d ** -0.5, max_seq_len=max(lens),
+                                          partition_blocks=partition)
+    for key, out in outs.items():
+        assert torch.equal(out, outs[1, 0]), key
+    assert_attn_close(outs[0, 0], _oracle(q, kv_cache, bt, lens, d ** -0.5), rows=_live(lens))
+
+
 @pytest.mark.parametrize("partition", [16, 32, 64])
 @pytest.mark.parametrize("hkv,group,d", [(4, 7, 128), (2, 7, 64), (1, 20, 128)])
 def test_long_groups_agree_on_every_wave_count_and_order(partition, hkv, group, d):
